@@ -229,6 +229,8 @@ int nfft2d_plan_num_points(const nfft2d_plan *plan);
  *   NFFT2D_NDFT_FP16    FP16 operands, each k1 row of `data` scaled by a power
  *                       of two into the FP16 range (undone after the product).
  * The phasors A and B are evaluated in FP32 from an FP64 phase reduction.
+ * FP32 and BF16X3 sum conjugate pairs of modes (k, -1 - k) with real cosines
+ * and sines, half the products; FP16 sums single modes.
  * Layouts and units are those of NFFT1_2D_GPU_c64.  The plan holds the mode
  * operand in the matrix cores' operand order (about 4 N1 N2 bytes for BF16X3);
  * nfft2d_ndft_set_modes fills it, nfft2d_ndft_eval contracts it with M

@@ -458,7 +458,7 @@ struct nfft2d_ndft_plan_s {
     int N1, N2, prec, device;
     int nch, nks;
     void *G;              // mode operand, nch * nks * C * 64 slices
-    float *scale;         // N1 per-row scales and their inverses
+    float *scale;         // FP16: N1 per-row scales and their inverses
     float *inv_scale;
 };
 
@@ -477,8 +477,10 @@ extern "C" int nfft2d_ndft_plan_create(nfft2d_ndft_plan **plan, int N1, int N2, 
     p->N2 = N2;
     p->prec = precision;
     NFFT2D_HIP_TRY(hipGetDevice(&p->device));
+    // K indices: pairs of modes, or (FP16) single modes
+    const int kn = precision == NFFT2D_NDFT_FP16 ? N2 : N2 / 2;
     p->nch = (N1 + ndft::kChunkK1 - 1) / ndft::kChunkK1;
-    p->nks = (N2 + 8 * ndft::kKsPad - 1) / (8 * ndft::kKsPad) * ndft::kKsPad;
+    p->nks = (kn + 8 * ndft::kKsPad - 1) / (8 * ndft::kKsPad) * ndft::kKsPad;
     const size_t gbytes = (size_t)p->nch * p->nks * kNdftC * 64 * ndft_slice_bytes(precision);
     if (nfft2d_malloc(&p->G, gbytes) != hipSuccess || nfft2d_malloc(&p->scale, sizeof(float) * N1) != hipSuccess ||
         nfft2d_malloc(&p->inv_scale, sizeof(float) * N1) != hipSuccess) {
@@ -507,9 +509,10 @@ extern "C" int nfft2d_ndft_set_modes(nfft2d_ndft_plan *p, const nfft2d_c64 *data
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     const float2 *F = reinterpret_cast<const float2 *>(data);
-    hipLaunchKernelGGL(ndft::k_ndft_rowscale, dim3(p->N1), dim3(256), 0, s, F, p->scale, p->inv_scale, p->N2,
-                       p->prec == NFFT2D_NDFT_FP16 ? 1 : 0);
-    NFFT2D_LAUNCH_CHECK();
+    if (p->prec == NFFT2D_NDFT_FP16) {   // the other precisions take their operands unscaled
+        hipLaunchKernelGGL(ndft::k_ndft_rowscale, dim3(p->N1), dim3(256), 0, s, F, p->scale, p->inv_scale, p->N2);
+        NFFT2D_LAUNCH_CHECK();
+    }
     const long long total = (long long)p->nch * p->nks * kNdftC * 64;
     const dim3 grid((unsigned)((total + 255) / 256));
     switch (p->prec) {
@@ -553,7 +556,7 @@ extern "C" int nfft2d_ndft_eval(nfft2d_ndft_plan *p, nfft2d_c64 *result, const f
                            p->nch, p->nks);
         break;
     case NFFT2D_NDFT_BF16X3:
-        hipLaunchKernelGGL((ndft::k_ndft_t2<ndft::kNdftBf16x3, 16, NDFT_SPLIT>), grid, block, 0, s,
+        hipLaunchKernelGGL((ndft::k_ndft_t2<ndft::kNdftBf16x3, 8, NDFT_SPLIT>), grid, block, 0, s,
                            (const ndft::Slice<ndft::kNdftBf16x3> *)p->G, p->inv_scale, x, y, out, p->N1, p->N2, M,
                            p->nch, p->nks);
         break;

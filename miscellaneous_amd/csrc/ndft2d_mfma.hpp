@@ -1,18 +1,27 @@
 // ndft2d_mfma.hpp -- type-2 NDFT (modes -> points) as a separable contraction on MFMA.
 //
 //   y_m = sum_{k1,k2} F[k1][k2] e^{-2 pi i (k1 x1_m / N1 + k2 x2_m / N2)}
-//       = sum_{k1} A[m][k1] T[m][k1],   T = B F^T,
-//   A[m][k1] = e^{-2 pi i k1 x1_m / N1},  B[m][k2] = e^{-2 pi i k2 x2_m / N2},
-//
 // the (M x N2)(N2 x N1) o (M x N1) form of the reference's direct sum
 // (NFFT/NDFT2_2D.cu:15-32 fills the M x N kernel matrix that cublasZgemv
 // contracts at :67; NFFT/NFFT2/Matlab/NDFT2_2D.m:9-14 is the same sum).
 //
-// T is one real GEMM: rows = points, K = 2 N2 (Re/Im of B interleaved per k2),
-// columns = 2 N1 (the Re and Im parts of T for every k1).  Its left operand
-// (the points' phasors) is generated in registers; its right operand (the
-// modes, G below) is prepared once per call in the exact per-lane order the
-// MFMA reads it.  The k1 contraction with A happens in the epilogue.
+// The modes k and -1 - k of a dimension carry conjugate phasors once half a
+// step is taken out: with t = x / N, h = j + 1/2, j < N / 2,
+//   e^{-2 pi i j t} = e^{pi i t} e^{-2 pi i h t},
+//   e^{-2 pi i (-1 - j) t} = e^{pi i t} e^{+2 pi i h t},
+// so a pair (F+, F-) contributes (F+ + F-) cos - i (F+ - F-) sin.  In both
+// dimensions (c, s = cos, sin of 2 pi (j + 1/2) x / N),
+//   y = e^{pi i (t1 + t2)} sum_{j1} c1 P[j1] - i s1 Q[j1],
+//   P = sum_{j2} EP c2 - i OP s2,   Q = sum_{j2} EQ c2 - i OQ s2,
+//   EP, OP = sum over the two k1 of F+ + F-, F+ - F- (the k2 pair);
+//   EQ, OQ = their difference over the two k1.
+// P and Q are one real GEMM: rows = points, K = N2 (c2 and s2 of each j2),
+// columns = 2 N1 (Re and Im of P and Q for every j1): half the products of
+// the sum over k2 with complex phasors (K = 2 N2).  256 x 256 modes, M =
+// 65,536, kernel time before / after: FP32 285 / 148 us, BF16x3 85 / 45 us.  Its left operand (the points' phasors) is
+// generated in registers; its right operand (the modes' sums and differences,
+// G below) is prepared once per call in the exact per-lane order the MFMA
+// reads it.  The j1 contraction happens in the epilogue.
 //
 // Precisions (the operand type of the T product; accumulation is FP32):
 //   kNdftFp32   v_mfma_f32_32x32x2f32, operands FP32;
@@ -20,6 +29,10 @@
 //               T = hi*hi + hi*lo + lo*hi;
 //   kNdftFp16   v_mfma_f32_32x32x16_f16, each k1 row of F scaled by a power of
 //               two into the FP16 range, the scale undone in the epilogue.
+//               Its operands are rounded once (2.7e-4 of the result), so their
+//               values set its results: it keeps the sum over single modes,
+//               T = B F^T (K = 2 N2, Re and Im of B per k2; columns Re and Im
+//               of T per k1) folded with A in the epilogue.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -35,6 +48,8 @@ constexpr int kWaves = 4;                  // waves per workgroup
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+
+template <int P> constexpr bool paired() { return P != kNdftFp16; }   // conjugate pairs of modes, or single modes
 
 // One lane's slice of one 32-column x 16-K tile of the right operand.
 template <int P> struct Slice;
@@ -121,9 +136,8 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 // e^{-2 pi i k x / N} for integer k and FP32 x: the phase k x / N is reduced
 // mod 1 in FP64 (k x is exact there), then split t = th + tl so that the FP32
 // sincospi of th is corrected to first order by tl.
-__device__ __forceinline__ float2 expi_neg(int k, float x, double invN)
+__device__ __forceinline__ float2 expi_neg_turns(double t)   // e^{-2 pi i t}
 {
-    double t = (double)k * (double)x * invN;
     t -= rint(t);
     const float th = (float)t;
     const float tl = (float)(t - (double)th);
@@ -132,14 +146,23 @@ __device__ __forceinline__ float2 expi_neg(int k, float x, double invN)
     const float d = 6.28318530717958647692f * tl;
     return make_float2(fmaf(-d, s, c), -fmaf(d, c, s));
 }
+__device__ __forceinline__ float2 expi_neg(int k, float x, double invN)
+{
+    return expi_neg_turns((double)k * (double)x * invN);
+}
 
 // Right operand G, slice (ch, ks, t, lane) -- tile (ch, ks, t) of 64 lane
 // slices, stored part-major (see the end of the kernel): element e of lane (h = lane / 32,
 // cc = lane % 32) is G[K = 16 ks + 8 h + e][col = ch * 32 C + 32 t + cc] with
-//   k2 index j2 = 8 ks + 4 h + e / 2, component e % 2 (0: Re B, 1: Im B),
-//   k1 index j1 = ch * 16 C + 32 (t / 2) + cc, part t % 2 (0: Re T, 1: Im T):
+//   pair index j2 = 8 ks + 4 h + e / 2, component e % 2 (0: cos, 1: -sin),
+//   pair index j1 = ch * 8 C + 16 (t / 2) + cc / 2, cc % 2 (0: P, 1: Q),
+//   part t % 2 (0: Re, 1: Im); for P (Q with EQ, OQ):
+//   Re P = sum c Re EP - (-s) Im OP,  Im P = sum c Im EP + (-s) Re OP.
+// Entries with j1 >= N1 / 2 or j2 >= N2 / 2 are zero (padding to whole tiles).
+// The sums of four modes are taken in FP64 and rounded once.
+// Single modes (FP16): k2 index j2 as above with components (Re B, Im B), k1
+// index j1 = ch * 16 C + 32 (t / 2) + cc, part t % 2 of T:
 //   Re T = sum Re B Re F - Im B Im F,  Im T = sum Re B Im F + Im B Re F.
-// Entries with j1 >= N1 or j2 >= N2 are zero (padding to whole tiles).
 template <int P, int C>
 __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F, const float* __restrict__ rowscale,
                                                    Slice<P>* __restrict__ G, int N1, int N2, int nch, int nks)
@@ -154,18 +177,39 @@ __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F,
     const int ks = (int)(r % nks);
     const int ch = (int)(r / nks);
     const int h = lane >> 5, cc = lane & 31;
-    const int j1 = ch * 16 * C + 32 * (t >> 1) + cc;
     const int part = t & 1;
-    const float sc = j1 < N1 ? rowscale[j1] : 1.0f;
     float v[8];
+    if constexpr (paired<P>()) {
+        const int j1 = ch * 8 * C + 16 * (t >> 1) + (cc >> 1);
+        const double sq = (cc & 1) ? -1.0 : 1.0;       // P adds, Q subtracts the second k1 row
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int j2 = 8 * ks + 4 * h + (e >> 1), comp = e & 1;
-        float2 f = make_float2(0.f, 0.f);
-        if (j1 < N1 && j2 < N2) f = F[(size_t)j1 * N2 + j2];
-        f.x *= sc;
-        f.y *= sc;
-        v[e] = part == 0 ? (comp == 0 ? f.x : -f.y) : (comp == 0 ? f.y : f.x);
+        for (int q = 0; q < 4; ++q) {
+            const int j2 = 8 * ks + 4 * h + q;
+            double2 e = make_double2(0.0, 0.0), o = e;
+            if (j1 < N1 / 2 && j2 < N2 / 2) {
+                const float2* rp = F + (size_t)(N1 / 2 + j1) * N2 + N2 / 2;        // k1 = j1
+                const float2* rm = F + (size_t)(N1 / 2 - 1 - j1) * N2 + N2 / 2;    // k1 = -1 - j1
+                const float2 pp = rp[j2], pm = rp[-1 - j2], mp = rm[j2], mm = rm[-1 - j2];
+                e.x = ((double)pp.x + (double)pm.x) + sq * ((double)mp.x + (double)mm.x);
+                e.y = ((double)pp.y + (double)pm.y) + sq * ((double)mp.y + (double)mm.y);
+                o.x = ((double)pp.x - (double)pm.x) + sq * ((double)mp.x - (double)mm.x);
+                o.y = ((double)pp.y - (double)pm.y) + sq * ((double)mp.y - (double)mm.y);
+            }
+            v[2 * q] = (float)(part == 0 ? e.x : e.y);
+            v[2 * q + 1] = (float)(part == 0 ? -o.y : o.x);
+        }
+    } else {
+        const int j1 = ch * 16 * C + 32 * (t >> 1) + cc;
+        const float sc = j1 < N1 ? rowscale[j1] : 1.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int j2 = 8 * ks + 4 * h + (e >> 1), comp = e & 1;
+            float2 f = make_float2(0.f, 0.f);
+            if (j1 < N1 && j2 < N2) f = F[(size_t)j1 * N2 + j2];
+            f.x *= sc;
+            f.y *= sc;
+            v[e] = part == 0 ? (comp == 0 ? f.x : -f.y) : (comp == 0 ? f.y : f.x);
+        }
     }
     Slice<P> s;
     if constexpr (P == kNdftFp32) {
@@ -208,18 +252,17 @@ __device__ __forceinline__ Slice<P> load_slice(const uint4* base, int tile, int 
 
 // Per-row scale of F for the FP16 operand: a power of two that brings the
 // row's largest |Re| or |Im| to [2^13, 2^14).  One block per row; rows with no
-// finite non-zero entry get 1.  The other precisions use 1.
+// finite non-zero entry get 1.
 __global__ __launch_bounds__(256) void k_ndft_rowscale(const float2* __restrict__ F, float* __restrict__ scale,
-                                                       float* __restrict__ inv_scale, int N2, int fp16)
+                                                       float* __restrict__ inv_scale, int N2)
 {
     __shared__ float red[256];
     const int j1 = blockIdx.x;
     float mx = 0.f;
-    if (fp16)
-        for (int j2 = threadIdx.x; j2 < N2; j2 += 256) {
-            const float2 f = F[(size_t)j1 * N2 + j2];
-            mx = fmaxf(mx, fmaxf(fabsf(f.x), fabsf(f.y)));
-        }
+    for (int j2 = threadIdx.x; j2 < N2; j2 += 256) {
+        const float2 f = F[(size_t)j1 * N2 + j2];
+        mx = fmaxf(mx, fmaxf(fabsf(f.x), fabsf(f.y)));
+    }
     red[threadIdx.x] = mx;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
@@ -249,9 +292,11 @@ static_assert(kKsPad % kKsExact == 0, "chunks start on an exact K-step");
 // L2-to-LDS copy of a K-step takes longer than the K-step's MFMAs, so the
 // copies run kAhead steps ahead (kAhead + 1 LDS buffers, rotating).
 constexpr int kAhead = 3;
-// Column tiles per chunk: 8 tiles = 4 groups of 32 k1 = 128 k1 per pass over K.
+// Column tiles per chunk: 8 tiles = 4 groups of 32 k1 (16 pairs j1) = 128 k1
+// (64 pairs) per pass over K.
 constexpr int kChunkTiles = 8;
 constexpr int kChunkK1 = 16 * kChunkTiles;
+constexpr int kChunkPairs = kChunkK1 / 2;
 // Row tiles (of 32 points) per wave: each right-operand slice read from LDS
 // feeds both.
 constexpr int kRowTiles = 2;
@@ -284,20 +329,23 @@ __device__ __forceinline__ void wave_sync()
 
 // Main contraction.  Workgroup = 4 waves, one per SIMD; wave w owns points
 // 64 w .. 64 w + 63 of the group as two MFMA row tiles of 32.  For each chunk
-// of 128 k1 (8 column tiles: Re and Im tiles of 4 groups of 32 k1) the wave
-// runs the K loop over all k2 with 2 x 8 accumulator tiles (256 registers per
-// lane): per K-step it generates the point operands of its two row tiles and
-// multiplies each right-operand slice, read once from LDS, into both.  The
-// slices of the next K-step are copied by the workgroup from global memory
-// straight into LDS while the current ones are multiplied (two buffers, one
-// barrier per K-step).  Accumulator element r of lane (h, cc) holds row
-// 8 (r / 4) + 4 h + r % 4, column cc.  After the K loop each (row tile, group
-// of 32 k1) is transposed through LDS so that lane (h, row) folds columns
-// 16 h .. 16 h + 15 of its row with A[m][k1] = e^{-2 pi i k1 x1_m / N1}, A
-// advancing by e^{-2 pi i x1_m / N1} per column from an exact value every
-// EANCHOR columns.  The point operand is evaluated exactly (one phase
-// reduction, then three products with the k2 step phasors) on every
+// of 64 pairs j1 (8 column tiles: Re and Im tiles of 4 groups of 16 pairs, P
+// and Q columns alternating) the wave runs the K loop over all j2 with 2 x 8
+// accumulator tiles (256 registers per lane): per K-step it generates the
+// point operands of its two row tiles and multiplies each right-operand slice,
+// read once from LDS, into both.  The slices of the next K-steps are copied by
+// the workgroup from global memory straight into LDS while the current ones
+// are multiplied (rotating buffers, one barrier per K-step).  Accumulator
+// element r of lane (h, cc) holds row 8 (r / 4) + 4 h + r % 4, column cc.
+// After the K loop each (row tile, group of 16 pairs) is transposed through
+// LDS so that lane (h, row) folds columns 16 h .. 16 h + 15 of its row (8
+// pairs) with (c1, s1) = e^{-2 pi i (j1 + 1/2) x1_m / N1}, advancing by
+// e^{-2 pi i x1_m / N1} per pair from an exact value every EANCHOR pairs.
+// The point operand is evaluated exactly (one phase
+// reduction, then three products with the j2 step phasors) on every
 // kKsExact-th K-step and advanced by e^{-2 pi i 8 x2 / N2} on the others.
+// (Single modes: j1 and j2 count k1 and k2 from -N/2, and a lane folds the 16
+// columns T of its half with A.)
 //
 // SPLIT = 2 runs two waves per SIMD: waves w and w + 4 hold the same points
 // and split each chunk's column tiles between them (128 accumulator registers
@@ -330,7 +378,12 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
     const int h = lane >> 5, cc = lane & 31;
     const int m0 = blockIdx.x * kPtsPerGroup + kPtsPerWave * pg;  // first point of this wave
     const double invN1 = 1.0 / N1, invN2 = 1.0 / N2;
+    constexpr bool kPair = paired<P>();
+    // phase of index j: pairs (2 j + 1) x / (2 N), single modes (j - N / 2) x / N
+    const double pu1 = (kPair ? 0.5 : 1.0) / N1, pu2 = (kPair ? 0.5 : 1.0) / N2;
     const int half1 = N1 / 2, half2 = N2 / 2;
+    auto ph1 = [&](int j) { return kPair ? 2 * j + 1 : j - half1; };
+    auto ph2 = [&](int j) { return kPair ? 2 * j + 1 : j - half2; };
     const int total = nch * nks;
     const uint4* Gw = reinterpret_cast<const uint4*>(G);
 
@@ -364,12 +417,12 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
     barrier_no_fence();
 
     f16v acc[R][CW];
-    // point operand of row tile r at K-step ks: e^{-2 pi i k2 x2 / N2} for
-    // k2 = 8 ks + 4 h + 0..3 - N2/2, (Re, Im) interleaved
-    // exact: z0 = e^{-2 pi i k2 x2 / N2} at the K-step's first k2 of this lane;
-    // otherwise z0 advances by 8 k2 from the previous K-step
+    // point operand of row tile r at K-step ks: e^{-2 pi i (j2 + 1/2) x2 / N2}
+    // for j2 = 8 ks + 4 h + 0..3, (cos, -sin) interleaved
+    // exact: z0 at the K-step's first j2 of this lane; otherwise z0 advances by
+    // 8 j2 from the previous K-step
     auto gen = [&](int r, int ks, bool exact) {
-        z0[r] = exact ? expi_neg(8 * ks + 4 * h - half2, xr2[r], invN2) : cmul(z0[r], w8[r]);
+        z0[r] = exact ? expi_neg(ph2(8 * ks + 4 * h), xr2[r], pu2) : cmul(z0[r], w8[r]);
         float2 z[4];
         z[0] = z0[r];
         z[1] = cmul(z[0], w1[r]);
@@ -443,14 +496,15 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
             step(g0 + 2, ks + 2, s_stage2, s_stage1, Advance{});
             step(g0 + 3, ks + 3, s_stage3, s_stage2, Exact{});
         }
-        // epilogue of chunk ch: y += sum_k1 A[m][k1] T[m][k1] over the wave's
-        // groups of 32 k1 of the chunk (group gg = its Re and Im tiles)
+        // epilogue of chunk ch: y += sum_j1 c1 P - i s1 Q (sum_k1 A T) over the
+        // wave's groups of 32 columns of the chunk (group gg = its Re and Im tiles)
+        constexpr int kFold = kPair ? 8 : 16;                                 // phasors per lane and group
 #pragma unroll
         for (int r = 0; r < R; ++r) {
 #pragma unroll
             for (int g = 0; g < CW / 2; ++g) {
                 const int gg = (CW / 2) * hc + g;
-                const int j1c = ch * kChunkK1 + 32 * gg + cc;       // k1 index of column cc
+                const int j1c = ch * kChunkK1 + 32 * gg + cc;                 // k1 index of column cc (FP16)
                 const float isc = (P == kNdftFp16 && j1c < N1) ? inv_scale[j1c] : 1.0f;
 #pragma unroll
                 for (int q = 0; q < 16; ++q) {
@@ -458,20 +512,31 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
                     s_t[w][ti][cc] = make_float2(acc[r][2 * g][q] * isc, acc[r][2 * g + 1][q] * isc);
                 }
                 wave_sync();
-                const int k1s = ch * kChunkK1 + 32 * gg + 16 * h - half1;  // k1 of this lane's first column
-                float2 A = make_float2(1.f, 0.f);
+                const int j1s = (kPair ? kChunkPairs : kChunkK1) * ch + 2 * kFold * gg + kFold * h;  // first index
+                float2 A = make_float2(1.f, 0.f);                             // (c1, -s1), or A
 #pragma unroll
-                for (int c = 0; c < 16; ++c) {
-                    if (c % EANCHOR == 0) A = expi_neg(k1s + c, xr1[r], invN1);
-                    const float2 tv = s_t[w][cc][16 * h + c];
-                    y[r].x = fmaf(A.x, tv.x, fmaf(-A.y, tv.y, y[r].x));
-                    y[r].y = fmaf(A.x, tv.y, fmaf(A.y, tv.x, y[r].y));
+                for (int c = 0; c < kFold; ++c) {
+                    if (c % EANCHOR == 0) A = expi_neg(ph1(j1s + c), xr1[r], pu1);
+                    if constexpr (kPair) {
+                        const float2 pv = s_t[w][cc][16 * h + 2 * c], qv = s_t[w][cc][16 * h + 2 * c + 1];
+                        y[r].x = fmaf(A.x, pv.x, fmaf(-A.y, qv.y, y[r].x));
+                        y[r].y = fmaf(A.x, pv.y, fmaf(A.y, qv.x, y[r].y));
+                    } else {
+                        const float2 tv = s_t[w][cc][16 * h + c];
+                        y[r].x = fmaf(A.x, tv.x, fmaf(-A.y, tv.y, y[r].x));
+                        y[r].y = fmaf(A.x, tv.y, fmaf(A.y, tv.x, y[r].y));
+                    }
                     if (c % EANCHOR != EANCHOR - 1) A = cmul(A, e1[r]);
                 }
                 wave_sync();
             }
         }
     }
+    // pairs: y carries e^{pi i (x1 / N1 + x2 / N2)}, the half steps of both dimensions
+    float2 half[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        half[r] = kPair ? expi_neg_turns(-((double)xr1[r] * pu1 + (double)xr2[r] * pu2)) : make_float2(1.f, 0.f);
     // the two halves of each row, then (SPLIT = 2) the two column shares
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -490,7 +555,7 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
                 v.y += o.y;
             }
             const int m = m0 + 32 * r + cc;
-            if (m < M) out[m] = v;
+            if (m < M) out[m] = kPair ? cmul(v, half[r]) : v;
         }
     }
 }
