@@ -112,8 +112,9 @@ void Destroy_cuFFT_plan_NFFT2_2D(void);
  * (:44,56) before its gemv (:67); neither happens here.  Outputs on a meshgrid
  * (u, v arithmetic progressions, either flattening; detected on the device)
  * take the FP64 matrix-core contraction, any other (u, v) the direct sum.  Runs
- * on the legacy default stream.  A workspace of at most 64 N + 2 M complex
- * values is kept per device and grown when a call needs more (the growth
+ * on the legacy default stream.  A workspace of at most 256 N + 5 M complex
+ * values (4.2 million + 5 M from N = 16,384 outputs on, N + 5 M from 4.2
+ * million on) is kept per device and grown when a call needs more (the growth
  * synchronises the device); concurrent calls on one device serialise on it. */
 int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, const double *u, const double *v,
                  const nfft2d_c128 *in, nfft2d_c128 *out, int Nu, int Nv, int M, int N);

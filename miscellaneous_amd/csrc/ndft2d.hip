@@ -5,10 +5,9 @@
 // M = N = 65536), writes it to a text file (:56) and calls cublasZgemv (:67).
 // Here nothing of that size is materialised: on the integer meshgrid the
 // reference's caller passes, the sum is an FP64 complex GEMM on the matrix
-// cores (k_ndft_grid + k_ndft_grid_sum, with a cached workspace of at most 64
-// partial output arrays); for other (u, v) each thread owns one output n and
-// streams the points through LDS in chunks, accumulating in FP64
-// (k_ndft_direct).
+// cores (k_ndft_grid + k_ndft_finish, with a cached workspace of at most 256
+// partial output arrays); for other (u, v) each thread takes one output over a
+// range of the points, accumulating in FP64.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -35,10 +34,10 @@ constexpr int kThreads = 256;
 // k_grid_detect recognises the two flattenings of such a grid (u constant
 // over runs of nv outputs, or v constant over runs of nu) and k_grid_verify
 // checks every output against it by exact FP64 comparison; the finding stays
-// in g_grid (one per device, as every __device__ variable); k_ndft_grid runs
-// when it is a grid, k_ndft_direct
-// (any u, v) when it did not.  Both read the flag on the device, so the call
-// stays asynchronous and capturable.  Two NDFT2_2D_GPU calls that overlap on
+// in g_grid (one per device, as every __device__ variable); k_ndft_grid takes
+// the matrix cores when it is a grid and the direct sum (any u, v) when it is
+// not.  It reads the flag on the device, so the call stays asynchronous and
+// capturable.  Two NDFT2_2D_GPU calls that overlap on
 // one device (different streams) race on g_grid.
 struct GridInfo {
     int ok;          // 1: (u, v) is a grid of nu x nv outputs
@@ -121,40 +120,6 @@ __global__ __launch_bounds__(kDetThreads) void k_grid_detect(const double *__res
     }
 }
 
-// Clears g_grid.ok when an output is not the grid's: u[n] = u0 + i du and
-// v[n] = v0 + j dv, exactly, for n's (i, j) in the detected flattening.
-__global__ __launch_bounds__(kThreads) void k_grid_verify(const double *__restrict__ u, const double *__restrict__ v,
-                                                          int N)
-{
-    const GridInfo g = g_grid;
-    if (!g.ok) return;
-    const int n = blockIdx.x * kThreads + threadIdx.x;
-    if (n >= N) return;
-    const int i = g.vmajor ? n % g.nu : n / g.nv, j = g.vmajor ? n / g.nu : n % g.nv;
-    if (u[n] != g.u0 + i * g.du || v[n] != g.v0 + j * g.dv) g_grid.ok = 0;
-}
-
-// The grid case on v_mfma_f64_16x16x4f64 (4 points per instruction): lane l
-// supplies A[i][k] at i = l % 16, k = l / 16 and B[k][j] at j = l % 16;
-// accumulator element r of lane l is C[4 r + l / 16][l % 16].  The complex
-// product is four real ones: Cr += Ar Br - Ai Bi, Ci += Ar Bi + Ai Br.
-//
-// A work item is one wave: a supertile of kTR x kTC MFMA tiles (32 x 64
-// outputs) over one range of the points.  Per K-step of 4 points a lane
-// evaluates its point's phasor at its first row and first column by an FP64
-// phase reduction and sincospi, and the phasors 16 rows / columns further on
-// by one complex product with the point's 16-step phasor each (rows and
-// columns are arithmetic progressions; the steps come from k_ndft_steps, once
-// per call), so that 8 MFMA tiles share 2 sincospi per lane instead of 16.  The partial supertile goes to range r's slice of a
-// workspace; k_ndft_grid_sum adds the ranges in a fixed order (the result does
-// not depend on the launch).  Work items are walked persistently (their count
-// is known on the device only).
-constexpr int kTR = 2, kTC = 4;                   // MFMA tiles per supertile: rows, columns
-constexpr int kSupRows = 16 * kTR, kSupCols = 16 * kTC;
-constexpr int kGridWavesTotal = 2048;             // waves of the persistent launch (2 per SIMD at 190 VGPRs)
-constexpr int kMaxRanges = 64;
-typedef double d4 __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ double2 phasor(double t)   // e^{-2 pi i t}
 {
     t -= floor(t);
@@ -168,146 +133,232 @@ __device__ __forceinline__ double2 zmul(double2 a, double2 b)
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// Supertiles per grid (device side, from the detector's nu, nv).
-__device__ __forceinline__ int n_super(const GridInfo &g, int &stv)
-{
-    stv = (g.nv + kSupCols - 1) / kSupCols;
-    return ((g.nu + kSupRows - 1) / kSupRows) * stv;
-}
+// One point of the grid case: its sample times the phasor of the grid's
+// centre, its 16-row and 16-column phasor steps, and X / Nu, Y / Nv.
+struct alignas(16) GridPt {
+    double2 d, step[2];
+    double xy[2];
+};
 
-// steps[m] = (e^{-2 pi i 16 du X_m / Nu}, e^{-2 pi i 16 dv Y_m / Nv}): the 16-row and 16-column
-// steps of point m's phasors, once per call instead of once per supertile.
-__global__ __launch_bounds__(kThreads) void k_ndft_steps(const double *__restrict__ X, const double *__restrict__ Y,
-                                                         double inv_Nu, double inv_Nv, int M,
-                                                         double4 *__restrict__ steps)
+// Two independent jobs on the detector's finding.  Blocks below nver clear
+// g_grid.ok when an output is not the grid's: u[n] = u0 + i du and v[n] =
+// v0 + j dv, exactly, for n's (i, j) in the detected flattening.  The others
+// prepare the points (what they write is unused when the check fails).
+__global__ __launch_bounds__(kThreads) void k_grid_verify(const double *__restrict__ u, const double *__restrict__ v,
+                                                          int N, int nver, const double *__restrict__ X,
+                                                          const double *__restrict__ Y,
+                                                          const double2 *__restrict__ in, double inv_Nu,
+                                                          double inv_Nv, int M, GridPt *__restrict__ pts)
 {
     const GridInfo g = g_grid;
     if (!g.ok) return;
-    const int m = blockIdx.x * kThreads + threadIdx.x;
+    if ((int)blockIdx.x < nver) {
+        const int n = blockIdx.x * kThreads + threadIdx.x;
+        if (n >= N) return;
+        const int i = g.vmajor ? n % g.nu : n / g.nv, j = g.vmajor ? n / g.nu : n % g.nv;
+        if (u[n] != g.u0 + i * g.du || v[n] != g.v0 + j * g.dv) g_grid.ok = 0;
+        return;
+    }
+    const int m = (blockIdx.x - nver) * kThreads + threadIdx.x;
     if (m >= M) return;
-    const double2 sa = phasor(16.0 * g.du * (X[m] * inv_Nu)), sb = phasor(16.0 * g.dv * (Y[m] * inv_Nv));
-    steps[m] = make_double4(sa.x, sa.y, sb.x, sb.y);
+    const double xm = X[m] * inv_Nu, ym = Y[m] * inv_Nv;
+    const double uc = g.u0 + 0.5 * (g.nu - 1) * g.du, vc = g.v0 + 0.5 * (g.nv - 1) * g.dv;
+    GridPt p;
+    p.d = zmul(zmul(in[m], phasor(uc * xm)), phasor(vc * ym));
+    p.step[0] = phasor(16.0 * g.du * xm);
+    p.step[1] = phasor(16.0 * g.dv * ym);
+    p.xy[0] = xm;
+    p.xy[1] = ym;
+    pts[m] = p;
 }
 
-__global__ __launch_bounds__(256) void k_ndft_grid(const double *__restrict__ X, const double *__restrict__ Y,
-                                                   const double2 *__restrict__ in, const double4 *__restrict__ steps,
-                                                   double2 *__restrict__ part, double inv_Nu, double inv_Nv, int M,
-                                                   int ranges, int chunk)
+// The grid case by conjugate pairs.  About the grid's centre (uc, vc) its rows
+// are uc +- delta_p, delta_p = (p + 1/2) du (nu even) or p du (nu odd), and so
+// are its columns, so with d_m the sample times the centre's phasor
+//     out[uc + s1 delta1, vc + s2 delta2] = sum_m d_m (c1 + i s1 t1) (c2 + i s2 t2),
+//     (c, t) = (cos, -sin) of the pair's phase, s1, s2 = +-1,
+// are four combinations of the real-phasor sums CC = sum d c1 c2, TC = sum d
+// t1 c2, CT and TT: 8 real products per 4 outputs and point, half of a complex
+// product for every output.
+//
+// Products on v_mfma_f64_16x16x4f64 (4 points per instruction): lane l
+// supplies A[i][k] at i = l % 16, k = l / 16 and B[k][j] at j = l % 16;
+// accumulator element r of lane l is C[4 r + l / 16][l % 16].  A block takes a
+// tile of 64 x 64 pairs (128 x 128 outputs) over one range of the points: wave
+// w the 16 x 32 pairs of row tile w / 2, column tiles 2 (w % 2) and + 1 (16
+// accumulator tiles, 128 VGPRs; 2 waves per SIMD).  FP64 VALU work does not
+// run under FP64 MFMAs, so the phasors are evaluated once per block: for a
+// chunk of 16 points each of the 512 threads takes one (point, row or column
+// index mod 16) by an FP64 phase reduction and sincospi, advances it three
+// times by the point's 16-step phasor, and leaves the four in LDS (two
+// buffers) while the previous chunk's products run.
+// 256 x 256 outputs from M = 65,536: 0.32 ms a call, 0.75 of the FP64 matrix rate (one wave per 32 x 64
+// outputs with its own phasors and complex products: 0.69 ms).
+// The partial sums go to range r's slice of a workspace; k_ndft_finish adds
+// the ranges in a fixed order (the result does not depend on the launch).
+// Work items are walked persistently (their count is known on the device only).
+constexpr int kTilePairs = 64;                    // pairs per block tile and dimension
+constexpr int kGridThreads = 512;
+constexpr int kGridBlocks = 256;                  // one per CU
+constexpr int kGridChunk = 16;                    // points per LDS buffer
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// Any other (u, v): the direct sum, one output per thread over one range of the
+// points (every thread of a block at the same point, so the point's values are
+// scalar loads), the partial sums going the same way.  One thread per output
+// over all points left most of the chip idle: 4,200 outputs from M = 4,000
+// points, 656 us; in ranges 62 us.
+__device__ __forceinline__ void direct_item(const double *__restrict__ X, const double *__restrict__ Y, double un,
+                                            double vn, const double2 *__restrict__ in, int m_lo, int m_hi,
+                                            double2 &acc)
+{
+    double ar = 0.0, ai = 0.0;
+    auto add = [&](double xm, double ym, double2 d) {
+        double t = un * xm + vn * ym;
+        t -= floor(t);
+        double s, c;
+        sincospi(2.0 * t, &s, &c);   // e^{-2 pi i t} = c - i s
+        ar += d.x * c + d.y * s;
+        ai += d.y * c - d.x * s;
+    };
+    // 8 points' loads ahead of their sums (2 waves per SIMD hide little of a load's latency)
+    constexpr int B = 8;
+    int m = m_lo;
+    for (; m + B <= m_hi; m += B) {
+        double xm[B], ym[B];
+        double2 d[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            xm[b] = X[m + b];
+            ym[b] = Y[m + b];
+            d[b] = in[m + b];
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b) add(xm[b], ym[b], d[b]);
+    }
+    for (; m < m_hi; ++m) add(X[m], Y[m], in[m]);
+    acc = make_double2(ar, ai);
+}
+
+__global__ __launch_bounds__(kGridThreads) void k_ndft_grid(const GridPt *__restrict__ pts,
+                                                            double2 *__restrict__ part, int M, int ranges, int chunk,
+                                                            const double *__restrict__ X, const double *__restrict__ Y,
+                                                            const double *__restrict__ u, const double *__restrict__ v,
+                                                            const double2 *__restrict__ in, double inv_Nu,
+                                                            double inv_Nv, int nout)
 {
     const GridInfo g = g_grid;
-    if (!g.ok) return;
-    const int lane = threadIdx.x & 63, q = lane & 15, k = lane >> 4;
-    int stv;
-    const int items = n_super(g, stv) * ranges;
-    const long long N = (long long)g.nu * g.nv;
-    for (int item = blockIdx.x * 4 + (threadIdx.x >> 6); item < items; item += gridDim.x * 4) {
-        const int r = item % ranges, st = item / ranges;
-        const int i0 = (st / stv) * kSupRows, j0 = (st % stv) * kSupCols;
-        const int m_lo = min(M, r * chunk), m_hi = min(M, m_lo + chunk);
-        const double a0 = g.u0 + (i0 + q) * g.du, b0 = g.v0 + (j0 + q) * g.dv;   // this lane's first row / column
-        bool row_in[kTR], col_in[kTC];
-#pragma unroll
-        for (int t = 0; t < kTR; ++t) row_in[t] = i0 + 16 * t + q < g.nu;
-#pragma unroll
-        for (int t = 0; t < kTC; ++t) col_in[t] = j0 + 16 * t + q < g.nv;
-        d4 cr[kTR][kTC], ci[kTR][kTC];
-#pragma unroll
-        for (int a = 0; a < kTR; ++a)
-#pragma unroll
-            for (int b = 0; b < kTC; ++b) {
-                cr[a][b] = d4{0.0, 0.0, 0.0, 0.0};
-                ci[a][b] = d4{0.0, 0.0, 0.0, 0.0};
-            }
-        // the point data of the next K-step is loaded while the current one is
-        // multiplied (one load round trip per K-step would set the pace)
-        struct Pt {
-            double2 d;
-            double x, y;
-            double4 st;
-        };
-        auto load_pt = [&](int m) {
-            Pt p;
-            if (m < m_hi) {
-                p.d = in[m];
-                p.x = X[m];
-                p.y = Y[m];
-                p.st = steps[m];
-            } else {
-                p.d = make_double2(0.0, 0.0);
-                p.x = p.y = 0.0;
-                p.st = make_double4(1.0, 0.0, 1.0, 0.0);
-            }
-            return p;
-        };
-        Pt cur = load_pt(m_lo + k);
-        for (int m0 = m_lo; m0 < m_hi; m0 += 4) {
-            const Pt nxt = load_pt(m0 + 4 + k);
-            double ar[kTR], ai[kTR], br[kTC], bi[kTC];
-            {
-                // a point past the range has d = 0: its A operands vanish
-                const double xm = cur.x * inv_Nu, ym = cur.y * inv_Nv;
-                double2 pa = phasor(a0 * xm), pb = phasor(b0 * ym);
-                const double2 sa = make_double2(cur.st.x, cur.st.y), sb = make_double2(cur.st.z, cur.st.w);
-#pragma unroll
-                for (int t = 0; t < kTR; ++t) {
-                    const double2 v = zmul(cur.d, pa);
-                    ar[t] = row_in[t] ? v.x : 0.0;
-                    ai[t] = row_in[t] ? v.y : 0.0;
-                    if (t + 1 < kTR) pa = zmul(pa, sa);
-                }
-#pragma unroll
-                for (int t = 0; t < kTC; ++t) {
-                    br[t] = col_in[t] ? pb.x : 0.0;
-                    bi[t] = col_in[t] ? pb.y : 0.0;
-                    if (t + 1 < kTC) pb = zmul(pb, sb);
-                }
-            }
-#pragma unroll
-            for (int a = 0; a < kTR; ++a)
-#pragma unroll
-                for (int b = 0; b < kTC; ++b) {
-                    cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], br[b], cr[a][b], 0, 0, 0);
-                    ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar[a], bi[b], ci[a][b], 0, 0, 0);
-                }
-#pragma unroll
-            for (int a = 0; a < kTR; ++a)
-#pragma unroll
-                for (int b = 0; b < kTC; ++b) {
-                    cr[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], -bi[b], cr[a][b], 0, 0, 0);
-                    ci[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai[a], br[b], ci[a][b], 0, 0, 0);
-                }
-            cur = nxt;
+    if (!g.ok) {
+        const long long nblk = ((long long)nout + kGridThreads - 1) / kGridThreads;
+        for (long long item = blockIdx.x; item < nblk * ranges; item += gridDim.x) {
+            const int r = (int)(item / nblk);
+            const long long n = (item % nblk) * kGridThreads + threadIdx.x;
+            const int m_lo = min(M, r * chunk), m_hi = min(M, m_lo + chunk);
+            const bool have = n < nout;
+            double2 acc;
+            direct_item(X, Y, have ? u[n] * inv_Nu : 0.0, have ? v[n] * inv_Nv : 0.0, in, m_lo, m_hi, acc);
+            if (have) part[(size_t)r * nout + n] = acc;
         }
+        return;
+    }
+    __shared__ double2 s_ph[2][2][kGridChunk][kTilePairs];   // [buffer][row, column][point][pair]
+    __shared__ double2 s_d[2][kGridChunk];
+    const int t = threadIdx.x, lane = t & 63, q = lane & 15, k = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int nu2 = (g.nu + 1) / 2, nv2 = (g.nv + 1) / 2;    // pairs (an odd length's centre is a pair of its own)
+    const int tcols = (nv2 + kTilePairs - 1) / kTilePairs;
+    const int items = (nu2 + kTilePairs - 1) / kTilePairs * tcols * ranges;
+    const long long N = (long long)g.nu * g.nv;
+    // phasor role of this thread: side, point of the chunk, index mod 16
+    const int side = t >> 8, pt = (t >> 4) & 15, pq = t & 15;
+    const int rt = w >> 1, ct = 2 * (w & 1);
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        const int r = item % ranges, st = item / ranges;
+        const int p1 = (st / tcols) * kTilePairs, p2 = (st % tcols) * kTilePairs;   // first pairs of the tile
+        const int m_lo = min(M, r * chunk), m_hi = min(M, m_lo + chunk);
+        const double idx = side ? p2 + pq + (g.nv & 1 ? 0.0 : 0.5) : p1 + pq + (g.nu & 1 ? 0.0 : 0.5);
+        const double off = idx * (side ? g.dv : g.du);
+        const bool act = p1 + 16 * rt < nu2;
+        const bool act0 = act && p2 + 16 * ct < nv2, act1 = act && p2 + 16 * ct + 16 < nv2;
+        struct Pt {
+            double2 d, step;
+            double x;
+        };
+        auto load = [&](int m) {
+            Pt o;
+            o.d = make_double2(0.0, 0.0);   // a point past the range adds nothing
+            o.step = make_double2(1.0, 0.0);
+            o.x = 0.0;
+            if (m < m_hi) {
+                const GridPt *p = pts + m;
+                o.d = p->d;
+                o.step = p->step[side];
+                o.x = p->xy[side];
+            }
+            return o;
+        };
+        auto stage = [&](const Pt &p, int b) {
+            double2 z = phasor(off * p.x);
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                s_ph[b][side][pt][16 * h + pq] = z;
+                if (h < 3) z = zmul(z, p.step);
+            }
+            if (side == 0 && pq == 0) s_d[b][pt] = p.d;
+        };
+        // [column tile][CC, TC, CT, TT]
+        d4 ar[2][4], ai[2][4];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ar[c][e] = ai[c][e] = d4{0.0, 0.0, 0.0, 0.0};
+        __syncthreads();                    // the previous item's reads are done
+        stage(load(m_lo + pt), 0);
+        Pt nxt = load(m_lo + kGridChunk + pt);
+        __syncthreads();
+        int b = 0;
+        for (int m0 = m_lo; m0 < m_hi; m0 += kGridChunk, b ^= 1) {
+            const Pt cur = nxt;
+            nxt = load(m0 + 2 * kGridChunk + pt);
+            if (m0 + kGridChunk < m_hi) stage(cur, b ^ 1);
+#pragma unroll
+            for (int s = 0; s < kGridChunk / 4; ++s) {
+                const double2 d = s_d[b][4 * s + k], a = s_ph[b][0][4 * s + k][16 * rt + q];
+                const double cr = d.x * a.x, ci = d.y * a.x, tr = d.x * a.y, ti = d.y * a.y;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    if (!(c ? act1 : act0)) continue;
+                    const double2 v = s_ph[b][1][4 * s + k][16 * (ct + c) + q];
+                    ar[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(cr, v.x, ar[c][0], 0, 0, 0);
+                    ai[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ci, v.x, ai[c][0], 0, 0, 0);
+                    ar[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, v.x, ar[c][1], 0, 0, 0);
+                    ai[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, v.x, ai[c][1], 0, 0, 0);
+                    ar[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(cr, v.y, ar[c][2], 0, 0, 0);
+                    ai[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(ci, v.y, ai[c][2], 0, 0, 0);
+                    ar[c][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, v.y, ar[c][3], 0, 0, 0);
+                    ai[c][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, v.y, ai[c][3], 0, 0, 0);
+                }
+            }
+            __syncthreads();
+        }
+        // the four outputs of each pair of pairs: rows nu / 2 + p and nu - 1 - (nu / 2 + p)
         double2 *dst = part + (size_t)r * N;
 #pragma unroll
-        for (int a = 0; a < kTR; ++a)
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int b = 0; b < kTC; ++b)
+            for (int e = 0; e < 4; ++e) {
+                const int i = g.nu / 2 + p1 + 16 * rt + 4 * e + k, j = g.nv / 2 + p2 + 16 * (ct + c) + q;
+                if (i >= g.nu || j >= g.nv) continue;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int i = i0 + 16 * a + 4 * e + k, j = j0 + 16 * b + q;
-                    if (i < g.nu && j < g.nv) dst[(size_t)i * g.nv + j] = make_double2(cr[a][b][e], ci[a][b][e]);
+                for (int sg = 0; sg < 4; ++sg) {
+                    const double s1 = sg & 2 ? -1.0 : 1.0, s2 = sg & 1 ? -1.0 : 1.0;
+                    const double re = ar[c][0][e] - s1 * s2 * ar[c][3][e] - (s1 * ai[c][1][e] + s2 * ai[c][2][e]);
+                    const double im = ai[c][0][e] - s1 * s2 * ai[c][3][e] + (s1 * ar[c][1][e] + s2 * ar[c][2][e]);
+                    const int ii = sg & 2 ? g.nu - 1 - i : i, jj = sg & 1 ? g.nv - 1 - j : j;
+                    dst[(size_t)ii * g.nv + jj] = make_double2(re, im);   // an odd length's centre: the same value twice
                 }
+            }
     }
-}
-
-// out[n] = sum over the ranges (in order) of the partial sums, in the caller's flattening.
-__global__ __launch_bounds__(kThreads) void k_ndft_grid_sum(const double2 *__restrict__ part, int ranges,
-                                                            double2 *__restrict__ out, int N)
-{
-    const GridInfo g = g_grid;
-    if (!g.ok) return;
-    const int n = blockIdx.x * kThreads + threadIdx.x;
-    if (n >= N) return;
-    const int i = g.vmajor ? n % g.nu : n / g.nv, j = g.vmajor ? n / g.nu : n % g.nv;
-    const size_t e = (size_t)i * g.nv + j;
-    double sr = 0.0, si = 0.0;
-    for (int r = 0; r < ranges; ++r) {
-        const double2 v = part[(size_t)r * N + e];
-        sr += v.x;
-        si += v.y;
-    }
-    out[n] = make_double2(sr, si);
 }
 
 // The partial sums' workspace, one per device, grown as needed (the
@@ -319,39 +370,39 @@ struct GridWs {
 std::mutex g_ws_mu;
 std::map<int, GridWs> g_ws;
 
-__global__ __launch_bounds__(kThreads) void k_ndft_direct(const double *__restrict__ X, const double *__restrict__ Y,
-                                                          const double *__restrict__ u, const double *__restrict__ v,
-                                                          const double2 *__restrict__ in, double2 *__restrict__ out,
-                                                          double inv_Nu, double inv_Nv, int M, int N)
+// out[n] = sum over the ranges (in a fixed order) of the partial sums, in the
+// caller's flattening: 64 outputs per block, 4 threads each over every fourth
+// range.
+constexpr int kSumOut = 64;
+__global__ __launch_bounds__(kThreads) void k_ndft_finish(const double2 *__restrict__ part, int ranges,
+                                                          double2 *__restrict__ out, int N)
 {
-    if (g_grid.ok) return;         // k_ndft_grid wrote the outputs
-    __shared__ double sX[kThreads], sY[kThreads];
-    __shared__ double2 sIn[kThreads];
-    const int n = blockIdx.x * kThreads + threadIdx.x;
-    const double un = n < N ? u[n] * inv_Nu : 0.0;
-    const double vn = n < N ? v[n] * inv_Nv : 0.0;
-    double ar = 0.0, ai = 0.0;
-    for (int m0 = 0; m0 < M; m0 += kThreads) {
-        const int m = m0 + threadIdx.x;
-        if (m < M) {
-            sX[threadIdx.x] = X[m];
-            sY[threadIdx.x] = Y[m];
-            sIn[threadIdx.x] = in[m];
+    const GridInfo g = g_grid;
+    __shared__ double2 s_sum[kThreads / kSumOut - 1][kSumOut];
+    const int o = threadIdx.x % kSumOut, sl = threadIdx.x / kSumOut, n = blockIdx.x * kSumOut + o;
+    double sr = 0.0, si = 0.0;
+    if (n < N) {
+        size_t e = n;
+        if (g.ok) {
+            const int i = g.vmajor ? n % g.nu : n / g.nv, j = g.vmajor ? n / g.nu : n % g.nv;
+            e = (size_t)i * g.nv + j;
         }
-        __syncthreads();
-        const int cnt = min(kThreads, M - m0);
-        for (int q = 0; q < cnt; ++q) {
-            double t = un * sX[q] + vn * sY[q];
-            t -= floor(t);
-            double s, c;
-            sincospi(2.0 * t, &s, &c);   // e^{-2 pi i t} = c - i s
-            const double2 d = sIn[q];
-            ar += d.x * c + d.y * s;
-            ai += d.y * c - d.x * s;
+        const double2 *src = part + e;
+#pragma unroll 4
+        for (int r = sl; r < ranges; r += kThreads / kSumOut) {
+            const double2 p = src[(size_t)r * N];
+            sr += p.x;
+            si += p.y;
         }
-        __syncthreads();
     }
-    if (n < N) out[n] = make_double2(ar, ai);
+    if (sl > 0) s_sum[sl - 1][o] = make_double2(sr, si);
+    __syncthreads();
+    if (sl > 0 || n >= N) return;
+    for (int h = 0; h < kThreads / kSumOut - 1; ++h) {
+        sr += s_sum[h][o].x;
+        si += s_sum[h][o].y;
+    }
+    out[n] = make_double2(sr, si);
 }
 
 }  // namespace
@@ -365,14 +416,14 @@ extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, cons
     if (N == 0) return NFFT2D_OK;
     if (!u || !v || !out || (M > 0 && (!X || !Y || !in)))
         return nfft2d_fail(NFFT2D_ERR_ARG, "NDFT2_2D_GPU: null pointer");
-    // (u, v) a grid: FP64 MFMA contraction; otherwise the direct sum (each kernel
-    // reads the detector's finding and returns at once when it is not its case)
-    // point ranges: enough work items for the whole chip at the supertile count a
-    // square grid of N outputs would have, each range at least 16 points
-    const long long nsup_est = std::max<long long>(1, (long long)N / (kSupRows * kSupCols));
-    int ranges = (int)std::min<long long>(kMaxRanges, std::max<long long>(1, kGridWavesTotal / nsup_est));
-    ranges = std::max(1, std::min(ranges, (M + 15) / 16));
-    const int chunk = ((M + ranges - 1) / ranges + 3) & ~3;   // a multiple of 4 points
+    // (u, v) a grid: FP64 MFMA contraction; otherwise the direct sum (k_ndft_grid
+    // reads the detector's finding and does one or the other).
+    // Point ranges: a work item per CU at the tile count a square grid of N
+    // outputs would have, each range at least one chunk of points.
+    const long long ntile_est = std::max<long long>(1, (long long)N / (4 * kTilePairs * kTilePairs));
+    int ranges = (int)std::max<long long>(1, kGridBlocks / ntile_est);
+    ranges = std::max(1, std::min(ranges, (M + kGridChunk - 1) / kGridChunk));
+    const int chunk = ((M + ranges - 1) / ranges + kGridChunk - 1) / kGridChunk * kGridChunk;
     const int dev = [] { int d = 0; (void)hipGetDevice(&d); return d; }();
     double2 *part = nullptr;
     // held until the launches are queued: a call from another host thread that
@@ -380,8 +431,8 @@ extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, cons
     std::lock_guard<std::mutex> lk(g_ws_mu);
     {
         GridWs &ws = g_ws[dev];
-        // partial sums, then (from an even double2 index: 32-byte aligned) the steps
-        const size_t need = (((size_t)ranges * (size_t)N + 1) & ~(size_t)1) + 2 * (size_t)M;
+        // partial sums, then the prepared points
+        const size_t need = (size_t)ranges * (size_t)N + sizeof(GridPt) / sizeof(double2) * (size_t)M;
         if (ws.count < need) {
             if (ws.ptr) {
                 (void)hipDeviceSynchronize();
@@ -398,25 +449,19 @@ extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, cons
         }
         part = ws.ptr;
     }
-    double4 *steps = reinterpret_cast<double4 *>(part + (((size_t)ranges * (size_t)N + 1) & ~(size_t)1));
+    GridPt *pts = reinterpret_cast<GridPt *>(part + (size_t)ranges * (size_t)N);
+    const double2 *din = reinterpret_cast<const double2 *>(in);
     hipLaunchKernelGGL(k_grid_detect, dim3(1), dim3(kDetThreads), 0, nullptr, u, v, N);
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_grid_verify, dim3((N + kThreads - 1) / kThreads), dim3(kThreads), 0, nullptr, u, v, N);
+    const int nver = (N + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(k_grid_verify, dim3(nver + (M + kThreads - 1) / kThreads), dim3(kThreads), 0, nullptr, u, v, N,
+                       nver, X, Y, din, 1.0 / Nu, 1.0 / Nv, M, pts);
     NFFT2D_LAUNCH_CHECK();
-    if (M > 0) {
-        hipLaunchKernelGGL(k_ndft_steps, dim3((M + kThreads - 1) / kThreads), dim3(kThreads), 0, nullptr, X, Y,
-                           1.0 / Nu, 1.0 / Nv, M, steps);
-        NFFT2D_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(k_ndft_grid, dim3(kGridWavesTotal / 4), dim3(256), 0, nullptr, X, Y,
-                       reinterpret_cast<const double2 *>(in), steps, part, 1.0 / Nu, 1.0 / Nv, M, ranges, chunk);
+    hipLaunchKernelGGL(k_ndft_grid, dim3(kGridBlocks), dim3(kGridThreads), 0, nullptr, pts, part, M, ranges, chunk, X, Y,
+                       u, v, din, 1.0 / Nu, 1.0 / Nv, N);
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_ndft_grid_sum, dim3((N + kThreads - 1) / kThreads), dim3(kThreads), 0, nullptr, part, ranges,
+    hipLaunchKernelGGL(k_ndft_finish, dim3((N + kSumOut - 1) / kSumOut), dim3(kThreads), 0, nullptr, part, ranges,
                        reinterpret_cast<double2 *>(out), N);
-    NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_ndft_direct, dim3((N + kThreads - 1) / kThreads), dim3(kThreads), 0, nullptr, X, Y, u, v,
-                       reinterpret_cast<const double2 *>(in), reinterpret_cast<double2 *>(out), 1.0 / Nu, 1.0 / Nv, M,
-                       N);
     NFFT2D_LAUNCH_CHECK();
     return NFFT2D_OK;
 }
