@@ -144,11 +144,12 @@ int nfft2d_setpts(nfft2d_plan *plan, const void *x, const void *y, int M, void *
 
 /* Type-2: result[l] = sum_k data[k] e^{-2 pi i k.x_l / N}  (result: M, data: N1*N2). */
 int nfft2d_type2(nfft2d_plan *plan, void *result, const void *data, void *stream);
-/* nfft2d_setpts followed by nfft2d_type2, with the tile sort on a second
+/* nfft2d_setpts followed by nfft2d_type2; where it pays (large grids in a
+ * captured graph, large chirp-z grids otherwise) the tile sort runs on a second
  * stream owned by the plan, concurrent with the grid passes (pre-compensation,
- * zero padding, FFT) on `stream`; the gather waits for both.  Everything stays
- * ordered on `stream` for the caller and can be captured into a hipGraph (the
- * first call creates the second stream: make it outside a capture).  The
+ * zero padding, FFT) on `stream`, and the gather waits for both.  Everything
+ * stays ordered on `stream` for the caller and can be captured into a hipGraph
+ * (the first call creates the second stream: make it outside a capture).  The
  * one-call form of the reference's type-2 (BP_FBP_FFBP/NFFT1_2D.m), which
  * NFFT1_2D_GPU_c64 / _c128 use. */
 int nfft2d_setpts_type2(nfft2d_plan *plan, void *result, const void *data, const void *x, const void *y, int M,

@@ -602,9 +602,13 @@ static int setpts_impl(nfft2d_plan *p, const T *x, const T *y, int M, hipStream_
     setpts_blocking(p, M, nblk, chunk);
     const bool lds = p->nbins <= kMaxLdsBins;
     const T inv1 = (T)(1.0 / p->L1), inv2 = (T)(1.0 / p->L2);
-    if (lds) {
+    const bool one = p->nbins <= kSmallBins && M <= kOnePts;
+    const bool small = one || (p->nbins <= kSmallBins && (long long)nblk * p->nbins <= kSmallHist);
+    if (one) {
+        // counted by the scatter block
+    } else if (lds) {
         hipLaunchKernelGGL(k_hist<T>, dim3(nblk), dim3(kHistThreads), sizeof(int) * p->nbins, s, x, y, M, chunk, p->L1,
-                           p->L2, inv1, inv2, p->nb1, p->nbins, p->hist, (int *)nullptr);
+                           p->L2, inv1, inv2, p->nb1, p->nbins, p->hist);
     } else {
         int rc = zero_fill<int>(p->hist, p->nbins, s);
         if (rc) return rc;
@@ -614,10 +618,18 @@ static int setpts_impl(nfft2d_plan *p, const T *x, const T *y, int M, hipStream_
     }
     NFFT2D_LAUNCH_CHECK();
     const int ngroups = (int)grid1d(p->nbins, kColBins);
-    hipLaunchKernelGGL(k_colscan, dim3(ngroups), dim3(256), 0, s, p->hist, nblk, p->nbins, p->maxpts, p->tot, p->gexcl,
-                       p->gsum);
-    NFFT2D_LAUNCH_CHECK();
-    if (lds) {
+    if (!small) {
+        hipLaunchKernelGGL(k_colscan, dim3(ngroups), dim3(256), 0, s, p->hist, nblk, p->nbins, p->maxpts, p->tot,
+                           p->gexcl, p->gsum);
+        NFFT2D_LAUNCH_CHECK();
+    }
+    if (small) {
+        auto kern = one ? k_scatter_small<T, true> : k_scatter_small<T, false>;
+        hipLaunchKernelGGL(kern, dim3(one ? 1 : nblk), dim3(kScatThreads), sizeof(int) * 2 * p->nbins, s, x, y, M,
+                           one ? std::max(M, 1) : chunk, p->L1, p->L2, inv1, inv2, p->nb1, p->nbins, p->maxpts, p->hist,
+                           p->tot, (PtRec<T> *)p->pts, p->subbeg, p->sub, p->nsub);
+        NFFT2D_LAUNCH_CHECK();
+    } else if (lds) {
         // ranks recomputed by the scatter blocks, which take the histogram blocks' points
         hipLaunchKernelGGL(k_scatter_lds<T>, dim3(nblk), dim3(kScatThreads), 0, s, x, y, M, chunk, p->L1, p->L2, inv1,
                            inv2, p->nb1, p->nbins, p->maxpts, p->hist, p->tot, p->gexcl, p->gsum, ngroups,
@@ -918,8 +930,30 @@ extern "C" int nfft2d_type2(nfft2d_plan *p, void *result, const void *data, void
     return nfft2d_type2_interp(p, result, stream);
 }
 
-// setpts + type-2 with the bin sort on the plan's second stream, concurrent
-// with the grid passes on `stream`; the gather waits for both.
+// Whether setpts_type2 runs the bin sort beside the grid passes.  The fork and
+// the join cost about 15 us of an eager call (two event records and waits
+// between the launches), more than the overlap saves where each branch fills
+// the chip or is a few launches long: two streams against one, eager, 128^2 /
+// 16K points 54.9 / 26.8 us, 512^2 / 1M 81.9 / 71.2, 1024^2 / 4M 216 / 214.
+// The chirp-z passes of large grids leave room beside them: 500^2 / 300K 78.1
+// / 81.5, 1000^2 / 1M 212 / 224.  In a captured graph the branches cost less:
+// 256^2 / 64K 38.8 / 36.1, 512^2 / 1M 71.0 / 76.1, 1024^2 / 4M 205 / 219.
+static bool fork_pays(const nfft2d_plan *p, hipStream_t s)
+{
+    const long long modes = (long long)p->N1 * p->N2;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
+        (void)hipGetLastError();
+        cs = hipStreamCaptureStatusNone;
+    }
+    if (cs == hipStreamCaptureStatusActive) return modes >= 1 << 18;
+    return (p->czt[0] || p->czt[1]) && modes >= 200000;
+}
+
+// setpts + type-2, in large cases (fork_pays) with the bin sort on the plan's
+// second stream, concurrent with the grid passes on `stream`; the gather waits
+// for both.  The second stream is made at the first call in any case, so that
+// a later captured one finds it.
 extern "C" int nfft2d_setpts_type2(nfft2d_plan *p, void *result, const void *data, const void *x, const void *y, int M,
                                    void *stream)
 {
@@ -933,7 +967,12 @@ extern "C" int nfft2d_setpts_type2(nfft2d_plan *p, void *result, const void *dat
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     rc = p->fk.init(p->device);
-    if (rc || (rc = p->fk.fork(s))) return rc;
+    if (rc) return rc;
+    if (!fork_pays(p, s)) {
+        if ((rc = nfft2d_setpts(p, x, y, M, stream))) return rc;
+        return nfft2d_type2(p, result, data, stream);
+    }
+    if ((rc = p->fk.fork(s))) return rc;
     rc = nfft2d_setpts(p, x, y, M, p->fk.aux);
     const int rg = rc ? NFFT2D_OK : nfft2d_type2_grid(p, data, stream);
     const int rj = p->fk.join(s);               // always rejoin, so that a capture stays well formed

@@ -105,8 +105,7 @@ __global__ __launch_bounds__(kHistThreads) void kb_hist(const BatchDesc* __restr
     extern __shared__ int h[];
     const int2 o = own[blockIdx.x];
     const BatchDesc& d = bd[o.x];
-    // no per-point rank: kb_scatter_lds ranks the points again in LDS
-    hist_body<float>(o.y, h, d.x, d.y, d.M, d.chunk, d.L1, d.L2, d.inv1, d.inv2, d.nb1, d.nbins, d.hist, nullptr);
+    hist_body<float>(o.y, h, d.x, d.y, d.M, d.chunk, d.L1, d.L2, d.inv1, d.inv2, d.nb1, d.nbins, d.hist);
 }
 
 __global__ __launch_bounds__(256) void kb_colscan(const BatchDesc* __restrict__ bd, const int2* __restrict__ own)

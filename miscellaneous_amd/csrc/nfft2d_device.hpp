@@ -149,8 +149,7 @@ __device__ __forceinline__ void locate(T x, int L, T invL, int& mu_wrapped, T& t
     }
     const T mu = rint(cx);
     t = cx - mu;
-    const int mi = (int)mu;
-    int r = mi - (int)floor(mu * invL) * L;
+    int r = (int)fma(-floor(mu * invL), (T)L, mu);   // an integer of a few L: the fma is exact
     while (r < 0) r += L;      // the estimate is exact or one off except for |c x| >~ 2^24
     while (r >= L) r -= L;
     mu_wrapped = r;

@@ -719,14 +719,17 @@ __device__ __forceinline__ int wave_run_rank(int* counter, int bin, bool act)
 }
 
 // Pass 1: block b counts the bins of points [b*chunk, (b+1)*chunk) in an LDS
-// histogram (integer LDS atomics, one per run of equal bins in a wave);
-// rank[i] is the point's rank inside its (block, bin), written unless rank is
-// null (k_scatter_lds recomputes it).  hist is [nblk][nbins].
+// histogram (one integer LDS atomic per point; nothing waits for its result,
+// so runs of equal bins need no aggregation: a wave's 64 increments of one
+// address are 64 cycles of the LDS atomic unit, less than the run search
+// costs the four SIMDs: 4M uniform points on 1024^2 modes 32 -> 20 us, 1M
+// polar points on 512^2 8.4 -> 8.1 us).  The scatter ranks the points again
+// in LDS.  hist is [nblk][nbins].
 constexpr int kHistThreads = 1024;   // 16 waves per block: 4 per SIMD to hide the load latency
 template <typename T>
 __device__ __forceinline__ void hist_body(int blk, int* h, const T* __restrict__ x, const T* __restrict__ y, int M,
                                           int chunk, int L1, int L2, T inv1, T inv2, int nb1, int nbins,
-                                          int* __restrict__ hist, int* __restrict__ rank)
+                                          int* __restrict__ hist)
 {
     for (int i = threadIdx.x; i < nbins; i += kHistThreads) h[i] = 0;
     __syncthreads();
@@ -746,12 +749,10 @@ __device__ __forceinline__ void hist_body(int blk, int* h, const T* __restrict__
 #pragma unroll
         for (int q = 0; q < kHistBatch; ++q) {
             const int i = b + q * kHistThreads + (int)threadIdx.x;
-            const bool act = i < hi;
             int m1, m2;
             T t1, t2;
             const int bin = bin_of(xv[q], yv[q], L1, L2, inv1, inv2, nb1, m1, m2, t1, t2);
-            const int r = wave_run_rank(h, bin, act);
-            if (act && rank != nullptr) rank[i] = r;
+            if (i < hi) atomicAdd(&h[bin], 1);
         }
     }
     __syncthreads();
@@ -761,10 +762,10 @@ __device__ __forceinline__ void hist_body(int blk, int* h, const T* __restrict__
 template <typename T>
 __global__ __launch_bounds__(kHistThreads) void k_hist(const T* __restrict__ x, const T* __restrict__ y, int M, int chunk,
                                                        int L1, int L2, T inv1, T inv2, int nb1, int nbins,
-                                                       int* __restrict__ hist, int* __restrict__ rank)
+                                                       int* __restrict__ hist)
 {
     extern __shared__ int h[];
-    hist_body<T>(blockIdx.x, h, x, y, M, chunk, L1, L2, inv1, inv2, nb1, nbins, hist, rank);
+    hist_body<T>(blockIdx.x, h, x, y, M, chunk, L1, L2, inv1, inv2, nb1, nbins, hist);
 }
 
 // Pass 1 for grids with more than kMaxLdsBins bins: one logical block, global
@@ -1099,6 +1100,130 @@ __global__ __launch_bounds__(kScatThreads) void k_scatter_lds(
 #pragma unroll
         for (int q = 0; q < kScatPer; ++q) {
             const int i = b0 + q * kScatThreads + t;
+            const bool act = i < hi;
+            int m1, m2;
+            T t1, t2;
+            const int bin = bin_of(xv[q], yv[q], L1, L2, inv1, inv2, nb1, m1, m2, t1, t2);
+            const int p = wave_run_rank(base, bin, act);
+            if (act) {
+                PtRec<T> rec;
+                rec.t1 = t1;
+                rec.t2 = t2;
+                rec.cell = (m2 << 16) | m1;
+                rec.idx = i;
+                pts[p] = rec;
+            }
+        }
+    }
+}
+
+// Small point sets: the whole scan in the scatter block, from the histogram
+// rows themselves (at most kSmallHist counts, kSmallBins bins), so that no
+// k_colscan launch stands between k_hist and the scatter; with ONE (one block,
+// at most kOnePts points) the block also counts its points, and the sort is
+// this launch alone.  At these sizes the three launches' fixed costs and
+// dependent loads are the sort's time: 1,936 points on 88^2 modes 14.8 us in
+// three launches, 7.9 in one; 16,384 points on 128^2 16.9 -> 12.3 us in two.
+// Writes tot, subbeg, sub and nsub as k_colscan and k_scatter_lds do.
+constexpr int kOnePts = kScatThreads * kScatPer;      // one batch of the block's points, held in registers
+constexpr int kSmallBins = 4096, kSmallHist = 32768;
+template <typename T, bool ONE>
+__global__ __launch_bounds__(kScatThreads) void k_scatter_small(
+    const T* __restrict__ x, const T* __restrict__ y, int M, int chunk, int L1, int L2, T inv1, T inv2, int nb1,
+    int nbins, int maxpts, const int* __restrict__ hist, int* __restrict__ tot, PtRec<T>* __restrict__ pts,
+    int* __restrict__ subbeg, int4* __restrict__ sub, int* __restrict__ nsub)
+{
+    extern __shared__ int small_lds[];
+    int *base = small_lds, *tl = small_lds + nbins;       // positions, totals of the bins
+    __shared__ int w_a[kScatThreads / 64], w_b[kScatThreads / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int nblk = ONE ? 1 : (int)gridDim.x, blk = ONE ? 0 : (int)blockIdx.x;
+    const int lo = blk * chunk, hi = min(lo + chunk, M);
+    T xv[kScatPer], yv[kScatPer];
+#pragma unroll
+    for (int q = 0; q < kScatPer; ++q) {
+        const int i = lo + q * kScatThreads + t;
+        xv[q] = i < hi ? x[i] : (T)0;
+        yv[q] = i < hi ? y[i] : (T)0;
+    }
+    if constexpr (ONE) {
+        for (int b = t; b < nbins; b += kScatThreads) base[b] = tl[b] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < kScatPer; ++q) {
+            const int i = lo + q * kScatThreads + t;
+            int m1, m2;
+            T t1, t2;
+            const int bin = bin_of(xv[q], yv[q], L1, L2, inv1, inv2, nb1, m1, m2, t1, t2);
+            if (i < hi) atomicAdd(&tl[bin], 1);
+        }
+    } else {
+        for (int b = t; b < nbins; b += kScatThreads) {
+            int before = 0, all = 0;
+            for (int k0 = 0; k0 < nblk; k0 += 8) {
+                int v[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = k0 + k < nblk ? hist[(size_t)(k0 + k) * nbins + b] : 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    all += v[k];
+                    before += k0 + k < blk ? v[k] : 0;
+                }
+            }
+            base[b] = before;
+            tl[b] = all;
+        }
+    }
+    __syncthreads();
+    // exclusive scan of (points, subproblems) over the bins, a run of bins per thread
+    const int per = (nbins + kScatThreads - 1) / kScatThreads;
+    const int b0 = min(t * per, nbins), b1 = min(b0 + per, nbins);
+    int va = 0, vb = 0;
+    for (int b = b0; b < b1; ++b) {
+        va += tl[b];
+        vb += (tl[b] + maxpts - 1) / maxpts;
+    }
+    int ia = va, ib = vb;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int na = __shfl_up(ia, o, 64), nb = __shfl_up(ib, o, 64);
+        if (lane >= o) { ia += na; ib += nb; }
+    }
+    if (lane == 63) { w_a[w] = ia; w_b[w] = ib; }
+    __syncthreads();
+    int pa = ia - va, pb = ib - vb;
+    for (int k = 0; k < w; ++k) { pa += w_a[k]; pb += w_b[k]; }
+    // subproblem lists: an even share of the bins per block
+    const int bpb = (nbins + nblk - 1) / nblk;
+    const int blo = blk * bpb, bhi = min(blo + bpb, nbins);
+    for (int b = b0; b < b1; ++b) {
+        const int c = tl[b], ns = (c + maxpts - 1) / maxpts;
+        base[b] += pa;
+        if (b >= blo && b < bhi) {
+            tot[b] = c;
+            subbeg[b] = pb;
+            for (int k = 0; k < ns; ++k) sub[pb + k] = make_int4(b, pa + k * maxpts, min(maxpts, c - k * maxpts), 0);
+        }
+        pa += c;
+        pb += ns;
+    }
+    if (blk == 0 && t == kScatThreads - 1) {
+        *nsub = pb;
+        subbeg[nbins] = pb;
+    }
+    __syncthreads();
+    for (int q0 = lo; q0 < hi; q0 += kScatPer * kScatThreads) {
+        if (q0 != lo) {
+#pragma unroll
+            for (int q = 0; q < kScatPer; ++q) {
+                const int i = q0 + q * kScatThreads + t;
+                xv[q] = i < hi ? x[i] : (T)0;
+                yv[q] = i < hi ? y[i] : (T)0;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kScatPer; ++q) {
+            const int i = q0 + q * kScatThreads + t;
             const bool act = i < hi;
             int m1, m2;
             T t1, t2;

@@ -161,9 +161,9 @@ class Plan:
 
     def setpts_type2(self, x: torch.Tensor, y: torch.Tensor, f: torch.Tensor,
                      out: torch.Tensor | None = None) -> torch.Tensor:
-        """setpts(x, y) then type2(f): the tile sort runs on the plan's second
-        stream, concurrent with the grid passes; the result is ordered on
-        torch's current stream."""
+        """setpts(x, y) then type2(f) in one call; on large grids the tile sort
+        may run on the plan's second stream, concurrent with the grid passes;
+        the result is ordered on torch's current stream."""
         M = x.numel()
         _require(x, self.rdtype, M, "x", self.device)
         _require(y, self.rdtype, M, "y", self.device)
