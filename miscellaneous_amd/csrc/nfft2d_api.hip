@@ -240,7 +240,7 @@ struct nfft2d_plan_s {
     WinArgs wa;
     Fork fk;                              // setpts beside the grid passes (nfft2d_setpts_type2)
     // chirp-z tables of a dimension whose N is not a power of two (null otherwise):
-    // [cin2 N][cout2 2N][hhat2 m][cin1 2N][cout1 N][hhat1 m][T1 m/64][T2 64]
+    // [cin2 N][cout2 2N][hhat2 m][cin1 2N][cout1 N][hhat1 m][tw m]
     void *czt[2] = {nullptr, nullptr};
     int cztm[2] = {0, 0};
 };
@@ -333,19 +333,19 @@ static void host_fft(std::vector<std::complex<double>> &a)
 // host: c[k] = e^{-i pi k^2 / L}, L = 2N (k^2 reduced mod 2L exactly); type-2
 // passes p0 = -N/2, q0 = 0 (P = N, Q = L), type-1 passes p0 = 0, q0 = -N/2
 // (P = L, Q = N); the kernel conj(c[d + q0 - p0]) at d mod m, d in [1 - P, Q),
-// transformed; the FFT's two twiddle tables.
+// transformed; the FFT's twiddles.
 template <typename T>
 static int czt_buffer(int N, void **out, int *mout)
 {
     using C = cplx<T>;
-    const int L = 2 * N, m = czt_m(N), nt1 = m >= 64 ? m / 64 : 1;
+    const int L = 2 * N, m = czt_m(N);
     auto chirp = [&](long long k) {
         const long long q = ((k * k) % (2LL * L) + 2LL * L) % (2LL * L);
         const double ang = -kPi * (double)q / (double)L;
         return std::complex<double>(std::cos(ang), std::sin(ang));
     };
     std::vector<C> h;
-    h.reserve((size_t)3 * L + 2 * (size_t)m + nt1 + 64);
+    h.reserve((size_t)3 * L + 3 * (size_t)m);
     auto put = [&](std::complex<double> v) {
         C c;
         c.x = (T)v.real();
@@ -362,8 +362,7 @@ static int czt_buffer(int N, void **out, int *mout)
     };
     pass(N, L, -N / 2, 0);   // type-2
     pass(L, N, 0, -N / 2);   // type-1
-    for (int j = 0; j < nt1; ++j) put(std::polar(1.0, -2.0 * kPi * 64.0 * j / m));
-    for (int j = 0; j < 64; ++j) put(std::polar(1.0, -2.0 * kPi * (double)j / m));
+    for (int j = 0; j < m; ++j) put(std::polar(1.0, -2.0 * kPi * (double)j / m));
     if (nfft2d_malloc(out, sizeof(C) * h.size()) != hipSuccess)
         return nfft2d_fail(NFFT2D_ERR_ALLOC, "plan tables: hipMalloc of the chirp-z tables failed");
     NFFT2D_HIP_TRY(hipMemcpy(*out, h.data(), sizeof(C) * h.size(), hipMemcpyHostToDevice));
@@ -382,33 +381,36 @@ static CztTables<T> czt_tables(const nfft2d_plan *p, int dim, bool t2)
     return czt_tables_of<T>(p->czt[dim], dim == 0 ? p->N1 : p->N2, p->cztm[dim], t2);
 }
 
-// Launches one chirp-z pass: `lines` lines (one block each).
-template <typename T, int SIGN, bool SCALE_IN, int U>
-static int czt_launch_u(const CztTables<T> &tb, int lines, const cplx<T> *in, long long in_ls, long long in_es,
-                        cplx<T> *out, long long out_ls, long long out_es, const T *sl, const T *se, hipStream_t s)
+// Launches one chirp-z pass over `lines` lines: MODE 0 both sides contiguous
+// along a line, 1 the input's lines side by side (in_ls = 1), 2 the output's.
+template <typename T, int LOGM, int MODE>
+static int czt_launch_m(const CztTables<T> &tb, int lines, const cplx<T> *in, long long in_ls, long long in_es,
+                        cplx<T> *out, long long out_ls, long long out_es, const T *sl, const T *se, bool scale_in,
+                        bool conj, hipStream_t s)
 {
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
-    std::call_once(once, [] {
-        attr = hipFuncSetAttribute((const void *)k_czt<T, SIGN, SCALE_IN, U>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(sizeof(cplx<T>) * czt_lds_entries(czt_m(kCztMaxN<T>))));
+    auto kern = k_czt<T, LOGM, MODE == 1, MODE == 2>;
+    constexpr int bytes = czt_lds_bytes<T, LOGM, MODE != 0>();
+    std::call_once(once, [&] {
+        attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     });
     if (attr != hipSuccess) return nfft2d_fail(NFFT2D_ERR_HIP, "chirp-z pass: %s", hipGetErrorString(attr));
-    const int nt = std::min(1024, std::max(64, tb.m / 4));
-    hipLaunchKernelGGL((k_czt<T, SIGN, SCALE_IN, U>), dim3(lines), dim3(nt), sizeof(cplx<T>) * czt_lds_entries(tb.m),
-                       s, in, in_ls, in_es, out, out_ls, out_es, sl, se, tb);
+    constexpr int B = czt_block_lines<LOGM, MODE != 0>();
+    const unsigned blocks = ((unsigned)(lines + B - 1) / B + 7) & ~7u;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(czt_threads<LOGM, MODE != 0>()), bytes, s, in, in_ls, in_es, out, out_ls, out_es,
+                       sl, se, scale_in, conj, lines, tb);
     NFFT2D_LAUNCH_CHECK();
     return NFFT2D_OK;
 }
-template <typename T, int SIGN, bool SCALE_IN>
-static int czt_launch(const CztTables<T> &tb, int lines, const cplx<T> *in, long long in_ls, long long in_es,
-                      cplx<T> *out, long long out_ls, long long out_es, const T *sl, const T *se, hipStream_t s)
+template <typename T, int MODE, int LOGM = kCztMinLog, typename... A>
+static int czt_launch(const CztTables<T> &tb, A... a)
 {
-    // at 1024 threads a thread holds 8 values up to m = 8192, 16 at m = 16384
-    if (tb.m > 8192)
-        return czt_launch_u<T, SIGN, SCALE_IN, 4>(tb, lines, in, in_ls, in_es, out, out_ls, out_es, sl, se, s);
-    return czt_launch_u<T, SIGN, SCALE_IN, 2>(tb, lines, in, in_ls, in_es, out, out_ls, out_es, sl, se, s);
+    if (tb.m == 1 << LOGM) return czt_launch_m<T, LOGM, MODE>(tb, a...);
+    if constexpr (LOGM < kCztMaxLog && (1 << LOGM) < czt_m(kCztMaxN<T>))
+        return czt_launch<T, MODE, LOGM + 1>(tb, a...);
+    else
+        return nfft2d_fail(NFFT2D_ERR_SIZE, "chirp-z pass: no transform of %d points", tb.m);
 }
 
 template <typename T>
@@ -709,7 +711,7 @@ static int t2_grid(nfft2d_plan *p, const void *data, hipStream_t s)
             }
         });
     } else if (p->czt[1]) {   // rows: f[k1][*] (N2) -> Tm[k1][*] (L2), pre-compensated
-        int rc = czt_launch<T, -1, true>(czt_tables<T>(p, 1, true), p->N1, f, p->N2, 1, Tm, p->L2, 1, D1, D2, s);
+        int rc = czt_launch<T, 0>(czt_tables<T>(p, 1, true), p->N1, f, p->N2, 1, Tm, p->L2, 1, D1, D2, true, false, s);
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL((k_t2_rows_direct<T, -1>), dim3(p->N1), dim3(256), sizeof(C) * 3 * p->N2, s, f, Tm, D1, D2, tw2,
@@ -726,8 +728,8 @@ static int t2_grid(nfft2d_plan *p, const void *data, hipStream_t s)
             }
         });
     } else if (p->czt[0]) {   // columns: Tm[*][n2] (N1) -> G[n2][*] (L1)
-        int rc = czt_launch<T, -1, true>(czt_tables<T>(p, 0, true), p->L2, Tm, 1, p->L2, G, p->L1, 1, (const T *)nullptr,
-                                         (const T *)nullptr, s);
+        int rc = czt_launch<T, 1>(czt_tables<T>(p, 0, true), p->L2, Tm, 1, p->L2, G, p->L1, 1, (const T *)nullptr,
+                                  (const T *)nullptr, true, false, s);
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL((k_t2_cols_direct<T, -1>), dim3(p->L2), dim3(256), sizeof(C) * 3 * p->N1, s, Tm, G, tw1, p->N1,
@@ -763,8 +765,8 @@ static int t1_passes(nfft2d_plan *p, void *result, hipStream_t s)
             }
         });
     } else if (p->czt[0]) {   // columns: G[n2][*] (L1) -> Tp[*][n2] (N1)
-        int rc = czt_launch<T, SIGN, false>(czt_tables<T>(p, 0, false), p->L2, G, p->L1, 1, Tp, 1, p->L2,
-                                            (const T *)nullptr, (const T *)nullptr, s);
+        int rc = czt_launch<T, 2>(czt_tables<T>(p, 0, false), p->L2, G, p->L1, 1, Tp, 1, p->L2, (const T *)nullptr,
+                                  (const T *)nullptr, false, SIGN > 0, s);
         if (rc) return rc;
     } else if (t1_plan_mfma<T>(p->N1)) {
         hipLaunchKernelGGL((k_t1_cols_mm<SIGN>), dim3(grid1d(p->L2, 16), grid1d(p->N1, 16)), dim3(256), 0, s, (const float2 *)G,
@@ -784,7 +786,8 @@ static int t1_passes(nfft2d_plan *p, void *result, hipStream_t s)
             }
         });
     } else if (p->czt[1]) {   // rows: Tp[k1][*] (L2) -> F[k1][*] (N2), deconvolved
-        int rc = czt_launch<T, SIGN, false>(czt_tables<T>(p, 1, false), p->N1, Tp, p->L2, 1, F, p->N2, 1, D1, D2, s);
+        int rc = czt_launch<T, 0>(czt_tables<T>(p, 1, false), p->N1, Tp, p->L2, 1, F, p->N2, 1, D1, D2, false, SIGN > 0,
+                                  s);
         if (rc) return rc;
     } else if (t1_plan_mfma<T>(p->N2)) {
         hipLaunchKernelGGL((k_t1_rows_mm<SIGN>), dim3(grid1d(p->N1, 16), grid1d(p->N2, 16)), dim3(256), 0, s, (const float2 *)Tp,
@@ -935,8 +938,8 @@ extern "C" int nfft2d_type2(nfft2d_plan *p, void *result, const void *data, void
 // between the launches), more than the overlap saves where each branch fills
 // the chip or is a few launches long: two streams against one, eager, 128^2 /
 // 16K points 54.9 / 26.8 us, 512^2 / 1M 81.9 / 71.2, 1024^2 / 4M 216 / 214.
-// The chirp-z passes of large grids leave room beside them: 500^2 / 300K 78.1
-// / 81.5, 1000^2 / 1M 212 / 224.  In a captured graph the branches cost less:
+// The chirp-z passes of large grids leave room beside them: 500^2 / 300K 79.2
+// / 74.1, 1000^2 / 1M 194 / 211.  In a captured graph the branches cost less:
 // 256^2 / 64K 38.8 / 36.1, 512^2 / 1M 71.0 / 76.1, 1024^2 / 4M 205 / 219.
 static bool fork_pays(const nfft2d_plan *p, hipStream_t s)
 {
@@ -947,7 +950,7 @@ static bool fork_pays(const nfft2d_plan *p, hipStream_t s)
         cs = hipStreamCaptureStatusNone;
     }
     if (cs == hipStreamCaptureStatusActive) return modes >= 1 << 18;
-    return (p->czt[0] || p->czt[1]) && modes >= 200000;
+    return (p->czt[0] || p->czt[1]) && modes >= 1 << 19;
 }
 
 // setpts + type-2, in large cases (fork_pays) with the bin sort on the plan's
@@ -1456,8 +1459,8 @@ extern "C" int nfft1d_type2(nfft1d_plan *p, nfft2d_c64 *result, const nfft2d_c64
                                tw, batch);
         });
     } else if (p->czt) {
-        if ((rc = czt_launch<float, -1, true>(czt_tables_of<float>(p->czt, p->N, p->cztm, true), batch, f, p->N, 1, G,
-                                              p->L, 1, ones, D, s)))
+        if ((rc = czt_launch<float, 0>(czt_tables_of<float>(p->czt, p->N, p->cztm, true), batch, f, p->N, 1, G, p->L,
+                                       1, ones, D, true, false, s)))
             return rc;
     } else {
         hipLaunchKernelGGL((k_t2_rows_direct<float, -1>), dim3(batch), dim3(256), sizeof(float2) * 3 * p->N, s, f, G, ones, D,
@@ -1492,8 +1495,8 @@ extern "C" int nfft1d_type1(nfft1d_plan *p, nfft2d_c64 *result, const nfft2d_c64
                                tw, batch);
         });
     } else if (p->czt) {
-        if ((rc = czt_launch<float, -1, false>(czt_tables_of<float>(p->czt, p->N, p->cztm, false), batch, G, p->L, 1,
-                                               F, p->N, 1, ones, D, s)))
+        if ((rc = czt_launch<float, 0>(czt_tables_of<float>(p->czt, p->N, p->cztm, false), batch, G, p->L, 1, F, p->N,
+                                       1, ones, D, false, false, s)))
             return rc;
     } else {
         hipLaunchKernelGGL((k_t1_rows_direct<float, -1>), dim3(batch), dim3(256), sizeof(float2) * 2 * p->L, s, G, F, ones,
@@ -1518,6 +1521,7 @@ struct nfft2d_batch_s {
     int2 *own = nullptr;                  // owner tables of the 5 per-transform stages, back to back
     int off_hist = 0, n_hist = 0, off_col = 0, n_col = 0;   // the scatter takes the histogram's blocks
     int off_rows = 0, n_rows = 0, off_cols = 0, n_cols = 0, off_merge = 0, n_merge = 0;
+    int off_czt[4] = {}, n_czt[4] = {};   // chirp-z lines of the four passes (kb_czt)
     // type-1 passes: the transforms whose lines go to the matrix cores (t1_pass_on_mfma)
     // in their own stages, the others in stages of the type-2 passes' shape
     int off_t1c = 0, n_t1c = 0, off_t1cm = 0, n_t1cm = 0, off_t1r = 0, n_t1r = 0, off_t1rm = 0, n_t1rm = 0;
@@ -1649,16 +1653,24 @@ extern "C" int nfft2d_batch_create(nfft2d_batch **out, int count, const int *N1,
     // the Stockham passes take R rows / B columns per block, the direct ones one
     add_stage(b->off_rows, b->n_rows, [&](int t) {
         const BatchDesc &d = b->hdesc[t];
-        return batch_fft_n(d.N2) ? (int)grid1d(d.N1, batch_rows_per_block(d.N2)) : d.N1;
+        return batch_fft_n(d.N2) ? (int)grid1d(d.N1, batch_rows_per_block(d.N2)) : d.czt2 ? 0 : d.N1;
     });
     add_stage(b->off_cols, b->n_cols, [&](int t) {
         const BatchDesc &d = b->hdesc[t];
-        return batch_fft_n(d.N1) ? (int)grid1d(d.L2, batch_cols_per_block(d.N1)) : d.L2;
+        return batch_fft_n(d.N1) ? (int)grid1d(d.L2, batch_cols_per_block(d.N1)) : d.czt1 ? 0 : d.L2;
     });
+    for (int pass = 0; pass < 4; ++pass)
+        add_stage(b->off_czt[pass], b->n_czt[pass], [&](int t) {
+            const BatchDesc &d = b->hdesc[t];
+            const bool cols = pass == 1 || pass == 2;
+            if (!(cols ? d.czt1 : d.czt2)) return 0;
+            return (int)grid1d(cols ? d.L2 : d.N1, batch_czt_lines(cols ? d.cztm1 : d.cztm2));
+        });
     // type-1: 16-column tiles (column pass) and 16-row tiles (row pass) on the matrix cores
     add_stage(b->off_t1c, b->n_t1c, [&](int t) {
         const BatchDesc &d = b->hdesc[t];
-        return t1_pass_on_mfma(d.N1) ? 0 : batch_fft_n(d.N1) ? (int)grid1d(d.L2, batch_cols_per_block(d.N1)) : d.L2;
+        if (t1_pass_on_mfma(d.N1) || d.czt1) return 0;
+        return batch_fft_n(d.N1) ? (int)grid1d(d.L2, batch_cols_per_block(d.N1)) : d.L2;
     });
     add_stage(b->off_t1cm, b->n_t1cm, [&](int t) {
         const BatchDesc &d = b->hdesc[t];
@@ -1666,7 +1678,8 @@ extern "C" int nfft2d_batch_create(nfft2d_batch **out, int count, const int *N1,
     });
     add_stage(b->off_t1r, b->n_t1r, [&](int t) {
         const BatchDesc &d = b->hdesc[t];
-        return t1_pass_on_mfma(d.N2) ? 0 : batch_fft_n(d.N2) ? (int)grid1d(d.N1, batch_rows_per_block(d.N2)) : d.N1;
+        if (t1_pass_on_mfma(d.N2) || d.czt2) return 0;
+        return batch_fft_n(d.N2) ? (int)grid1d(d.N1, batch_rows_per_block(d.N2)) : d.N1;
     });
     add_stage(b->off_t1rm, b->n_t1rm, [&](int t) {
         const BatchDesc &d = b->hdesc[t];
@@ -1807,11 +1820,22 @@ extern "C" int nfft2d_batch_setpts(nfft2d_batch *b, void *stream)
     return NFFT2D_OK;
 }
 
+template <int PASS>
+static void batch_czt(nfft2d_batch *b, hipStream_t s)
+{
+    if (b->n_czt[PASS] > 0)
+        hipLaunchKernelGGL(kb_czt<PASS>, dim3(b->n_czt[PASS]), dim3(256), 0, s, b->ddesc, b->own + b->off_czt[PASS]);
+}
+
 static int batch_grid(nfft2d_batch *b, hipStream_t s)
 {
-    hipLaunchKernelGGL(kb_t2_rows, dim3(b->n_rows), dim3(128), 0, s, b->ddesc, b->own + b->off_rows);
+    if (b->n_rows > 0)
+        hipLaunchKernelGGL(kb_t2_rows, dim3(b->n_rows), dim3(128), 0, s, b->ddesc, b->own + b->off_rows);
+    batch_czt<0>(b, s);
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(kb_t2_cols, dim3(b->n_cols), dim3(256), 0, s, b->ddesc, b->own + b->off_cols);
+    if (b->n_cols > 0)
+        hipLaunchKernelGGL(kb_t2_cols, dim3(b->n_cols), dim3(256), 0, s, b->ddesc, b->own + b->off_cols);
+    batch_czt<1>(b, s);
     NFFT2D_LAUNCH_CHECK();
     return NFFT2D_OK;
 }
@@ -1896,11 +1920,15 @@ extern "C" int nfft2d_batch_type1(nfft2d_batch *b, void *stream)
     if (b->n_t1c > 0)
         hipLaunchKernelGGL(kb_t1_cols, dim3(b->n_t1c), dim3(256), 0, s, b->ddesc, b->own + b->off_t1c);
     NFFT2D_LAUNCH_CHECK();
+    batch_czt<2>(b, s);
+    NFFT2D_LAUNCH_CHECK();
     if (b->n_t1cm > 0)
         hipLaunchKernelGGL(kb_t1_cols_mm, dim3(b->n_t1cm), dim3(256), 0, s, b->ddesc, b->own + b->off_t1cm);
     NFFT2D_LAUNCH_CHECK();
     if (b->n_t1r > 0)
         hipLaunchKernelGGL(kb_t1_rows, dim3(b->n_t1r), dim3(128), 0, s, b->ddesc, b->own + b->off_t1r);
+    NFFT2D_LAUNCH_CHECK();
+    batch_czt<3>(b, s);
     NFFT2D_LAUNCH_CHECK();
     if (b->n_t1rm > 0)
         hipLaunchKernelGGL(kb_t1_rows_mm, dim3(b->n_t1rm), dim3(256), 0, s, b->ddesc, b->own + b->off_t1rm);

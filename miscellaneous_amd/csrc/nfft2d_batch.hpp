@@ -226,18 +226,51 @@ __global__ __launch_bounds__(kScatThreads) void kb_scatter_lds(const BatchDesc* 
 
 // ---------------------------------------------------------------- grid passes
 // Row passes: 128 threads, block o.y of the transform's rows (R rows of N2 for
-// the Stockham passes, one row for the chirp-z and direct ones); column
-// passes: 256 threads, likewise over the L2 columns.  The LDS buffer fits the
-// largest N of every form: the direct passes stage one line of up to
-// 2 kBatchMaxN, the chirp-z passes (the plans' for lengths up to
-// kBatchCztMaxN; longer ones take the direct passes here) one FFT of up to
-// 2048 points with its twiddles.
+// the Stockham passes, one row for the direct ones); column passes: 256
+// threads, likewise over the L2 columns.  The LDS buffer fits the largest N of
+// both forms: the direct passes stage one line of up to 2 kBatchMaxN.  The
+// chirp-z lines (up to kBatchCztMaxM points; longer ones take the direct
+// passes) have launches of their own, kb_czt: inside these kernels their
+// registers (120 against 60) would halve the Stockham passes' occupancy (a
+// batch of 256 power-of-two transforms: column pass 303 -> 530 us).
 constexpr int kBatchCztMaxM = 2048;
-constexpr int kBatchCztU = 4;   // values per thread: 4 U >= kBatchCztMaxM / 128
-constexpr int kBatchLineLds = 2 * kBatchMaxN > czt_lds_entries(kBatchCztMaxM) ? 2 * kBatchMaxN
-                                                                             : czt_lds_entries(kBatchCztMaxM);
+constexpr int kBatchLineLds = 2 * kBatchMaxN;
 constexpr int batch_lds_rows() { return batch_rows_lds() > kBatchLineLds ? batch_rows_lds() : kBatchLineLds; }
 constexpr int batch_lds_cols() { return batch_cols_lds() > kBatchLineLds ? batch_cols_lds() : kBatchLineLds; }
+
+// Chirp-z lines of a pass (0 type-2 rows, 1 type-2 columns, 2 type-1 columns,
+// 3 type-1 rows): block o.y takes 2048 / m lines of its transform, 256 roles.
+__host__ __device__ constexpr int batch_czt_lines(int m) { return kBatchCztMaxM / m; }
+template <int PASS>
+__global__ __launch_bounds__(256) void kb_czt(const BatchDesc* __restrict__ bd, const int2* __restrict__ own)
+{
+    __shared__ float2 lds[4 * lds_line<512>()];   // = 2 lines of 1024, 1 of 2048
+    const int2 o = own[blockIdx.x];
+    const BatchDesc& d = bd[o.x];
+    const float* none = nullptr;
+    constexpr bool cols = PASS == 1 || PASS == 2, type2 = PASS < 2;
+    const int m = cols ? d.cztm1 : d.cztm2;
+    const CztTables<float> tb = czt_tables_of<float>(cols ? d.czt1 : d.czt2, cols ? d.N1 : d.N2, m, type2);
+    auto run = [&](auto lg) {
+        constexpr int LG = decltype(lg)::value, B = batch_czt_lines(1 << LG);
+        const int b0 = o.y * B, N2 = d.N2;
+        if constexpr (PASS == 0)        // f[k1][*] (N2) -> Tm[k1][*] (L2), pre-compensated
+            czt_lines<float, LG, B, 1, false, false>(b0, d.N1, lds, d.f, N2, 1, d.Tm, 2 * N2, 1, d.D1, d.D2, true, false,
+                                                     tb);
+        else if constexpr (PASS == 1)   // Tm[*][n2] (N1) -> Gt[n2][*] (L1)
+            czt_lines<float, LG, B, 1, true, false>(b0, d.L2, lds, d.Tm, 1, d.L2, d.Gt, d.L1, 1, none, none, true, false,
+                                                    tb);
+        else if constexpr (PASS == 2)   // Gt[n2][*] (L1) -> Tm[*][n2] (N1)
+            czt_lines<float, LG, B, 1, false, true>(b0, d.L2, lds, d.Gt, d.L1, 1, d.Tm, 1, d.L2, none, none, false,
+                                                    false, tb);
+        else                            // Tm[k1][*] (L2) -> F1[k1][*] (N2), deconvolved
+            czt_lines<float, LG, B, 1, false, false>(b0, d.N1, lds, d.Tm, 2 * N2, 1, d.F1, N2, 1, d.D1, d.D2, false,
+                                                     false, tb);
+    };
+    if (m == 512) run(std::integral_constant<int, 9>{});
+    else if (m == 1024) run(std::integral_constant<int, 10>{});
+    else run(std::integral_constant<int, 11>{});
+}
 
 __global__ __launch_bounds__(128) void kb_t2_rows(const BatchDesc* __restrict__ bd, const int2* __restrict__ own)
 {
@@ -245,12 +278,8 @@ __global__ __launch_bounds__(128) void kb_t2_rows(const BatchDesc* __restrict__ 
     const int2 o = own[blockIdx.x];
     const BatchDesc& d = bd[o.x];
     if (!batch_fft_n(d.N2)) {
-        if (d.czt2)   // row o.y: f[k1][*] (N2) -> Tm[k1][*] (L2), pre-compensated
-            czt_line<float, -1, true, kBatchCztU>(o.y, lds, d.f, d.N2, 1, d.Tm, 2 * d.N2, 1, d.D1, d.D2,
-                                                  czt_tables_of<float>(d.czt2, d.N2, d.cztm2, true));
-        else
-            t2_rows_direct_body<float, -1>(o.y, lds, d.f, d.Tm, d.D1, d.D2, d.tw2, d.N1, d.N2,
-                                           3 * d.N2 <= batch_lds_rows() ? lds + d.N2 : nullptr);
+        t2_rows_direct_body<float, -1>(o.y, lds, d.f, d.Tm, d.D1, d.D2, d.tw2, d.N1, d.N2,
+                                       3 * d.N2 <= batch_lds_rows() ? lds + d.N2 : nullptr);
         return;
     }
     batch_dispatch_n(d.N2, [&](auto n) {
@@ -265,12 +294,7 @@ __global__ __launch_bounds__(256) void kb_t2_cols(const BatchDesc* __restrict__ 
     const int2 o = own[blockIdx.x];
     const BatchDesc& d = bd[o.x];
     if (!batch_fft_n(d.N1)) {
-        if (d.czt1)   // column o.y: Tm[*][n2] (N1) -> Gt[n2][*] (L1)
-            czt_line<float, -1, true, kBatchCztU>(o.y, lds, d.Tm, 1, d.L2, d.Gt, d.L1, 1, (const float*)nullptr,
-                                                  (const float*)nullptr,
-                                                  czt_tables_of<float>(d.czt1, d.N1, d.cztm1, true));
-        else
-            t2_cols_direct_body<float, -1>(o.y, lds, d.Tm, d.Gt, d.tw1, d.N1, d.L2,
+        t2_cols_direct_body<float, -1>(o.y, lds, d.Tm, d.Gt, d.tw1, d.N1, d.L2,
                                            3 * d.N1 <= batch_lds_cols() ? lds + d.N1 : nullptr);
         return;
     }
@@ -315,12 +339,7 @@ __global__ __launch_bounds__(256) void kb_t1_cols(const BatchDesc* __restrict__ 
     const int2 o = own[blockIdx.x];
     const BatchDesc& d = bd[o.x];
     if (!batch_fft_n(d.N1)) {
-        if (d.czt1)   // column o.y: Gt[n2][*] (L1) -> Tm[*][n2] (N1)
-            czt_line<float, -1, false, kBatchCztU>(o.y, lds, d.Gt, d.L1, 1, d.Tm, 1, d.L2, (const float*)nullptr,
-                                                   (const float*)nullptr,
-                                                   czt_tables_of<float>(d.czt1, d.N1, d.cztm1, false));
-        else
-            t1_cols_direct_body<float, -1>(o.y, lds, d.Gt, d.Tm, d.tw1, d.N1, d.L2,
+        t1_cols_direct_body<float, -1>(o.y, lds, d.Gt, d.Tm, d.tw1, d.N1, d.L2,
                                            4 * d.N1 <= batch_lds_cols() ? lds + 2 * d.N1 : nullptr);
         return;
     }
@@ -336,11 +355,7 @@ __global__ __launch_bounds__(128) void kb_t1_rows(const BatchDesc* __restrict__ 
     const int2 o = own[blockIdx.x];
     const BatchDesc& d = bd[o.x];
     if (!batch_fft_n(d.N2)) {
-        if (d.czt2)   // row o.y: Tm[k1][*] (L2) -> F1[k1][*] (N2), deconvolved
-            czt_line<float, -1, false, kBatchCztU>(o.y, lds, d.Tm, 2 * d.N2, 1, d.F1, d.N2, 1, d.D1, d.D2,
-                                                   czt_tables_of<float>(d.czt2, d.N2, d.cztm2, false));
-        else
-            t1_rows_direct_body<float, -1>(o.y, lds, d.Tm, d.F1, d.D1, d.D2, d.tw2, d.N1, d.N2,
+        t1_rows_direct_body<float, -1>(o.y, lds, d.Tm, d.F1, d.D1, d.D2, d.tw2, d.N1, d.N2,
                                            4 * d.N2 <= batch_lds_rows() ? lds + 2 * d.N2 : nullptr);
         return;
     }

@@ -8,15 +8,24 @@
 // ab = (a^2 + b^2 - (b - a)^2) / 2 and c[k] = w^{k^2/2} = e^{-i pi k^2 / L} is
 //     Y[q] = c[q + q0] sum_p (x[p] c[p + p0]) conj(c[(q - p) + q0 - p0]),
 // a linear convolution, taken circularly at the power of two m >= P + Q - 1
-// through two LDS-resident FFTs of m points.  The inverse direction (e^{+})
-// conjugates the input and the output.  The chirps (P and Q entries), the
-// transform of the convolution kernel (m entries) and the FFT's twiddles
-// (e^{-2 pi i t / m} = T1[t / 64] T2[t % 64]) are computed on the host in FP64
-// at plan creation.  One block per line; O(m log m) per line instead of the
-// O(N L) of the direct passes.
+// through two FFTs of m points.  The inverse direction (e^{+}) conjugates the
+// input and the output.  The chirps (P and Q entries), the transform of the
+// convolution kernel and the FFT's twiddles e^{-2 pi i t / m} (m entries each)
+// are computed on the host in FP64 at plan creation.  O(m log m) per line
+// instead of the O(N L) of the direct passes.
+//
+// What bounds these passes is the LDS: a radix-4 form that kept the line there
+// moved it through LDS 26 times at m = 2048 (with two twiddle reads per
+// product besides) and ran at a twentieth of the copy rate.  So a line lives
+// in registers, 8 values j + q m/8 (q < 8) per role j < m/8, the order in
+// which every radix-8 stage of the Stockham form reads and the last one
+// leaves them: the kernel product and the start of the second FFT need no
+// exchange, and each FFT makes stages - 1 (three) trips through LDS.  Measured
+// on FP64 lines of 500 and 250 (500 x 250 modes, both passes of a type-2 /
+// type-1): 36 / 35 -> 25 / 24 us.
 #pragma once
 
-#include "nfft2d_device.hpp"
+#include "nfft2d_kernels.hpp"
 
 namespace nfft2d {
 
@@ -25,12 +34,11 @@ struct CztTables {
     const cplx<T> *cin = nullptr;    // c[p + p0], P
     const cplx<T> *cout = nullptr;   // c[q + q0], Q
     const cplx<T> *hhat = nullptr;   // FFT_m of the kernel conj(c[d + q0 - p0]), d = q - p
-    const cplx<T> *t1 = nullptr;     // e^{-2 pi i 64 j / m}, max(1, m / 64)
-    const cplx<T> *t2 = nullptr;     // e^{-2 pi i j / m}, 64
+    const cplx<T> *tw = nullptr;     // e^{-2 pi i j / m}, m
     int P = 0, Q = 0, m = 0;
 };
 
-__host__ __device__ constexpr int czt_lds_entries(int m) { return m + (m >= 64 ? m / 64 : 1) + 64; }
+constexpr int kCztMinLog = 9, kCztMaxLog = 14;   // m = 512 (N >= 128) .. 16,384 (N <= 4096)
 
 // Smallest power of two m >= 3N - 1 (P + Q - 1 = N + 2N - 1): the chirp-z FFT length of a line of N.
 __host__ __device__ constexpr int czt_m(int N)
@@ -41,8 +49,8 @@ __host__ __device__ constexpr int czt_m(int N)
 }
 
 // The chirp-z tables of a line length N inside one table buffer (layout
-// [cin2 N][cout2 L][hhat2 m][cin1 L][cout1 N][hhat1 m][T1 m/64][T2 64],
-// L = 2N), for its type-2 (t2 = true) or type-1 pass.
+// [cin2 N][cout2 L][hhat2 m][cin1 L][cout1 N][hhat1 m][tw m], L = 2N), for
+// its type-2 (t2 = true) or type-1 pass.
 template <typename T>
 __host__ __device__ inline CztTables<T> czt_tables_of(const void* buf, int N, int m, bool t2)
 {
@@ -51,9 +59,7 @@ __host__ __device__ inline CztTables<T> czt_tables_of(const void* buf, int N, in
     const C* b = (const C*)buf;
     CztTables<T> t;
     t.m = m;
-    const C* tw = b + 3 * L + 2 * m;   // after both passes' chirps and kernels
-    t.t1 = tw;
-    t.t2 = tw + (m >= 64 ? m / 64 : 1);
+    t.tw = b + 3 * L + 2 * m;          // after both passes' chirps and kernels
     if (t2) {
         t.P = N;
         t.Q = L;
@@ -71,137 +77,203 @@ __host__ __device__ inline CztTables<T> czt_tables_of(const void* buf, int N, in
     return t;
 }
 
-// In-place radix-4 (+ one radix-2) Stockham FFT of m = 2^a points in LDS
-// (Govindaraju et al., SC 2008): stage with span Ns reads v_r = X[j + r m/R],
-// twiddles it by e^{-2 pi i r (j mod Ns) / (Ns R)}, and writes the R-point DFT
-// to X[(j - j mod Ns) R + j mod Ns + r Ns]; all reads of a stage precede its
-// writes (barrier).  Each thread holds at most 4 U values (blockDim >= m / (4 U)):
-// U = 2 up to m = 8192 at 1024 threads, U = 4 for m = 16384.
-template <typename T, int U>
-__device__ void czt_fft(cplx<T> *X, int m, const cplx<T> *t1, const cplx<T> *t2)
+// a b with the order of the roundings written out: left to contract a.x b.x -
+// a.y b.y, the compiler fuses either product, one way in a plan's pass and the
+// other in a batch's.
+template <typename C> __device__ __forceinline__ C cmul_f(C a, C b)
+{
+    return mk(fma(-a.y, b.y, a.x * b.x), fma(a.y, b.x, a.x * b.y));
+}
+
+// FFT of 2^LOGM points (e^{-2 pi i jk / m}), the Stockham stages of
+// nfft2d_device.hpp with the line in registers between the LDS exchanges.
+// A role is one of the m/8 workers of a line: role (l, j) holds x[j + q m/8]
+// in v[q] on entry and X[j + q m/8] on return.  A thread plays K roles
+// (act: the role exists); a role may name another (line, j) for the input
+// (la, ja), the middle stages (lm, jm) and the output (lo, jo), the exchanges
+// make the remap free.  lds: line l at l * lds_line<m>().  Every barrier is
+// reached by all threads; the LDS must be free on entry, and is being read
+// when the function returns.
+template <typename T, int LOGM, int K>
+__device__ __forceinline__ void czt_fft(cplx<T> (&v)[K][8], cplx<T>* lds, const cplx<T>* __restrict__ tw,
+                                        const bool (&act)[K], const int (&la)[K], const int (&ja)[K],
+                                        const int (&lm)[K], const int (&jm)[K], const int (&lo)[K],
+                                        const int (&jo)[K])
 {
     using C = cplx<T>;
-    const int NT = blockDim.x, tid = threadIdx.x;
-    auto tw = [&](int t) { return cmul(t1[t >> 6], t2[t & 63]); };
-    for (int Ns = 1; Ns < m;) {
-        const int R = (m / Ns) >= 4 ? 4 : 2;
-        const int nb = m / R, per = (nb + NT - 1) / NT;
-        const int tstep = m / (Ns * R);
-        C v[4 * U];
-        if (R == 4) {
+    constexpr int M = 1 << LOGM, TPL = M / 8, LL = lds_line<M>(), R0 = FftPlan<M>::r0, B0 = 8 / R0;
+    constexpr int S = FftPlan<M>::stages;
+    static_assert(S >= 3, "m >= 512");
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = tid + u * NT;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1);
-                    C a0 = X[j], a1 = X[j + nb], a2 = X[j + 2 * nb], a3 = X[j + 3 * nb];
-                    if (Ns > 1) {
-                        a1 = cmul(a1, tw(k * tstep));
-                        a2 = cmul(a2, tw(2 * k * tstep));
-                        a3 = cmul(a3, tw(3 * k * tstep));
-                    }
-                    const C b0 = cadd(a0, a2), b1 = csub(a0, a2), b2 = cadd(a1, a3);
-                    const C d = csub(a1, a3);
-                    const C b3 = mk(d.y, -d.x);   // (a1 - a3) (-i)
-                    v[4 * u + 0] = cadd(b0, b2);
-                    v[4 * u + 1] = cadd(b1, b3);
-                    v[4 * u + 2] = csub(b0, b2);
-                    v[4 * u + 3] = csub(b1, b3);
-                }
-            }
-            __syncthreads();
+    for (int u = 0; u < K; ++u) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int j = tid + u * NT;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1), o = (j - k) * 4 + k;
-                    X[o] = v[4 * u];
-                    X[o + Ns] = v[4 * u + 1];
-                    X[o + 2 * Ns] = v[4 * u + 2];
-                    X[o + 3 * Ns] = v[4 * u + 3];
-                }
-            }
-        } else {
+        for (int b = 0; b < B0; ++b) {
+            C a[R0];
 #pragma unroll
-            for (int u = 0; u < 2 * U; ++u) {
-                const int j = tid + u * NT;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1);
-                    C a0 = X[j], a1 = X[j + nb];
-                    if (Ns > 1) a1 = cmul(a1, tw(k * tstep));
-                    v[2 * u] = cadd(a0, a1);
-                    v[2 * u + 1] = csub(a0, a1);
-                }
-            }
-            __syncthreads();
+            for (int r = 0; r < R0; ++r) a[r] = v[u][b + r * B0];
+            dftR<R0, -1>(a);
+            if (act[u]) {
 #pragma unroll
-            for (int u = 0; u < 2 * U; ++u) {
-                const int j = tid + u * NT;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1), o = (j - k) * 2 + k;
-                    X[o] = v[2 * u];
-                    X[o + Ns] = v[2 * u + 1];
-                }
+                for (int r = 0; r < R0; ++r) lds[la[u] * LL + lpad((ja[u] + b * TPL) * R0 + r)] = a[r];
             }
+        }
+    }
+#pragma unroll
+    for (int s = 1; s < S; ++s) {
+        const int NS = FftPlan<M>::ns(s);
+        const bool last = s == S - 1;
+        // the stage's twiddles, in flight across the barrier and the LDS reads
+        C w[K][7];
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int e = ((last ? jo[u] : jm[u]) & (NS - 1)) * (TPL / NS);
+#pragma unroll
+            for (int r = 1; r < 8; ++r) w[u][r - 1] = tw[r * e];
         }
         __syncthreads();
-        Ns *= R;
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int l = last ? lo[u] : lm[u], j = last ? jo[u] : jm[u];
+            if (act[u]) {
+#pragma unroll
+                for (int q = 0; q < 8; ++q) v[u][q] = lds[l * LL + lpad(j + q * TPL)];
+            }
+        }
+        if (!last) __syncthreads();
+#pragma unroll
+        for (int u = 0; u < K; ++u) {
+            const int j = last ? jo[u] : jm[u], k = j & (NS - 1);
+#pragma unroll
+            for (int r = 1; r < 8; ++r) v[u][r] = cmul_f(v[u][r], w[u][r - 1]);
+            dft8<-1>(v[u]);
+            if (!last && act[u]) {
+                const int o = (j - k) * 8 + k;
+#pragma unroll
+                for (int r = 0; r < 8; ++r) lds[lm[u] * LL + lpad(o + r * NS)] = v[u][r];
+            }
+        }
     }
 }
 
-// Line b of a chirp-z pass, by the whole block (smem: czt_lds_entries(m)
-// entries; blockDim.x >= m / (4 U)).  The line reads x[p] = in[b * in_ls +
-// p * in_es] and writes out[b * out_ls + q * out_es].  Type-2 rows scale the
-// input by sl[b] se[p] (the pre-compensation D1[k1] D2[k2]); type-1 rows
-// scale the output by sl[b] se[q] (the deconvolution); null: no scaling.
-// Every butterfly and product is the same whatever the block size, so plans
-// and batches (other block sizes) get the same bits.
-template <typename T, int SIGN, bool SCALE_IN, int U>
-__device__ __forceinline__ void czt_line(int b, cplx<T>* smem, const cplx<T>* __restrict__ in, long long in_ls,
-                                         long long in_es, cplx<T>* __restrict__ out, long long out_ls,
-                                         long long out_es, const T* __restrict__ sl, const T* __restrict__ se,
-                                         const CztTables<T>& tb)
+// Lines line0 .. line0 + B - 1 (below `lines`) of a chirp-z pass by the whole
+// block: B m/8 roles, K per thread (blockDim.x * K >= B m/8).  Line b reads
+// x[p] = in[b in_ls + p in_es] and writes out[b out_ls + q out_es]; COL_IN /
+// COL_OUT: the lines lie side by side there (ls = 1), neighbouring threads
+// take neighbouring lines.  scale_in (type-2 rows): the input is scaled by
+// sl[b] se[p] (the pre-compensation D1[k1] D2[k2]); else the output by sl[b]
+// se[q] (the deconvolution); sl null: no scaling.  conj: the inverse
+// direction.  Every butterfly and product is the same whatever B and K, so
+// plans and batches (other block sizes) get the same bits.
+template <typename T, int LOGM, int B, int K, bool COL_IN, bool COL_OUT>
+__device__ __forceinline__ void czt_lines(int line0, int lines, cplx<T>* lds, const cplx<T>* __restrict__ in,
+                                          long long in_ls, long long in_es, cplx<T>* __restrict__ out,
+                                          long long out_ls, long long out_es, const T* __restrict__ sl,
+                                          const T* __restrict__ se, bool scale_in, bool conj, const CztTables<T>& tb)
 {
     using C = cplx<T>;
-    C *X = smem;
-    C *t1 = X + tb.m, *t2 = t1 + (tb.m >= 64 ? tb.m / 64 : 1);
-    const int NT = blockDim.x, m = tb.m;
-    for (int k = threadIdx.x; k < 64; k += NT) t2[k] = tb.t2[k];
-    for (int k = threadIdx.x; k < (m >= 64 ? m / 64 : 1); k += NT) t1[k] = tb.t1[k];
-    const T lsc = sl ? sl[b] : (T)1;
-    for (int p = threadIdx.x; p < m; p += NT) {
-        C v = mk((T)0, (T)0);
-        if (p < tb.P) {
-            v = in[b * in_ls + p * in_es];
-            if (SCALE_IN && sl) v = cscale(v, lsc * se[p]);
-            if (SIGN > 0) v = cconj(v);
-            v = cmul(v, tb.cin[p]);
-        }
-        X[p] = v;
+    constexpr int M = 1 << LOGM, TPL = M / 8;
+    bool act[K];
+    int la[K], ja[K], lm[K], jm[K], lo[K], jo[K];
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+        const int role = (int)threadIdx.x + u * (int)blockDim.x;
+        act[u] = role < B * TPL;
+        lm[u] = role / TPL;
+        jm[u] = role % TPL;
+        la[u] = COL_IN ? role % B : lm[u];
+        ja[u] = COL_IN ? role / B : jm[u];
+        lo[u] = COL_OUT ? role % B : lm[u];
+        jo[u] = COL_OUT ? role / B : jm[u];
     }
+    // every load at a clamped index, so that none waits in a branch
+    C v[K][8], h[K][8];
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+        const int b = min(line0 + la[u], lines - 1);
+        C c[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int p = min(ja[u] + q * TPL, tb.P - 1);
+            v[u][q] = in[b * in_ls + p * in_es];
+            c[q] = tb.cin[p];
+        }
+        if (scale_in && sl) {
+            const T lsc = sl[b];
+            T e[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) e[q] = se[min(ja[u] + q * TPL, tb.P - 1)];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) v[u][q] = cscale(v[u][q], lsc * e[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            C x = v[u][q];
+            if (conj) x = cconj(x);
+            x = cmul_f(x, c[q]);
+            v[u][q] = ja[u] + q * TPL < tb.P ? x : mk((T)0, (T)0);
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) h[u][q] = tb.hhat[(jm[u] + q * TPL) & (M - 1)];
+    }
+    czt_fft<T, LOGM, K>(v, lds, tb.tw, act, la, ja, lm, jm, lm, jm);
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[u][q] = cconj(cmul_f(v[u][q], h[u][q]));
     __syncthreads();
-    czt_fft<T, U>(X, m, t1, t2);
-    for (int k = threadIdx.x; k < m; k += NT) X[k] = cconj(cmul(X[k], tb.hhat[k]));
-    __syncthreads();
-    czt_fft<T, U>(X, m, t1, t2);
-    const T inv = (T)1 / (T)m;
-    for (int q = threadIdx.x; q < tb.Q; q += NT) {
-        C v = cmul(cscale(cconj(X[q]), inv), tb.cout[q]);
-        if (SIGN > 0) v = cconj(v);
-        if (!SCALE_IN && sl) v = cscale(v, lsc * se[q]);
-        out[b * out_ls + q * out_es] = v;
+#pragma unroll
+    for (int u = 0; u < K; ++u)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) h[u][q] = tb.cout[min(jo[u] + q * TPL, tb.Q - 1)];
+    czt_fft<T, LOGM, K>(v, lds, tb.tw, act, lm, jm, lm, jm, lo, jo);
+    const T inv = (T)1 / (T)M;
+#pragma unroll
+    for (int u = 0; u < K; ++u) {
+        const int b = line0 + lo[u];
+        if (!act[u] || b >= lines) continue;
+        const T lsc = !scale_in && sl ? sl[b] : (T)1;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int o = jo[u] + q * TPL;
+            if (o < tb.Q) {
+                C x = cmul_f(cscale(cconj(v[u][q]), inv), h[u][q]);
+                if (conj) x = cconj(x);
+                if (!scale_in && sl) x = cscale(x, lsc * se[o]);
+                out[b * out_ls + o * out_es] = x;
+            }
+        }
     }
 }
 
-// One line per block.
-template <typename T, int SIGN, bool SCALE_IN, int U>
-__global__ __launch_bounds__(1024) void k_czt(const cplx<T> *__restrict__ in, long long in_ls, long long in_es,
-                                              cplx<T> *__restrict__ out, long long out_ls, long long out_es,
-                                              const T *__restrict__ sl, const T *__restrict__ se, CztTables<T> tb)
+// A plan's pass: one line per block where the lines are contiguous on both
+// sides, else 4,096 values (512 roles) of neighbouring lines; one role per
+// thread up to m = 8192, two at 16,384.  Neighbouring blocks go to
+// one XCD (grid: a multiple of 8), so that the lines that share cache lines in
+// the strided direction meet in one L2.
+template <int LOGM, bool COL> constexpr int czt_block_lines() { return !COL || LOGM >= 12 ? 1 : 4096 >> LOGM; }
+template <int LOGM> constexpr int czt_roles_per_thread() { return LOGM > 13 ? 2 : 1; }
+template <int LOGM, bool COL> constexpr int czt_threads()
+{
+    return czt_block_lines<LOGM, COL>() * ((1 << LOGM) / 8) / czt_roles_per_thread<LOGM>();
+}
+template <typename T, int LOGM, bool COL> constexpr int czt_lds_bytes()
+{
+    return (int)sizeof(cplx<T>) * czt_block_lines<LOGM, COL>() * lds_line<1 << LOGM>();
+}
+template <typename T, int LOGM, bool COL_IN, bool COL_OUT>
+__global__ __launch_bounds__((czt_threads<LOGM, COL_IN || COL_OUT>())) void k_czt(const cplx<T> *__restrict__ in, long long in_ls,
+                                                            long long in_es, cplx<T> *__restrict__ out,
+                                                            long long out_ls, long long out_es,
+                                                            const T *__restrict__ sl, const T *__restrict__ se,
+                                                            bool scale_in, bool conj, int lines, CztTables<T> tb)
 {
     extern __shared__ unsigned char smem_raw[];
-    czt_line<T, SIGN, SCALE_IN, U>((int)blockIdx.x, reinterpret_cast<cplx<T> *>(smem_raw), in, in_ls, in_es, out,
-                                   out_ls, out_es, sl, se, tb);
+    constexpr int B = czt_block_lines<LOGM, COL_IN || COL_OUT>();
+    const int line0 = xcd_block((int)blockIdx.x, (int)gridDim.x) * B;
+    if (line0 >= lines) return;
+    czt_lines<T, LOGM, B, czt_roles_per_thread<LOGM>(), COL_IN, COL_OUT>(
+        line0, lines, reinterpret_cast<cplx<T> *>(smem_raw), in, in_ls, in_es, out, out_ls, out_es, sl, se, scale_in,
+        conj, tb);
 }
 
 }  // namespace nfft2d
