@@ -381,38 +381,6 @@ static CztTables<T> czt_tables(const nfft2d_plan *p, int dim, bool t2)
     return czt_tables_of<T>(p->czt[dim], dim == 0 ? p->N1 : p->N2, p->cztm[dim], t2);
 }
 
-// Launches one chirp-z pass over `lines` lines: MODE 0 both sides contiguous
-// along a line, 1 the input's lines side by side (in_ls = 1), 2 the output's.
-template <typename T, int LOGM, int MODE>
-static int czt_launch_m(const CztTables<T> &tb, int lines, const cplx<T> *in, long long in_ls, long long in_es,
-                        cplx<T> *out, long long out_ls, long long out_es, const T *sl, const T *se, bool scale_in,
-                        bool conj, hipStream_t s)
-{
-    static std::once_flag once;
-    static hipError_t attr = hipSuccess;
-    auto kern = k_czt<T, LOGM, MODE == 1, MODE == 2>;
-    constexpr int bytes = czt_lds_bytes<T, LOGM, MODE != 0>();
-    std::call_once(once, [&] {
-        attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    });
-    if (attr != hipSuccess) return nfft2d_fail(NFFT2D_ERR_HIP, "chirp-z pass: %s", hipGetErrorString(attr));
-    constexpr int B = czt_block_lines<LOGM, MODE != 0>();
-    const unsigned blocks = ((unsigned)(lines + B - 1) / B + 7) & ~7u;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(czt_threads<LOGM, MODE != 0>()), bytes, s, in, in_ls, in_es, out, out_ls, out_es,
-                       sl, se, scale_in, conj, lines, tb);
-    NFFT2D_LAUNCH_CHECK();
-    return NFFT2D_OK;
-}
-template <typename T, int MODE, int LOGM = kCztMinLog, typename... A>
-static int czt_launch(const CztTables<T> &tb, A... a)
-{
-    if (tb.m == 1 << LOGM) return czt_launch_m<T, LOGM, MODE>(tb, a...);
-    if constexpr (LOGM < kCztMaxLog && (1 << LOGM) < czt_m(kCztMaxN<T>))
-        return czt_launch<T, MODE, LOGM + 1>(tb, a...);
-    else
-        return nfft2d_fail(NFFT2D_ERR_SIZE, "chirp-z pass: no transform of %d points", tb.m);
-}
-
 template <typename T>
 static int upload_tables(nfft2d_plan *p)
 {

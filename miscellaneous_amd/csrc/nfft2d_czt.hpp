@@ -25,7 +25,11 @@
 // type-1): 36 / 35 -> 25 / 24 us.
 #pragma once
 
-#include "nfft2d_kernels.hpp"
+#include <mutex>
+
+#include "../../include/nfft2d.h"
+#include "nfft2d_device.hpp"
+#include "nfft2d_internal.hpp"
 
 namespace nfft2d {
 
@@ -38,7 +42,8 @@ struct CztTables {
     int P = 0, Q = 0, m = 0;
 };
 
-constexpr int kCztMinLog = 9, kCztMaxLog = 14;   // m = 512 (N >= 128) .. 16,384 (N <= 4096)
+constexpr int kCztMinLog = 9;   // m = 512 (N >= 128) .. 16,384 (N <= 4096), FP64 8,192 (N <= 2048)
+template <typename T> constexpr int kCztMaxLog = sizeof(T) == 4 ? 14 : 13;
 
 // Smallest power of two m >= 3N - 1 (P + Q - 1 = N + 2N - 1): the chirp-z FFT length of a line of N.
 __host__ __device__ constexpr int czt_m(int N)
@@ -274,6 +279,38 @@ __global__ __launch_bounds__((czt_threads<LOGM, COL_IN || COL_OUT>())) void k_cz
     czt_lines<T, LOGM, B, czt_roles_per_thread<LOGM>(), COL_IN, COL_OUT>(
         line0, lines, reinterpret_cast<cplx<T> *>(smem_raw), in, in_ls, in_es, out, out_ls, out_es, sl, se, scale_in,
         conj, tb);
+}
+
+// Launches one chirp-z pass over `lines` lines: MODE 0 both sides contiguous
+// along a line, 1 the input's lines side by side (in_ls = 1), 2 the output's.
+template <typename T, int LOGM, int MODE>
+int czt_launch_m(const CztTables<T> &tb, int lines, const cplx<T> *in, long long in_ls, long long in_es,
+                        cplx<T> *out, long long out_ls, long long out_es, const T *sl, const T *se, bool scale_in,
+                        bool conj, hipStream_t s)
+{
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    auto kern = k_czt<T, LOGM, MODE == 1, MODE == 2>;
+    constexpr int bytes = czt_lds_bytes<T, LOGM, MODE != 0>();
+    std::call_once(once, [&] {
+        attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    });
+    if (attr != hipSuccess) return nfft2d_fail(NFFT2D_ERR_HIP, "chirp-z pass: %s", hipGetErrorString(attr));
+    constexpr int B = czt_block_lines<LOGM, MODE != 0>();
+    const unsigned blocks = ((unsigned)(lines + B - 1) / B + 7) & ~7u;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(czt_threads<LOGM, MODE != 0>()), bytes, s, in, in_ls, in_es, out, out_ls, out_es,
+                       sl, se, scale_in, conj, lines, tb);
+    NFFT2D_LAUNCH_CHECK();
+    return NFFT2D_OK;
+}
+template <typename T, int MODE, int LOGM = kCztMinLog, typename... A>
+int czt_launch(const CztTables<T> &tb, A... a)
+{
+    if (tb.m == 1 << LOGM) return czt_launch_m<T, LOGM, MODE>(tb, a...);
+    if constexpr (LOGM < kCztMaxLog<T>)
+        return czt_launch<T, MODE, LOGM + 1>(tb, a...);
+    else
+        return nfft2d_fail(NFFT2D_ERR_SIZE, "chirp-z pass: no transform of %d points", tb.m);
 }
 
 }  // namespace nfft2d

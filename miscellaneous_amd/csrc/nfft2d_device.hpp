@@ -17,6 +17,26 @@ constexpr int kPolyDeg = 8;           // degree of the per-tap window polynomial
 constexpr int kNE = kPolyDeg / 2 + 1; // even-part coefficients (in t^2)
 constexpr int kNO = kPolyDeg / 2;     // odd-part coefficients (in t^2)
 
+// ---------------------------------------------------------------- block order
+// Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
+// b % 8), each with its own L2.  Give every XCD a contiguous range of logical
+// blocks so that neighbouring column blocks, which share cache lines, meet in
+// the same L2.  Identity when the grid is not a multiple of 8.
+__device__ __forceinline__ int xcd_block(int b, int n)
+{
+    if (n & 7) return b;
+    return (b & 7) * (n >> 3) + (b >> 3);
+}
+
+// For work of uneven cost in logical order (subproblems of a point set's
+// bins): every XCD takes runs of 8 consecutive logical blocks, the runs dealt
+// round-robin, so that neighbouring subproblems share an L2 while the XCDs
+// stay evenly loaded.  Grid: a multiple of 64.
+__device__ __forceinline__ int xcd_runs(int b)
+{
+    return (b & ~63) | ((b & 7) << 3) | ((b >> 3) & 7);
+}
+
 // ---------------------------------------------------------------- complex types
 template <typename T> struct cvec;
 template <> struct cvec<float> { using type = float2; };

@@ -48,25 +48,6 @@ __device__ __forceinline__ int wrap(int g, int L)
     return g < 0 ? g + L : g;
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
-// b % 8), each with its own L2.  Give every XCD a contiguous range of logical
-// blocks so that neighbouring column blocks, which share cache lines, meet in
-// the same L2.  Identity when the grid is not a multiple of 8.
-__device__ __forceinline__ int xcd_block(int b, int n)
-{
-    if (n & 7) return b;
-    return (b & 7) * (n >> 3) + (b >> 3);
-}
-
-// For work of uneven cost in logical order (subproblems of a point set's
-// bins): every XCD takes runs of 8 consecutive logical blocks, the runs dealt
-// round-robin, so that neighbouring subproblems share an L2 while the XCDs
-// stay evenly loaded.  Grid: a multiple of 64.
-__device__ __forceinline__ int xcd_runs(int b)
-{
-    return (b & ~63) | ((b & 7) << 3) | ((b >> 3) & 7);
-}
-
 // Row-group / column-block sizes of the FFT passes.
 template <int N> constexpr int rows_per_block() { return N >= 1024 ? 1 : 1024 / N; }
 template <int N> constexpr int cols_per_block() { return N >= 2048 ? 1 : 2048 / N; }

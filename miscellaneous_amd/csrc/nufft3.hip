@@ -8,34 +8,43 @@
 // One call:
 //   1. k3_extent / k3_extent_final: min and max of x, y, s, t (and whether all
 //      are finite).  The host reads them back -- the call's one
-//      synchronisation -- and derives every parameter exactly as :214-267.
-//   2. k3_prep_in / k3_prep_out: per input its pre-modulated sample and grid
-//      cell, per output its cell; both are counted into bins (inputs 8 x 8
-//      cells, outputs 16 x 16 cells and row) and sorted (k3_scan_*, k3_scatter*).
-//   3. k3_spread: one block per 16 x 16 tile of the grid sums
+//      synchronisation -- and derives every parameter exactly as :214-267, and
+//      from the extremes' own cells the part of the grid that the inputs reach
+//      and the part of the spectrum that the outputs read (about half and two
+//      fifths per side: the reference's grid holds R = 2.2 times the band, the
+//      inputs lie in its middle half).  Everything below works on those parts.
+//   2. k3_prep: per input its pre-modulated sample and grid cell, per output
+//      its cell and post-compensation factor; both are counted into bins
+//      (inputs 8 x 8 cells, outputs 16 x 16 cells and 8 x 2 blocks of them) and
+//      sorted (k3_scan_local, k3_scan_totals, k3_scatter).
+//   3. k3_spread: one block per 16 x 16 tile of the reached cells sums
 //      c_k ey_k(j) ex_k(i) over the inputs within reach of the tile, four
 //      inputs per v_mfma_f64_16x16x4f64 (the Gaussian of :76 is separable);
 //      the cell factor fact e^{b (Dx^2 dsi^2 + Dy^2 dsj^2)} multiplies the
 //      finished tile.  Each cell is written once: no atomics, no zero fill.
-//   4. The forward 2-D DFT of the grid (:280-292): a pass over the rows, a
-//      transpose, a pass over the rows of the transpose.  Each line is one
-//      LDS-resident radix-4 Stockham FFT; lengths that are not powers of two
-//      go through Bluestein's chirp-z convolution at the next power of two
-//      >= 2n - 1.
-//   5. k3_interp: one block per output bin stages the bin's grid patch in LDS
-//      with the circular and FFT shifts and the checkerboard sign of
-//      circAndFFTShiftsFunction (:135-151) folded into the index; one wave
-//      per output sums the (2 msp + 1)^2 separable Gaussian taps and applies
-//      the post-compensation of spectralConvolutionFunctionCompensation
-//      (:156-194).
+//   4. The forward 2-D DFT of the grid (:280-292) from the reached rows and
+//      cells to the read frequencies, as two chirp-z passes (nfft2d_czt.hpp):
+//      P inputs and Q outputs of a line are a convolution of P + Q - 1 points,
+//      a grid side of 1,638 takes 2,048 instead of the 4,096 of a full
+//      Bluestein transform, on half and two fifths of the lines.  The first
+//      pass writes its lines side by side: no transpose.  The circular and FFT
+//      shifts and the checkerboard sign of circAndFFTShiftsFunction (:135-151)
+//      are the passes' output offset and a sign in their output factors.
+//   5. k3_interp: one block per output bin stages the bin's patch of the
+//      spectrum in LDS; one wave per 16 outputs sums the (2 R + 1)^2
+//      separable Gaussian taps and applies the post-compensation of
+//      spectralConvolutionFunctionCompensation (:156-194).
+// 300,000 -> 300,000, X1 S = Y1 T = 500, eps 1e-6 (grid 1,638^2): 835 -> 299 us.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <chrono>
 #include <cmath>
 #include <map>
 #include <mutex>
 
 #include "../../include/nfft2d.h"
+#include "nfft2d_czt.hpp"
 #include "nfft2d_internal.hpp"
 
 namespace nufft3 {
@@ -43,29 +52,28 @@ namespace nufft3 {
 constexpr int kTile = 16;              // grid tile and output bin edge, cells
 constexpr int kInBin = 8;              // input bin edge, cells (finer: fewer out-of-reach candidates per tile)
 constexpr int kMaxMsp = 42;            // LDS patch (16 + 2 msp)^2 x 16 B <= 160 000 B
-constexpr int kMaxFft = 8192;          // longest LDS-resident FFT (128 KB)
+constexpr int kMaxFft = 8192;          // longest FFT of a chirp-z line (139 KB of LDS)
 constexpr int kExtentBlocks = 1024;
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 struct Par {
     double xb, yb, sb, tb, kkx, kky, Dx, Dy, b, t1, fact;
-    int msp, Mrx, Mry, nbx, nby;   // grid, and its 16 x 16-cell tiles (spread) / output bins (interpolation)
-    int ibx, iby;                   // 8 x 8-cell input bins
+    int reach, Mrx, Mry;      // taps per side in use (at most msp, see tap_reach)
+    int ci, cj, ni, nj;       // input cells [ci, ci + ni) x [cj, cj + nj); 8 x 8-cell bins from (ci, cj)
+    int oi, oj, mi, mj;       // output cells [oi, oi + mi) x [oj, oj + mj); 16 x 16-cell bins from (oi, oj)
+    int ibx, iby, nbx, nby;   // input bins, output bins
+    int gi, gj, Px, Py;       // reached cells [gi, gi + Px) x [gj, gj + Py)
+    int qi, qj, Qx, Qy;       // read frequencies qi + [0, Qx), qj + [0, Qy) (mod Mrx, Mry)
 };
 
 struct alignas(16) InRec {     // one input, in bin order
     double xt, yt, re, im;     // scaled offsets (x - xb) / Dx, (y - yb) / Dy; pre-modulated sample
-    int nno, mmo, pad0, pad1;  // its cell
 };
 struct alignas(16) OutRec {    // one output, in bin order
-    double difs, dift, sd, td; // fractional cell offsets; s - sb, t - tb (rescaled)
+    double difs, dift;         // fractional cell offsets
+    double pr, pi;             // post-compensation factor
     int nsn, ntn, idx, pad;
 };
-
-__device__ __forceinline__ double2 cmul(double2 a, double2 b)
-{
-    return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
-}
 
 // ------------------------------------------------------------ 1. extents
 // 9 values per block: max x, min x, max y, min y, max s, min s, max t, min t,
@@ -127,112 +135,189 @@ __global__ __launch_bounds__(256) void k3_extent(const double *__restrict__ x, c
     }
 }
 
-__global__ __launch_bounds__(64) void k3_extent_final(const double *__restrict__ part, int nblk,
-                                                      double *__restrict__ out)
+// One wave per quantity, its loads in flight together (one wave for all nine
+// in turn took 26 us); the results go straight to the host's buffer (pinned memory), then the call's number, for which the host polls: a stream
+// synchronisation returns about 10 us later.
+__global__ __launch_bounds__(64 * 9) void k3_extent_final(const double *__restrict__ part, int nblk, double call,
+                                                          double *__restrict__ out)
 {
-    for (int q = 0; q < 9; ++q) {
-        const bool mn = (q & 1) && q < 8;
-        double r = mn ? (double)FLT_MAX : -(double)FLT_MAX;
-        if (q == 8) r = 0.0;
-        for (int b = threadIdx.x; b < nblk; b += 64) r = mn ? fmin(r, part[b * 9 + q]) : fmax(r, part[b * 9 + q]);
-        r = mn ? wmin(r) : wmax(r);
-        if (threadIdx.x == 0) out[q] = r;
-    }
+    const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const bool mn = (q & 1) && q < 8;
+    const double none = q == 8 ? 0.0 : mn ? (double)FLT_MAX : -(double)FLT_MAX;
+    double v[kExtentBlocks / 64];
+#pragma unroll
+    for (int k = 0; k < kExtentBlocks / 64; ++k) v[k] = 64 * k + lane < nblk ? part[(64 * k + lane) * 9 + q] : none;
+    double r = none;
+#pragma unroll
+    for (int k = 0; k < kExtentBlocks / 64; ++k) r = mn ? fmin(r, v[k]) : fmax(r, v[k]);
+    r = mn ? wmin(r) : wmax(r);
+    if (lane == 0) __hip_atomic_store(&out[q], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(&out[9], call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ------------------------------------------------------------ 2. points and bins
-__device__ __forceinline__ int bin_of(int i, int j, const Par &p)
-{
-    return (j / kTile) * p.nbx + i / kTile;
-}
-
-__global__ __launch_bounds__(256) void k3_prep_in(const double *__restrict__ x0, const double *__restrict__ y0,
-                                                  const double2 *__restrict__ f, int n, Par p,
-                                                  InRec *__restrict__ rec, int2 *__restrict__ kr,
-                                                  int *__restrict__ cnt)
+// Keys: inputs their 8 x 8-cell bin; outputs their 16 x 16-cell bin and the
+// 8 x 2 block inside it (8 rows, 2 columns), so that 16 outputs in a row share
+// most of their windows: 39 taps cover 46 rows (three MFMA tiles, as one window
+// does) and about 41 columns.  Key nki / nko (never read) takes cells outside the grid,
+// which the extents rule out but for rounding at huge offsets.
+__device__ __forceinline__ void prep_in(int k, const double *__restrict__ x0, const double *__restrict__ y0,
+                                        const double2 *__restrict__ f, const Par &p, InRec *__restrict__ rec,
+                                        int2 *__restrict__ kr, int *__restrict__ cnt)
 {
 #pragma clang fp contract(off)
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
     // spatialConvolutionFunction (:38-63), on the rescaled x / kk_x, y / kk_y (:247-248)
     const double x = x0[k] / p.kkx, y = y0[k] / p.kky;
+    const double2 v = f[k];
+    InRec r;
+    r.xt = (x - p.xb) / p.Dx;
+    r.yt = (y - p.yb) / p.Dy;
+    const int i = (int)floor((double)(p.Mrx / 2) + r.xt) - p.ci, j = (int)floor((double)(p.Mry / 2) + r.yt) - p.cj;
+    const bool ok = i >= 0 && i < p.ni && j >= 0 && j < p.nj;
+    const int bin = ok ? (j / kInBin) * p.ibx + i / kInBin : p.ibx * p.iby;
+    const int rank = atomicAdd(&cnt[bin], 1);
     const double arg = p.sb * x + p.tb * y;
     double sn, cs;
     sincos(arg, &sn, &cs);
-    const double2 v = f[k];
-    InRec r;
     r.re = v.x * cs + v.y * sn;
     r.im = v.y * cs - v.x * sn;
-    r.xt = (x - p.xb) / p.Dx;
-    r.yt = (y - p.yb) / p.Dy;
-    r.nno = (int)floor((double)(p.Mrx / 2) + r.xt);
-    r.mmo = (int)floor((double)(p.Mry / 2) + r.yt);
-    r.pad0 = r.pad1 = 0;
-    // the extents put every cell in [Mrx / 4 - 1, 3 Mrx / 4]; the bound keeps
-    // a rounding at the edge from leaving the grid
-    const int nb = p.ibx * p.iby;
-    const bool ok = r.nno >= 0 && r.nno < p.Mrx && r.mmo >= 0 && r.mmo < p.Mry;
-    const int bin = ok ? (r.mmo / kInBin) * p.ibx + r.nno / kInBin : nb;   // bin nb is never read
     rec[k] = r;
-    kr[k] = make_int2(bin, atomicAdd(&cnt[bin], 1));
+    kr[k] = make_int2(bin, rank);
 }
 
-__global__ __launch_bounds__(256) void k3_prep_out(const double *__restrict__ s0, const double *__restrict__ t0,
-                                                   int n, Par p, OutRec *__restrict__ rec,
-                                                   int2 *__restrict__ kr, int *__restrict__ cnt,
-                                                   double2 *__restrict__ F)
+__device__ __forceinline__ void prep_out(int k, const double *__restrict__ s0, const double *__restrict__ t0,
+                                         const Par &p, OutRec *__restrict__ rec, int2 *__restrict__ kr,
+                                         int *__restrict__ cnt, double2 *__restrict__ F)
 {
 #pragma clang fp contract(off)
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
     // spectralConvolutionFunctionCompensation (:164-167), s * kk_x, t * kk_y (:249-250), Ds = Dt = 1
     const double s = s0[k] * p.kkx, t = t0[k] * p.kky;
+    const double sd = s - p.sb, td = t - p.tb;
     OutRec r;
-    r.sd = s - p.sb;
-    r.td = t - p.tb;
-    r.nsn = (int)floor((double)(p.Mrx / 2) + r.sd);
-    r.difs = ((double)(p.Mrx / 2) + r.sd) - r.nsn;
-    r.ntn = (int)floor((double)(p.Mry / 2) + r.td);
-    r.dift = ((double)(p.Mry / 2) + r.td) - r.ntn;
+    r.nsn = (int)floor((double)(p.Mrx / 2) + sd);
+    r.difs = ((double)(p.Mrx / 2) + sd) - r.nsn;
+    r.ntn = (int)floor((double)(p.Mry / 2) + td);
+    r.dift = ((double)(p.Mry / 2) + td) - r.ntn;
     r.idx = k;
     r.pad = 0;
-    const int nb = p.nbx * p.nby * kTile;   // keys: bin and the row inside it
-    const bool ok = r.nsn >= 0 && r.nsn < p.Mrx && r.ntn >= 0 && r.ntn < p.Mry;
-    const int bin = ok ? bin_of(r.nsn, r.ntn, p) * kTile + r.ntn % kTile : nb;
+    const int i = r.nsn - p.oi, j = r.ntn - p.oj;
+    const bool ok = i >= 0 && i < p.mi && j >= 0 && j < p.mj;
+    const int bin = ok ? ((j / kTile) * p.nbx + i / kTile) * kTile + (j % kTile) / 8 * 8 + (i % kTile) / 2
+                       : p.nbx * p.nby * kTile;
+    const int rank = atomicAdd(&cnt[bin], 1);
     if (!ok) F[k] = make_double2(NAN, NAN);
+    const double a1 = p.Dy * td, a2 = p.Dx * sd;
+    const double temp = exp(p.b * (a1 * a1 + a2 * a2));
+    const double arg = sd * p.xb + td * p.yb;
+    double sn, cs;
+    sincos(arg, &sn, &cs);
+    r.pr = cs * temp;
+    r.pi = sn * temp;
     rec[k] = r;
-    kr[k] = make_int2(bin, atomicAdd(&cnt[bin], 1));
+    kr[k] = make_int2(bin, rank);
 }
 
-// Exclusive scan of the key counts in three steps: k3_scan_local scans each
-// 1024-key segment in LDS and writes the segment totals, k3_scan_totals scans
-// those (one block, a run of totals per thread), k3_scan_add adds them back.
-// start[n] is the total.
-__global__ __launch_bounds__(1024) void k3_scan_local(const int *__restrict__ cnt, int n, int *__restrict__ start,
-                                                      int *__restrict__ tot)
+// Blocks below gin take inputs, the others outputs: one launch, so that the
+// two sides' atomics and arithmetic run beside each other.
+__global__ __launch_bounds__(256) void k3_prep(const double *__restrict__ x, const double *__restrict__ y,
+                                               const double2 *__restrict__ f, int len_in, int gin, Par p,
+                                               InRec *__restrict__ rin, int2 *__restrict__ kin, int *__restrict__ cin,
+                                               const double *__restrict__ s, const double *__restrict__ t, int len_out,
+                                               OutRec *__restrict__ rout, int2 *__restrict__ kout,
+                                               int *__restrict__ cout, double2 *__restrict__ F)
 {
-    __shared__ int sums[1024];
-    const int i = blockIdx.x * 1024 + threadIdx.x;
-    const int v = i < n ? cnt[i] : 0;
-    sums[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        const int u = threadIdx.x >= o ? sums[threadIdx.x - o] : 0;
-        __syncthreads();
-        sums[threadIdx.x] += u;
-        __syncthreads();
+    if ((int)blockIdx.x < gin) {
+        const int k = blockIdx.x * 256 + threadIdx.x;
+        if (k < len_in) prep_in(k, x, y, f, p, rin, kin, cin);
+    } else {
+        const int k = (blockIdx.x - gin) * 256 + threadIdx.x;
+        if (k < len_out) prep_out(k, s, t, p, rout, kout, cout, F);
     }
-    if (i < n) start[i] = sums[threadIdx.x] - v;
-    if (threadIdx.x == 1023) tot[blockIdx.x] = sums[1023];
 }
 
-__global__ __launch_bounds__(1024) void k3_scan_totals(int *__restrict__ tot, int n)
+// One dimension's chirp-z tables (nfft2d_czt.hpp): lines of P cells from p0 on
+// to Q frequencies from q0 on of a side of n, c[k] = e^{-i pi k^2 / n} (k^2
+// reduced mod 2n exactly).
+struct AxisTables {
+    double2 *cin, *cout, *hhat, *tw;   // P, Q, m, m
+    int n, P, Q, p0, q0, m;
+};
+__device__ __forceinline__ double2 chirp3(long long k, int n)
+{
+    double sn, cs;
+    sincospi((double)((k * k) % (2LL * n)) / n, &sn, &cs);
+    return make_double2(cs, -sn);
+}
+// Entry e of the tables; hhat gets the kernel conj(c[d + q0 - p0]) at d mod m,
+// d in (-P, Q), which k3_kernel_fft transforms.  The output factors carry the
+// checkerboard sign (-1)^k of circAndFFTShiftsFunction (:135-151).
+__device__ __forceinline__ void axis_entry(const AxisTables &t, int e)
+{
+    if (e < t.P) t.cin[e] = chirp3((long long)e + t.p0, t.n);
+    if (e < t.Q) {
+        const double2 c = chirp3((long long)e + t.q0, t.n);
+        t.cout[e] = ((e + t.q0) & 1) ? make_double2(-c.x, -c.y) : c;
+    }
+    if (e < t.m) {
+        double sn, cs;
+        sincospi(2.0 * e / t.m, &sn, &cs);
+        t.tw[e] = make_double2(cs, -sn);
+        double2 h = make_double2(0.0, 0.0);
+        const int d = e < t.Q ? e : e - t.m;
+        if (d > -t.P) {
+            h = chirp3((long long)d + t.q0 - t.p0, t.n);
+            h.y = -h.y;
+        }
+        t.hhat[e] = h;
+    }
+}
+
+// Exclusive scan of the key counts in two steps: k3_scan_local scans each
+// 1024-key segment and writes the segment totals, k3_scan_totals scans those;
+// key i starts at start[i] + tot[i >> 10].  Side 0 the inputs, side 1 the
+// outputs; the scan's launch also fills the chirp-z tables (its last blocks).
+struct ScanSide {
+    int *cnt, *start, *tot;
+    int n, segs;   // keys (the out-of-grid one and the end among them), segments
+};
+__global__ __launch_bounds__(1024) void k3_scan_local(ScanSide a, ScanSide b, AxisTables tx, AxisTables ty)
+{
+    __shared__ int wsum[16];
+    int seg = blockIdx.x;
+    if (seg >= a.segs + b.segs) {
+        const int e = (seg - a.segs - b.segs) * 1024 + threadIdx.x;
+        axis_entry(tx, e);
+        axis_entry(ty, e);
+        return;
+    }
+    const ScanSide &s = seg < a.segs ? a : b;
+    if (seg >= a.segs) seg -= a.segs;
+    const int i = seg * 1024 + threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int v = i < s.n ? s.cnt[i] : 0;
+    int inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    int before = 0;
+    for (int k = 0; k < w; ++k) before += wsum[k];
+    if (i < s.n) s.start[i] = before + inc - v;
+    if (threadIdx.x == 1023) s.tot[seg] = before + inc;
+}
+
+__global__ __launch_bounds__(1024) void k3_scan_totals(ScanSide a, ScanSide b)
 {
     __shared__ int sums[1024];
-    const int per = (n + 1023) / 1024;
-    const int lo = min(n, (int)threadIdx.x * per), hi = min(n, lo + per);
+    const ScanSide &s = blockIdx.x ? b : a;
+    const int per = (s.segs + 1023) / 1024;
+    const int lo = min(s.segs, (int)threadIdx.x * per), hi = min(s.segs, lo + per);
     int acc = 0;
-    for (int i = lo; i < hi; ++i) acc += tot[i];
+    for (int i = lo; i < hi; ++i) acc += s.tot[i];
     sums[threadIdx.x] = acc;
     __syncthreads();
     for (int o = 1; o < 1024; o <<= 1) {
@@ -243,156 +328,208 @@ __global__ __launch_bounds__(1024) void k3_scan_totals(int *__restrict__ tot, in
     }
     int run = sums[threadIdx.x] - acc;
     for (int i = lo; i < hi; ++i) {
-        const int v = tot[i];
-        tot[i] = run;
+        const int v = s.tot[i];
+        s.tot[i] = run;
         run += v;
     }
-    if (threadIdx.x == 1023) tot[n] = sums[1023];
 }
 
-__global__ __launch_bounds__(256) void k3_scan_add(int *__restrict__ start, int n, const int *__restrict__ tot)
+__device__ __forceinline__ int key_start(const int *__restrict__ st, const int *__restrict__ tot, int i)
 {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) start[i] += tot[i >> 10];
-    if (i == n) start[n] = tot[(n + 1023) >> 10];
+    return st[i] + tot[i >> 10];
 }
 
-template <typename R>
-__global__ __launch_bounds__(256) void k3_scatter(const R *__restrict__ rec, const int2 *__restrict__ kr, int n,
-                                                  const int *__restrict__ st, R *__restrict__ out)
+__global__ __launch_bounds__(256) void k3_scatter(const InRec *__restrict__ rin, const int2 *__restrict__ kin,
+                                                  int len_in, int gin, ScanSide a, InRec *__restrict__ sin_,
+                                                  const OutRec *__restrict__ rout, const int2 *__restrict__ kout,
+                                                  int len_out, ScanSide b, OutRec *__restrict__ sout)
 {
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    const int2 e = kr[k];
-    out[st[e.x] + e.y] = rec[k];
-}
-
-// The inputs' scatter also writes their cells, in the same order, to an
-// 8-byte array: the spread's reach test reads only that.
-__global__ __launch_bounds__(256) void k3_scatter_in(const InRec *__restrict__ rec, const int2 *__restrict__ kr,
-                                                     int n, const int *__restrict__ st, InRec *__restrict__ out,
-                                                     int2 *__restrict__ cells)
-{
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= n) return;
-    const int2 e = kr[k];
-    const InRec r = rec[k];
-    const int pos = st[e.x] + e.y;
-    out[pos] = r;
-    cells[pos] = make_int2(r.nno, r.mmo);
+    if ((int)blockIdx.x < gin) {
+        const int k = blockIdx.x * 256 + threadIdx.x;
+        if (k >= len_in) return;
+        const int2 e = kin[k];
+        sin_[key_start(a.start, a.tot, e.x) + e.y] = rin[k];
+    } else {
+        const int k = (blockIdx.x - gin) * 256 + threadIdx.x;
+        if (k >= len_out) return;
+        const int2 e = kout[k];
+        sout[key_start(b.start, b.tot, e.x) + e.y] = rout[k];
+    }
 }
 
 // ------------------------------------------------------------ 3. Gaussian gridding
-// Block per 16 x 16 tile (tx, ty) of the row-major Mry x Mrx grid: cells
-// i in [16 tx, 16 tx + 16), j in [16 ty, 16 ty + 16).  An input k reaches cell
-// (i, j) when |i - nno_k| <= msp and |j - mmo_k| <= msp (:65-72).  The 4 waves
-// take turns over the 64-input chunks of the 8 x 8-cell input bins within
-// ceil(msp / 8) of the tile (the reach test reads the 8-byte cell array; only
-// inputs within reach load their record) and sum their partial tiles in LDS
-// at the end, in wave order.
-// In a chunk, each input that reaches the tile writes its 16 row and 16
-// column Gaussian factors for the tile to a slot in LDS (zero outside its
-// reach), from two exponentials per dimension and a product recurrence (fast
-// Gaussian gridding, Greengard & Lee, SIAM Rev. 46 (2004)): with
-// u = yt - (j0 - Mry/2),
-//     e^{-t1 (u - r - 1)^2} = e^{-t1 (u - r)^2} rho_r,
-//     rho_r = e^{2 t1 (u - r) - t1},  rho_{r+1} = rho_r e^{-2 t1}.
+// Block per 16 x 16 tile (tx, ty) of the reached cells: i in [i0, i0 + 16),
+// i0 = gi + 16 tx, j likewise.  An input k reaches cell (i, j) when
+// |i - nno_k| <= R and |j - mmo_k| <= R, R = msp (:65-72) or less (tap_reach).
+// The 4 waves take turns over the 64-input chunks of the 8 x 8-cell input bins that can reach the
+// tile, the next chunk's records in flight.  The inputs within reach (about
+// two thirds) go to a queue in LDS, and each full batch of 32 is spread: lane l
+// of the lower half takes input l of the batch and writes its 16 row factors
+// ey to a slot, lane l + 32 its 16 column factors ex, from two exponentials
+// and one product each (fast Gaussian gridding, Greengard & Lee, SIAM Rev. 46
+// (2004)): with u = yt - (j0 - Mry/2),
+//     e^{-t1 (u - r)^2} = e^{-t1 u^2} (e^{2 t1 u})^r e^{-t1 r^2},
+// the last factor, the same for every input, taken into the finished cell's.
+// (e^{2 t1 u r} stays below e^{2 t1 (R + 16) 15}, far inside the range.)
 // The slots are then taken four per MFMA step: lane l supplies
 // A[r][k] = c_k ey_k(j0 + r) and B[k][r] = ex_k(i0 + r) at r = l % 16,
 // k = l / 16, and accumulator element q of lane l is cell
 // (j0 + 4 q + l / 16, i0 + l % 16).
+// MASK: factors outside an input's reach are set to zero.  Without it an input
+// that reaches the tile adds its tails there too; beyond R cells a factor is
+// below e^{-t1 R^2}, which the host finds to be under 2^-54 of the input's
+// largest, and the two selects per factor would cost more than its product.
+// What bounds it is FP64 arithmetic: this GPU's FP64 matrix rate is its vector
+// rate, and the counters add up as if both shared one pipe (112K matrix and
+// about 80K vector cycles of 245K with R = 19).  So the batches keep every lane
+// of the factors' work busy (one lane per candidate left a third idle, and its
+// slots held LDS for two blocks a CU only), and tails that change nothing are
+// not formed.  300,000 inputs, msp 19: 229 us; in batches 119, with one product
+// a factor and without the floors in the reach test 116, with R = 16 90.
 constexpr int kSpreadWaves = 4;
 constexpr int kChunk = 64;        // candidate inputs per wave and round
-constexpr int kRow = kTile + 1;   // padded slot row (doubles): lane-strided writes spread over the banks
+constexpr int kBatch = 32;        // inputs spread at a time
+constexpr int kQueue = kBatch - 1 + kChunk;
+constexpr int kRow = kTile + 2;   // padded slot row (doubles, 16-byte aligned)
+constexpr int kMaxBinRows = (kTile + 2 * kMaxMsp) / kInBin + 2;   // bin rows that can reach a tile
+static_assert(kMaxBinRows <= 64, "one lane per bin row");
 
+struct SpreadLds {
+    InRec q[kQueue];
+    double ey[kBatch][kRow], ex[kBatch][kRow];
+};
+
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <bool MASK>
 __global__ __launch_bounds__(64 * kSpreadWaves) void k3_spread(const InRec *__restrict__ pts,
-                                                                const int2 *__restrict__ cells,
-                                                                const int *__restrict__ st, Par p,
+                                                                const int *__restrict__ st,
+                                                                const int *__restrict__ tot, Par p, int ntx,
                                                                 double2 *__restrict__ G)
 {
     __shared__ union {
-        struct {
-            double ey[kSpreadWaves][kChunk][kRow], ex[kSpreadWaves][kChunk][kRow];
-            double2 c[kSpreadWaves][kChunk];
-        } s;
+        SpreadLds s[kSpreadWaves];
         double2 part[kSpreadWaves][kTile * kTile];
     } sh;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int tx = blockIdx.x % p.nbx, ty = blockIdx.x / p.nbx;
-    const int i0 = tx * kTile, j0 = ty * kTile;
+    SpreadLds &L = sh.s[w];
+    const int tx = blockIdx.x % ntx, ty = blockIdx.x / ntx;
+    const int i0 = p.gi + tx * kTile, j0 = p.gj + ty * kTile;
     const int r = lane & 15, ks = lane >> 4;
-    const double oy = (double)(j0 - p.Mry / 2), ox = (double)(i0 - p.Mrx / 2);
-    const double kap = exp(-2.0 * p.t1);
-    const int msp = p.msp, reach = (msp + kInBin - 1) / kInBin;   // in input bins
-    const int rows = min(kTile, p.Mry - j0), cols = min(kTile, p.Mrx - i0);   // cells inside the grid
+    const bool rows_half = lane < 32;                     // this lane's factors: rows (ey) or columns (ex)
+    const int sl = lane & 31;
+    const double org = rows_half ? (double)(j0 - p.Mry / 2) : (double)(i0 - p.Mrx / 2);
+    const int half_grid = rows_half ? p.Mry / 2 : p.Mrx / 2, cell0 = rows_half ? j0 : i0;
+    const int R = p.reach;
     d4 accr = {0.0, 0.0, 0.0, 0.0}, acci = {0.0, 0.0, 0.0, 0.0};
-    constexpr int kSub = kTile / kInBin;   // input bins per tile side
-    const int by0 = max(0, kSub * ty - reach), by1 = min(p.iby - 1, kSub * ty + kSub - 1 + reach);
-    const int bx0 = max(0, kSub * tx - reach), bx1 = min(p.ibx - 1, kSub * tx + kSub - 1 + reach);
-    const int2 far = make_int2(-(1 << 29), -(1 << 29));   // reaches nothing
-    for (int by = by0; by <= by1; ++by) {
-        const int s0 = st[by * p.ibx + bx0], s1 = st[by * p.ibx + bx1 + 1];   // the row's bins are contiguous
-        int base = s0 + kChunk * w;
-        int2 nxt = base + lane < s1 ? cells[base + lane] : far;
-        for (; base < s1; base += kChunk * kSpreadWaves) {
-            const int2 cell = nxt;
-            const int after = base + kChunk * kSpreadWaves + lane;
-            nxt = after < s1 ? cells[after] : far;
-            const bool in = cell.x + msp >= i0 && cell.x - msp < i0 + kTile && cell.y + msp >= j0 &&
-                            cell.y - msp < j0 + kTile;
-            const unsigned long long mask = __ballot(in);
-            if (mask == 0ull) continue;
-            if (in) {
-                const InRec *ep = pts + base + lane;   // only inputs within reach load their record
-                const double2 xy = *reinterpret_cast<const double2 *>(&ep->xt);
-                const double2 cv = *reinterpret_cast<const double2 *>(&ep->re);
-                const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
-                                                          __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-                sh.s.c[w][pos] = cv;
-                // rows: reach [mmo - msp, mmo + msp] relative to j0, cells inside the grid
-                const int ylo = max(0, cell.y - msp - j0), yhi = min(rows - 1, cell.y + msp - j0);
-                const int xlo = max(0, cell.x - msp - i0), xhi = min(cols - 1, cell.x + msp - i0);
-                const double uy = xy.y - oy, ux = xy.x - ox;
-                double gy = exp(-p.t1 * (uy * uy)), ry = exp(2.0 * p.t1 * uy - p.t1);
-                double gx = exp(-p.t1 * (ux * ux)), rx = exp(2.0 * p.t1 * ux - p.t1);
-                double *py = sh.s.ey[w][pos], *px = sh.s.ex[w][pos];
-#pragma unroll
-                for (int q = 0; q < kTile; ++q) {
-                    py[q] = q >= ylo && q <= yhi ? gy : 0.0;
-                    px[q] = q >= xlo && q <= xhi ? gx : 0.0;
-                    gy *= ry;
-                    ry *= kap;
-                    gx *= rx;
-                    rx *= kap;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            const int n = __popcll(mask);
-            for (int q = 0; q < n; q += 4) {
-                const int sl = q + ks;
-                double ar = 0.0, ai = 0.0, bb = 0.0;
-                if (sl < n) {
-                    const double2 c = sh.s.c[w][sl];
-                    const double wy = sh.s.ey[w][sl][r];
-                    ar = c.x * wy;
-                    ai = c.y * wy;
-                    bb = sh.s.ex[w][sl][r];
-                }
-                accr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bb, accr, 0, 0, 0);
-                acci = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bb, acci, 0, 0, 0);
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();   // slot reads done before the next chunk's writes
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int by0 = max(0, j0 - R - p.cj) / kInBin, by1 = min(p.iby - 1, (j0 + kTile - 1 + R - p.cj) / kInBin);
+    const int bx0 = max(0, i0 - R - p.ci) / kInBin, bx1 = min(p.ibx - 1, (i0 + kTile - 1 + R - p.ci) / kInBin);
+    // a bin row's inputs are contiguous; lane l holds row by0 + l's range
+    int lo_l = 0, hi_l = 0;
+    if (by0 + lane <= by1 && bx0 <= bx1) {
+        const int k0 = (by0 + lane) * p.ibx + bx0;
+        lo_l = key_start(st, tot, k0);
+        hi_l = key_start(st, tot, k0 + bx1 - bx0 + 1);
+    }
+
+    // inputs whose cell is in [i0 - R, i0 + 16 + R) x [j0 - R, j0 + 16 + R) reach the tile
+    const double ilo = i0 - R, ihi = i0 + kTile + R, jlo = j0 - R, jhi = j0 + kTile + R;
+    int n = 0;                                            // queued inputs
+    auto batch = [&](int q0) {
+        // factors of the batch's inputs q0 .. q0 + 31
+        const InRec &e = L.q[q0 + sl];
+        const double d = rows_half ? e.yt : e.xt, u = d - org;
+        double g = exp(-p.t1 * (u * u));
+        const double e1 = exp(2.0 * p.t1 * u);
+        int lo = 0, hi = kTile - 1;
+        if (MASK) {
+            const int c = (int)floor((double)half_grid + d) - cell0;
+            lo = c - R;
+            hi = c + R;
         }
+        double *o = rows_half ? L.ey[sl] : L.ex[sl];
+#pragma unroll
+        for (int k = 0; k < kTile; k += 2) {
+            double2 v;
+            v.x = !MASK || (k >= lo && k <= hi) ? g : 0.0;
+            g *= e1;
+            v.y = !MASK || (k + 1 >= lo && k + 1 <= hi) ? g : 0.0;
+            g *= e1;
+            *reinterpret_cast<double2 *>(o + k) = v;
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < kBatch; q += 4) {
+            const int b = q + ks;
+            const double2 c = *reinterpret_cast<const double2 *>(&L.q[q0 + b].re);
+            const double wy = L.ey[b][r], wx = L.ex[b][r];
+            accr = __builtin_amdgcn_mfma_f64_16x16x4f64(c.x * wy, wx, accr, 0, 0, 0);
+            acci = __builtin_amdgcn_mfma_f64_16x16x4f64(c.y * wy, wx, acci, 0, 0, 0);
+        }
+        wave_lds_sync();                                  // slots and queue entries are free again
+    };
+
+    // this wave's chunks, row after row: chunk k of a row is wave (turn + k) % 4's
+    int by = by0 - 1, base = 0, s1 = 0, turn = 0;
+    auto advance = [&]() {
+        base += kChunk * kSpreadWaves;
+        while (base >= s1 && ++by <= by1) {
+            const int s0 = __builtin_amdgcn_readlane(lo_l, by - by0);
+            s1 = __builtin_amdgcn_readlane(hi_l, by - by0);
+            base = s0 + kChunk * ((w - turn) & (kSpreadWaves - 1));
+            turn += (s1 - s0 + kChunk - 1) / kChunk;
+        }
+    };
+    auto fetch = [&]() {
+        InRec v;
+        v.xt = v.yt = 1e300;                              // reaches nothing
+        v.re = v.im = 0.0;
+        if (by <= by1 && base + lane < s1) v = pts[base + lane];
+        return v;
+    };
+    advance();
+    InRec cur = fetch();
+    while (by <= by1) {
+        advance();
+        const InRec nxt = fetch();
+        // the cell is the floor of these, as k3_prep found it
+        const double vi = (double)(p.Mrx / 2) + cur.xt, vj = (double)(p.Mry / 2) + cur.yt;
+        const bool in = vi >= ilo && vi < ihi && vj >= jlo && vj < jhi;
+        const unsigned long long mask = __ballot(in);
+        if (in) {
+            const int pos = __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+            L.q[n + pos] = cur;
+        }
+        n += __popcll(mask);
+        wave_lds_sync();
+        while (n >= kBatch) {
+            n -= kBatch;
+            batch(n);
+        }
+        cur = nxt;
+    }
+    if (n > 0) {                                          // the rest, zero samples behind it
+        if (lane >= n && lane < kBatch) {
+            InRec z;
+            z.xt = (double)(i0 - p.Mrx / 2);
+            z.yt = (double)(j0 - p.Mry / 2);
+            z.re = z.im = 0.0;
+            L.q[lane] = z;
+        }
+        wave_lds_sync();
+        batch(0);
     }
     __syncthreads();   // every wave's slot reads are done: the partial tiles may overwrite them
 #pragma unroll
     for (int q = 0; q < 4; ++q) sh.part[w][(4 * q + ks) * kTile + r] = make_double2(accr[q], acci[q]);
     __syncthreads();
-    if (threadIdx.x < kTile * kTile) {
+    {
         const int cell = threadIdx.x, ii = i0 + cell % kTile, jj = j0 + cell / kTile;
         double sr = 0.0, si = 0.0;
 #pragma unroll
@@ -401,231 +538,89 @@ __global__ __launch_bounds__(64 * kSpreadWaves) void k3_spread(const InRec *__re
             sr += v.x;
             si += v.y;
         }
-        if (jj < p.Mry && ii < p.Mrx) {
+        if (jj < p.gj + p.Py && ii < p.gi + p.Px) {
             const double ddi = (double)(ii - p.Mrx / 2), ddj = (double)(jj - p.Mry / 2);
-            const double sc = p.fact * exp(p.b * (p.Dy * p.Dy * ddj * ddj) + p.b * (p.Dx * p.Dx * ddi * ddi));
-            G[(size_t)jj * p.Mrx + ii] = make_double2(sr * sc, si * sc);
+            const double ri = (double)(ii - i0), rj = (double)(jj - j0);
+            const double sc = p.fact * exp(p.b * (p.Dy * p.Dy * ddj * ddj) + p.b * (p.Dx * p.Dx * ddi * ddi)) *
+                              exp(-p.t1 * (ri * ri + rj * rj));
+            G[(size_t)(jj - p.gj) * p.Px + (ii - p.gi)] = make_double2(sr * sc, si * sc);
         }
     }
 }
+static_assert(64 * kSpreadWaves == kTile * kTile, "one cell per thread in the sum");
 
 // ------------------------------------------------------------ 4. FFTs of the grid lines
-// In-place radix-4 (and one radix-2) Stockham FFT of m = 2^a points in LDS,
-// forward (e^{-2 pi i jk / m}), after Govindaraju et al., "High performance
-// discrete Fourier transforms on graphics processors" (SC 2008): stage with
-// span Ns reads v_r = X[j + r m/R], twiddles it by e^{-2 pi i r (j mod Ns) /
-// (Ns R)}, and writes the R-point DFT of v to X[(j - j mod Ns) R + j mod Ns
-// + r Ns].  All reads of a stage precede its writes (barrier), so one buffer
-// serves.  Twiddles e^{-2 pi i t / m} = T1[t / 64] T2[t % 64] from two small
-// LDS tables.  Every thread holds at most 8 values.
-struct TwLds {
-    const double2 *t1, *t2;
-    __device__ double2 operator[](int t) const { return cmul(t1[t >> 6], t2[t & 63]); }
-};
-
-__device__ void lds_fft(double2 *X, int m, const TwLds tw)
-{
-    const int T = blockDim.x, tid = threadIdx.x;
-    for (int Ns = 1; Ns < m;) {
-        const int R = (m / Ns) >= 4 ? 4 : 2;
-        const int nb = m / R, per = (nb + T - 1) / T;   // butterflies per thread: <= 2 (radix 4), <= 4 (radix 2)
-        const int tstep = m / (Ns * R);
-        double2 v[8];
-        if (R == 4) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int j = tid + u * T;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1);
-                    double2 a0 = X[j], a1 = X[j + nb], a2 = X[j + 2 * nb], a3 = X[j + 3 * nb];
-                    if (Ns > 1) {
-                        a1 = cmul(a1, tw[k * tstep]);
-                        a2 = cmul(a2, tw[2 * k * tstep]);
-                        a3 = cmul(a3, tw[3 * k * tstep]);
-                    }
-                    const double2 b0 = make_double2(a0.x + a2.x, a0.y + a2.y);
-                    const double2 b1 = make_double2(a0.x - a2.x, a0.y - a2.y);
-                    const double2 b2 = make_double2(a1.x + a3.x, a1.y + a3.y);
-                    const double2 b3 = make_double2(a1.y - a3.y, a3.x - a1.x);   // (a1 - a3) (-i)
-                    v[4 * u + 0] = make_double2(b0.x + b2.x, b0.y + b2.y);
-                    v[4 * u + 1] = make_double2(b1.x + b3.x, b1.y + b3.y);
-                    v[4 * u + 2] = make_double2(b0.x - b2.x, b0.y - b2.y);
-                    v[4 * u + 3] = make_double2(b1.x - b3.x, b1.y - b3.y);
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int j = tid + u * T;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1), o = (j - k) * 4 + k;
-                    X[o] = v[4 * u];
-                    X[o + Ns] = v[4 * u + 1];
-                    X[o + 2 * Ns] = v[4 * u + 2];
-                    X[o + 3 * Ns] = v[4 * u + 3];
-                }
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = tid + u * T;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1);
-                    double2 a0 = X[j], a1 = X[j + nb];
-                    if (Ns > 1) a1 = cmul(a1, tw[k * tstep]);
-                    v[2 * u] = make_double2(a0.x + a1.x, a0.y + a1.y);
-                    v[2 * u + 1] = make_double2(a0.x - a1.x, a0.y - a1.y);
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int j = tid + u * T;
-                if (u < per && j < nb) {
-                    const int k = j & (Ns - 1), o = (j - k) * 2 + k;
-                    X[o] = v[2 * u];
-                    X[o + Ns] = v[2 * u + 1];
-                }
-            }
-        }
-        __syncthreads();
-        Ns *= R;
-    }
-}
-
-// Forward DFT of `lines` contiguous lines of n points (line stride n), one
-// line per block, m = n (n a power of two) or Bluestein at m >= 2n - 1:
-//   X_k = w_k sum_j (x_j w_j) conj(w_{k-j}),  w_j = e^{-i pi j^2 / n},
-// the convolution taken as IFFT(FFT(x w) * bh), bh = FFT of the wrapped
-// conj(w) sequence, and IFFT(Y) = conj(FFT(conj(Y))) / m.
-// LDS: m data values, then the twiddle tables T1 (m / 64 entries, at least
-// 1) and T2 (64).
-__host__ __device__ constexpr int fft_lds_entries(int m) { return m + (m >= 64 ? m / 64 : 1) + 64; }
-
-__global__ __launch_bounds__(1024) void k3_fft_lines(double2 *__restrict__ data, int n, int m,
-                                                     const double2 *__restrict__ twg,
-                                                     const double2 *__restrict__ chirp,
-                                                     const double2 *__restrict__ bh)
+// The convolution kernels' transforms in place, block 0 for x, 1 for y (a
+// block whose side has another length leaves at once).
+template <int LOGM>
+__global__ __launch_bounds__((1 << LOGM) / 8) void k3_kernel_fft(AxisTables tx, AxisTables ty)
 {
     extern __shared__ double2 X[];
-    double2 *t1 = X + m, *t2 = t1 + (m >= 64 ? m / 64 : 1);
-    double2 *row = data + (size_t)blockIdx.x * n;
-    const int T = blockDim.x;
-    for (int k = threadIdx.x; k < 64; k += T) t2[k] = k < m ? twg[k] : make_double2(1.0, 0.0);
-    for (int k = threadIdx.x; k < (m >= 64 ? m / 64 : 1); k += T) t1[k] = twg[64 * k];
-    const TwLds tw{t1, t2};
-    if (!chirp) {
-        for (int k = threadIdx.x; k < m; k += T) X[k] = row[k];
-        __syncthreads();
-        lds_fft(X, m, tw);
-        for (int k = threadIdx.x; k < m; k += T) row[k] = X[k];
-        return;
-    }
-    for (int k = threadIdx.x; k < m; k += T) X[k] = k < n ? cmul(row[k], chirp[k]) : make_double2(0.0, 0.0);
-    __syncthreads();
-    lds_fft(X, m, tw);
-    for (int k = threadIdx.x; k < m; k += T) {
-        const double2 z = cmul(X[k], bh[k]);
-        X[k] = make_double2(z.x, -z.y);
-    }
-    __syncthreads();
-    lds_fft(X, m, tw);
-    const double inv = 1.0 / m;
-    for (int k = threadIdx.x; k < n; k += T) {
-        const double2 z = X[k];
-        row[k] = cmul(make_double2(z.x * inv, -z.y * inv), chirp[k]);
-    }
-}
-
-// tw[t] = e^{-2 pi i t / m}, t < m.
-__global__ __launch_bounds__(256) void k3_twiddles(int m, double2 *__restrict__ tw)
-{
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= m) return;
-    double sn, cs;
-    sincospi(2.0 * t / m, &sn, &cs);
-    tw[t] = make_double2(cs, -sn);
-}
-
-// Bluestein tables of a length-n line: chirp[j] = e^{-i pi j^2 / n} (j < n;
-// j^2 reduced mod 2n exactly) and b = the length-m sequence holding
-// conj(chirp[j]) at j and at m - j, zero between (transformed in place
-// afterwards).
-__global__ __launch_bounds__(256) void k3_chirp(int n, int m, double2 *__restrict__ chirp, double2 *__restrict__ b)
-{
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    if (j >= m) return;
-    double2 bj = make_double2(0.0, 0.0);
-    const int jj = j < n ? j : (j > m - n ? m - j : -1);
-    if (jj >= 0) {
-        const long long q = ((long long)jj * jj) % (2LL * n);
-        double sn, cs;
-        sincospi((double)q / n, &sn, &cs);
-        if (j < n) chirp[j] = make_double2(cs, -sn);
-        bj = make_double2(cs, sn);
-    }
-    b[j] = bj;
-}
-
-// out[c][r] = in[r][c], in: rows x cols.
-__global__ __launch_bounds__(256) void k3_transpose(const double2 *__restrict__ in, double2 *__restrict__ out,
-                                                    int rows, int cols)
-{
-    __shared__ double2 tile[32][33];
-    const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-    for (int k = ty; k < 32; k += 8) {
-        const int rr = r0 + k, cc = c0 + tx;
-        if (rr < rows && cc < cols) tile[k][tx] = in[(size_t)rr * cols + cc];
-    }
-    __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-        const int cc = c0 + k, rr = r0 + tx;
-        if (rr < rows && cc < cols) out[(size_t)cc * rows + rr] = tile[tx][k];
-    }
+    const AxisTables &t = blockIdx.x ? ty : tx;
+    if (t.m != 1 << LOGM) return;
+    constexpr int TPL = (1 << LOGM) / 8;
+    const bool act[1] = {true};
+    const int line[1] = {0}, j[1] = {(int)threadIdx.x};
+    double2 v[1][8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[0][q] = t.hhat[j[0] + q * TPL];
+    nfft2d::czt_fft<double, LOGM, 1>(v, X, t.tw, act, line, j, line, j, line, j);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) t.hhat[j[0] + q * TPL] = v[0][q];
 }
 
 // ------------------------------------------------------------ 5. interpolation at the outputs
-// Block per output bin (by, bx), 8 waves.  The patch of the shifted spectrum
-//     gs[mm][nn] = (-1)^(i + j) FT[j][i],  i = (nn + Mrx/2) mod Mrx,
-//     j = (mm + Mry/2) mod Mry
-// (FT the 2-D DFT, held transposed as FTt[i][j]) for mm in
-// [16 by - msp, 16 by + 16 + msp) and nn likewise goes to LDS as P[c][a]
-// (c = nn offset, a = mm offset, W = 16 + 2 msp per side; wrapped indices
-// outside the grid are loaded but never weighted).  The outputs of the bin
-// come sorted by their row ntn.  A wave takes 16 of them at a time and
-// contracts, for each output j, H_j[a] = sum_c P[c][a] ex_j[c] on
-// v_mfma_f64_16x16x4f64 (A[a][k] = P[c0 + k][a0 + a] from LDS,
+// Block per output bin (by, bx), 8 waves.  The patch of the spectrum for mm in
+// [m0 - R, m0 + 16 + R), m0 = oj + 16 by, and nn likewise goes to LDS as
+// P[c][a] (c = nn offset, a = mm offset, W = 16 + 2 R per side; entries past
+// the read frequencies are loaded from the edge and never weighted).  The
+// outputs of the bin come sorted by 8 x 2-cell blocks.  A wave takes 16 of
+// them at a time and contracts, for each output j, H_j[a] = sum_c P[c][a]
+// ex_j[c] on v_mfma_f64_16x16x4f64 (A[a][k] = P[c0 + k][a0 + a] from LDS,
 // B[k][j] = ex_j[c0 + k], accumulator element q of lane l = H_{l % 16}[a0 + 4 q
 // + l / 16]) over the rows and columns that the 16 windows cover, then
-// F_j = sum_a ey_j[a] H_j[a] and the post-compensation.  Along c the taps
-// follow e^{-t1 (d - c - 4)^2} = e^{-t1 (d - c)^2} rho_c, rho_{c+4} = rho_c
-// e^{-32 t1} (two multiplications per step).
+// F_j = sum_a ey_j[a] H_j[a] and the post-compensation.  The taps follow
+// e^{-t1 (d - c - 4)^2} = e^{-t1 (d - c)^2} rho_c, rho_{c+4} = rho_c e^{-32 t1}
+// along both c and a (two multiplications per step).
+// Bound by FP64 arithmetic, most of it two 64-cycle products per 16 rows, 4
+// columns and 16 outputs.  Outputs sorted by rows covered 54 columns a group,
+// sorted by blocks about 41.  300,000 outputs, msp 19: 136 us; by blocks, with
+// recurrences along both sides and the compensation in k3_prep 96, without the
+// masks 81, with R = 16 69.
+// MASK as in the spread: past its window an output's tails are below 2^-54 of
+// its largest tap.
 constexpr int kInterpWaves = 8;
 
-__global__ __launch_bounds__(64 * kInterpWaves) void k3_interp(const double2 *__restrict__ FTt,
+// Minimum over the 16 lanes of a row.
+__device__ __forceinline__ int row_min(int v)
+{
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0xB1, 0xf, 0xf, false));    // lanes 1 0 3 2
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x4E, 0xf, 0xf, false));    // lanes 2 3 0 1
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x141, 0xf, 0xf, false));   // mirrored in 8
+    return min(v, __builtin_amdgcn_update_dpp(v, v, 0x140, 0xf, 0xf, false));   // mirrored in 16
+}
+
+template <bool MASK>
+__global__ __launch_bounds__(64 * kInterpWaves) void k3_interp(const double2 *__restrict__ S,
                                                                 const OutRec *__restrict__ outs,
-                                                                const int *__restrict__ st, Par p,
+                                                                const int *__restrict__ st,
+                                                                const int *__restrict__ tot, Par p,
                                                                 double2 *__restrict__ F)
 {
     extern __shared__ double2 P[];
     const int bin = blockIdx.x;
-    const int s0 = st[bin * kTile], s1 = st[bin * kTile + kTile];   // the bin's 16 row keys
+    const int s0 = key_start(st, tot, bin * kTile), s1 = key_start(st, tot, bin * kTile + kTile);   // its 16 keys
     if (s0 == s1) return;
     const int bx = bin % p.nbx, by = bin / p.nbx;
-    const int msp = p.msp, W = kTile + 2 * msp, taps = 2 * msp + 1;
-    const int mm0 = by * kTile - msp, nn0 = bx * kTile - msp;
+    const int R = p.reach, W = kTile + 2 * R, taps = 2 * R + 1;
+    const int mm0 = p.oj + by * kTile - R, nn0 = p.oi + bx * kTile - R;
+    // S[i][j]: frequency qi + i, qj + j; cell nn is frequency nn - Mrx/2
     for (int e = threadIdx.x; e < W * W; e += 64 * kInterpWaves) {
-        const int a = e % W, c = e / W;   // a: mm offset (contiguous in FTt), c: nn offset
-        int mm = mm0 + a, nn = nn0 + c;
-        mm += mm < 0 ? p.Mry : (mm >= p.Mry ? -p.Mry : 0);
-        nn += nn < 0 ? p.Mrx : (nn >= p.Mrx ? -p.Mrx : 0);
-        int i = nn + p.Mrx / 2, j = mm + p.Mry / 2;
-        i -= i >= p.Mrx ? p.Mrx : 0;
-        j -= j >= p.Mry ? p.Mry : 0;
-        double2 v = FTt[(size_t)i * p.Mry + j];
-        if ((i + j) & 1) v = make_double2(-v.x, -v.y);
-        P[c * W + a] = v;
+        const int a = e % W, c = e / W;   // a: mm offset (contiguous in S), c: nn offset
+        int i = nn0 + c - p.Mrx / 2 - p.qi, j = mm0 + a - p.Mry / 2 - p.qj;
+        i = i >= p.Qx && p.Qx == p.Mrx ? i - p.Mrx : i;   // the whole side is held: periodic
+        j = j >= p.Qy && p.Qy == p.Mry ? j - p.Mry : j;
+        P[c * W + a] = S[(size_t)min(i, p.Qx - 1) * p.Qy + min(j, p.Qy - 1)];
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -635,58 +630,55 @@ __global__ __launch_bounds__(64 * kInterpWaves) void k3_interp(const double2 *__
         const int o = g + jo;
         const bool valid = o < s1;
         const OutRec rec = outs[valid ? o : s1 - 1];
-        const int ra = rec.ntn - msp - mm0, ca = rec.nsn - msp - nn0;   // window origin in the patch, in [0, 16)
-        int rlo = valid ? ra : 1 << 20, rhi = valid ? ra : -(1 << 20);
-        int clo = valid ? ca : 1 << 20, chi = valid ? ca : -(1 << 20);
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-            rlo = min(rlo, __shfl_xor(rlo, off, 64));
-            rhi = max(rhi, __shfl_xor(rhi, off, 64));
-            clo = min(clo, __shfl_xor(clo, off, 64));
-            chi = max(chi, __shfl_xor(chi, off, 64));
-        }
-        rhi += taps - 1;
-        chi += taps - 1;
-        const double dxc = rec.difs + ca + msp;   // ex_j[c] = e^{-t1 (dxc - c)^2} on c in [ca, ca + 2 msp]
-        const double dya = rec.dift + ra + msp;   // ey_j[a] = e^{-t1 (dya - a)^2} on a in [ra, ra + 2 msp]
+        const int ra = rec.ntn - R - mm0, ca = rec.nsn - R - nn0;   // window origin in the patch, in [0, 16)
+        const int rlo = row_min(valid ? ra : 1 << 20), rhi = taps - 1 - row_min(valid ? -ra : 1 << 20);
+        const int clo = row_min(valid ? ca : 1 << 20), chi = taps - 1 - row_min(valid ? -ca : 1 << 20);
+        const double dxc = rec.difs + ca + R;   // ex_j[c] = e^{-t1 (dxc - c)^2} on c in [ca, ca + 2 R]
+        const double dya = rec.dift + ra + R;   // ey_j[a] = e^{-t1 (dya - a)^2} on a in [ra, ra + 2 R]
+        // columns cs .. cs + 4 steps - 1 cover clo .. chi and end inside the patch; where they begin before it
+        // (W not a multiple of 4), the entries before column 0 are column 0's and weigh nothing
+        const int steps = (chi - clo + 4) / 4, cs = min(clo, W - 4 * steps);
+        const double dc = dxc - (double)(cs + kq), da = dya - (double)(rlo + kq);
+        const double ev0 = exp(-p.t1 * (dc * dc)), rho0 = exp(8.0 * p.t1 * dc - 16.0 * p.t1);
+        double ey = exp(-p.t1 * (da * da)), sig = exp(8.0 * p.t1 * da - 16.0 * p.t1);
         double sr = 0.0, si = 0.0;
         for (int a0 = rlo; a0 <= rhi; a0 += 16) {
             d4 hr = {0.0, 0.0, 0.0, 0.0}, hi = {0.0, 0.0, 0.0, 0.0};
-            const int arow = a0 + jo;
-            double dc = dxc - (double)(clo + kq);
-            double ev = exp(-p.t1 * (dc * dc)), rho = exp(8.0 * p.t1 * dc - 16.0 * p.t1);
-            for (int c0 = clo; c0 <= chi; c0 += 4) {
-                const int c = c0 + kq;
-                const double bv = valid && c >= ca && c < ca + taps ? ev : 0.0;
-                const double2 av = arow < W && c < W ? P[c * W + arow] : make_double2(0.0, 0.0);
+            const double2 *col = P + min(a0 + jo, W - 1);             // rows past W: never weighted
+            double ev = ev0, rho = rho0;
+            int c = cs + kq;
+            col += max(c, 0) * W;
+            auto step = [&](const double2 av) {
+                const double bv = !MASK || (c >= ca && c < ca + taps) ? ev : 0.0;
                 hr = __builtin_amdgcn_mfma_f64_16x16x4f64(av.x, bv, hr, 0, 0, 0);
                 hi = __builtin_amdgcn_mfma_f64_16x16x4f64(av.y, bv, hi, 0, 0, 0);
+                c += 4;
                 ev *= rho;
                 rho *= kappa;
+            };
+            step(*col);
+            col = P + min(a0 + jo, W - 1) + c * W;                    // c >= 0 from the second step on
+#pragma unroll 4
+            for (int k = 1; k < steps; ++k) {
+                step(*col);
+                col += 4 * W;
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int a = a0 + 4 * q + kq;
-                if (a >= ra && a < ra + taps) {
-                    const double da = dya - (double)a;
-                    const double ey = exp(-p.t1 * (da * da));
-                    sr = fma(ey, hr[q], sr);
-                    si = fma(ey, hi[q], si);
-                }
+                const double wy = a >= ra && a < ra + taps ? ey : 0.0;
+                sr = fma(wy, hr[q], sr);
+                si = fma(wy, hi[q], si);
+                ey *= sig;
+                sig *= kappa;
             }
         }
         sr += __shfl_xor(sr, 16, 64);
         si += __shfl_xor(si, 16, 64);
         sr += __shfl_xor(sr, 32, 64);
         si += __shfl_xor(si, 32, 64);
-        if (kq == 0 && valid) {
-            const double a1 = p.Dy * rec.td, a2 = p.Dx * rec.sd;
-            const double temp = exp(p.b * (a1 * a1 + a2 * a2));
-            const double arg = rec.sd * p.xb + rec.td * p.yb;
-            double sn, cs;
-            sincos(arg, &sn, &cs);
-            F[rec.idx] = make_double2((sr * cs + si * sn) * temp, (si * cs - sr * sn) * temp);
-        }
+        if (kq == 0 && valid)
+            F[rec.idx] = make_double2(sr * rec.pr + si * rec.pi, si * rec.pr - sr * rec.pi);
     }
 }
 
@@ -737,12 +729,56 @@ void derive(const double *ext, double eps, double *out)
 }
 #pragma clang fp contract(on)
 
+// Cells that the coordinates between mn and mx fall into, first and count,
+// inside a side of M.  cell(v) must be k3_prep's own operations: each is
+// monotone in v, rounding included, so the extremes' cells bound all others.
+#pragma clang fp contract(off)
+template <typename Cell>
+void cell_range(double mn, double mx, int M, Cell cell, int &first, int &count)
+{
+    const double lo = std::min(std::max(cell(mn), 0.0), M - 1.0), hi = std::min(std::max(cell(mx), lo), M - 1.0);
+    first = (int)lo;
+    count = (int)hi - (int)lo + 1;
+}
+void in_cells(double mn, double mx, double kk, double base, double D, int M, int &first, int &count)
+{
+    auto cell = [&](double v) {
+        const double u = v / kk;
+        const double o = (u - base) / D;
+        return std::floor((double)(M / 2) + o);
+    };
+    cell_range(mn, mx, M, cell, first, count);
+}
+void out_cells(double mn, double mx, double kk, double base, int M, int &first, int &count)
+{
+    auto cell = [&](double v) {
+        const double u = v * kk;
+        const double o = u - base;
+        return std::floor((double)(M / 2) + o);
+    };
+    cell_range(mn, mx, M, cell, first, count);
+}
+#pragma clang fp contract(on)
+
+// Taps per side that change a sum: at distance d a Gaussian factor is
+// e^{-t1 d^2} of its point's largest, below 2^-58 beyond d = sqrt(58 ln 2 / t1),
+// where msp (the reference's, chosen for eps at the grid's band edge) goes on:
+// msp 19 -> 16, 27 -> 19, 34 -> 22.  Each side's work falls with the square of
+// (2 R + 16).
+int tap_reach(int msp, double t1)
+{
+    const double d = std::ceil(std::sqrt(58.0 * 0.69314718055994531 / t1));
+    return d < msp ? (int)d : msp;
+}
+
 struct Workspace {
     unsigned char *ptr = nullptr;
     size_t size = 0;
 };
 std::mutex g_mu;
 std::map<int, Workspace> g_ws;
+double *g_ext = nullptr;   // pinned: the nine extents of the running call and its number (under g_mu)
+double g_call = 0.0;
 
 int ensure(Workspace &ws, size_t bytes)
 {
@@ -789,27 +825,72 @@ int check_args(const void *x, const void *y, const void *s, const void *t, const
     return NFFT2D_OK;
 }
 
-// Extents on the device, parameters on the host; out[14] as orc_nufft3_params.
+// Extents on the device, parameters on the host; ext[9] as k3_extent_final
+// leaves them, out[14] as orc_nufft3_params.
 int params(Workspace &ws, const double *x, const double *y, const double *s, const double *t, double eps,
-           int len_in, int len_out, double *out)
+           int len_in, int len_out, double *ext, double *out)
 {
     const int L = std::max(len_in, len_out);
     const int nblk = std::max(1, std::min(kExtentBlocks, (L + 255) / 256));
-    int rc = ensure(ws, al(sizeof(double) * 9 * (kExtentBlocks + 1)));
+    int rc = ensure(ws, al(sizeof(double) * 9 * kExtentBlocks));
     if (rc) return rc;
-    double *part = reinterpret_cast<double *>(ws.ptr), *fin = part + 9 * kExtentBlocks;
+    if (!g_ext && hipHostMalloc((void **)&g_ext, sizeof(double) * 10, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        g_ext = nullptr;
+        return nfft2d_fail(NFFT2D_ERR_ALLOC, "type-3: pinned buffer of the extents");
+    }
+    if (g_call == 0.0) g_ext[9] = 0.0;
+    g_call += 1.0;
+    double *part = reinterpret_cast<double *>(ws.ptr), *fin = nullptr;
+    NFFT2D_HIP_TRY(hipHostGetDevicePointer((void **)&fin, g_ext, 0));
     hipLaunchKernelGGL(k3_extent, dim3(nblk), dim3(256), 0, nullptr, x, y, s, t, len_in, len_out, part);
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k3_extent_final, dim3(1), dim3(64), 0, nullptr, part, nblk, fin);
+    hipLaunchKernelGGL(k3_extent_final, dim3(1), dim3(64 * 9), 0, nullptr, part, nblk, g_call, fin);
     NFFT2D_LAUNCH_CHECK();
-    double ext[9];
-    NFFT2D_HIP_TRY(hipMemcpy(ext, fin, sizeof(ext), hipMemcpyDeviceToHost));
+    // poll for at most a millisecond (longer work ahead on the stream, or an error, goes to the runtime)
+    const auto t0 = std::chrono::steady_clock::now();
+    while (__atomic_load_n(reinterpret_cast<const unsigned long long *>(g_ext + 9), __ATOMIC_ACQUIRE) !=
+           __builtin_bit_cast(unsigned long long, g_call)) {
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) {
+            NFFT2D_HIP_TRY(hipStreamSynchronize(nullptr));
+            break;
+        }
+    }
+    for (int q = 0; q < 9; ++q) ext[q] = g_ext[q];
     if (ext[8] != 0.0) return nfft2d_fail(NFFT2D_ERR_ARG, "a coordinate is not finite");
     if (!(ext[0] > ext[1]) || !(ext[2] > ext[3]))
         return nfft2d_fail(NFFT2D_ERR_ARG,
                            "the inputs span no extent in x or y (all equal): the type-3 scaling divides by it");
     derive(ext, eps, out);
     return NFFT2D_OK;
+}
+
+template <int LOGM>
+int kernel_fft(int m, const AxisTables &tx, const AxisTables &ty, hipStream_t st)
+{
+    if (m == 1 << LOGM) {
+        constexpr int bytes = (int)sizeof(double2) * nfft2d::lds_line<1 << LOGM>();
+        NFFT2D_HIP_TRY(hipFuncSetAttribute((const void *)k3_kernel_fft<LOGM>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, bytes));
+        hipLaunchKernelGGL(k3_kernel_fft<LOGM>, dim3(2), dim3(m / 8), bytes, st, tx, ty);
+        NFFT2D_LAUNCH_CHECK();
+        return NFFT2D_OK;
+    }
+    if constexpr (LOGM < nfft2d::kCztMaxLog<double>) return kernel_fft<LOGM + 1>(m, tx, ty, st);
+    return nfft2d_fail(NFFT2D_ERR_SIZE, "no chirp-z transform of %d points", m);
+}
+
+nfft2d::CztTables<double> lines_of(const AxisTables &t)
+{
+    nfft2d::CztTables<double> c;
+    c.cin = t.cin;
+    c.cout = t.cout;
+    c.hhat = t.hhat;
+    c.tw = t.tw;
+    c.P = t.P;
+    c.Q = t.Q;
+    c.m = t.m;
+    return c;
 }
 
 int run(const double *x, const double *y, const double *s, const double *t, const nfft2d_c128 *f,
@@ -826,8 +907,8 @@ int run(const double *x, const double *y, const double *s, const double *t, cons
     int dev = 0;
     NFFT2D_HIP_TRY(hipGetDevice(&dev));
     Workspace &ws = g_ws[dev];
-    double pv[14];
-    if ((rc = params(ws, x, y, s, t, eps, len_in, len_out, pv))) return rc;
+    double ext[9], pv[14];
+    if ((rc = params(ws, x, y, s, t, eps, len_in, len_out, ext, pv))) return rc;
     if (!(pv[12] <= kMaxFft && pv[13] <= kMaxFft))
         return nfft2d_fail(NFFT2D_ERR_SIZE,
                            "grid %.0f x %.0f (Mrx x Mry): at most 4096 (8192 for powers of two) per side; reduce the "
@@ -836,119 +917,123 @@ int run(const double *x, const double *y, const double *s, const double *t, cons
     Par p;
     p.xb = pv[0]; p.yb = pv[1]; p.sb = pv[2]; p.tb = pv[3]; p.kkx = pv[4]; p.kky = pv[5];
     p.Dx = pv[6]; p.Dy = pv[7]; p.b = pv[8]; p.t1 = pv[9]; p.fact = pv[10];
-    p.msp = (int)pv[11]; p.Mrx = (int)pv[12]; p.Mry = (int)pv[13];
-    if (p.msp < 0 || p.msp > kMaxMsp)
-        return nfft2d_fail(NFFT2D_ERR_SIZE, "eps = %g gives %d taps per side; at most %d (eps >= ~1e-14)", eps, p.msp,
+    p.Mrx = (int)pv[12]; p.Mry = (int)pv[13];
+    const int msp = (int)pv[11];
+    if (msp < 0 || msp > kMaxMsp)
+        return nfft2d_fail(NFFT2D_ERR_SIZE, "eps = %g gives %d taps per side; at most %d (eps >= ~1e-14)", eps, msp,
                            kMaxMsp);
-    const int mx = fft_len(p.Mrx), my = fft_len(p.Mry);
-    if (mx > kMaxFft || my > kMaxFft)
+    p.reach = tap_reach(msp, p.t1);
+    const bool mask = !(p.t1 * p.reach * p.reach > 54.0 * 0.69314718055994531);   // tails of 2^-54 and more
+    if (fft_len(p.Mrx) > kMaxFft || fft_len(p.Mry) > kMaxFft)
         return nfft2d_fail(NFFT2D_ERR_SIZE,
                            "grid %d x %d (Mrx x Mry) needs FFTs of %d and %d points; at most %d (Mrx, Mry <= 4096, "
                            "or 8192 for powers of two): reduce the products of the extents X1 S and Y1 T",
-                           p.Mrx, p.Mry, mx, my, kMaxFft);
-    p.nbx = (p.Mrx + kTile - 1) / kTile;
-    p.nby = (p.Mry + kTile - 1) / kTile;
-    p.ibx = (p.Mrx + kInBin - 1) / kInBin;
-    p.iby = (p.Mry + kInBin - 1) / kInBin;
-    const int nb = p.nbx * p.nby;       // tiles / output bins
-    const int nki = p.ibx * p.iby;      // input keys: 8 x 8-cell bins
-    const int nko = nb * kTile;         // output keys: bin and the row inside it
-    const size_t cells = (size_t)p.Mrx * p.Mry;
+                           p.Mrx, p.Mry, fft_len(p.Mrx), fft_len(p.Mry), kMaxFft);
+    // the reached part of the grid and the read part of the spectrum
+    in_cells(ext[1], ext[0], p.kkx, p.xb, p.Dx, p.Mrx, p.ci, p.ni);
+    in_cells(ext[3], ext[2], p.kky, p.yb, p.Dy, p.Mry, p.cj, p.nj);
+    out_cells(ext[5], ext[4], p.kkx, p.sb, p.Mrx, p.oi, p.mi);
+    out_cells(ext[7], ext[6], p.kky, p.tb, p.Mry, p.oj, p.mj);
+    p.gi = std::max(0, p.ci - p.reach);
+    p.gj = std::max(0, p.cj - p.reach);
+    p.Px = std::min(p.Mrx, p.ci + p.ni + p.reach) - p.gi;
+    p.Py = std::min(p.Mry, p.cj + p.nj + p.reach) - p.gj;
+    p.qi = p.oi - p.reach - p.Mrx / 2;
+    p.qj = p.oj - p.reach - p.Mry / 2;
+    p.Qx = std::min(p.mi + 2 * p.reach, p.Mrx);
+    p.Qy = std::min(p.mj + 2 * p.reach, p.Mry);
+    const int mx = std::max(1 << nfft2d::kCztMinLog, next_pow2(p.Px + p.Qx - 1));
+    const int my = std::max(1 << nfft2d::kCztMinLog, next_pow2(p.Py + p.Qy - 1));
+    if (mx > kMaxFft || my > kMaxFft)   // only coordinates rounded far off their cells (huge offsets) get here
+        return nfft2d_fail(NFFT2D_ERR_SIZE, "grid %d x %d (Mrx x Mry): the inputs reach %d x %d cells", p.Mrx, p.Mry,
+                           p.Px, p.Py);
+    p.nbx = (p.mi + kTile - 1) / kTile;
+    p.nby = (p.mj + kTile - 1) / kTile;
+    p.ibx = (p.ni + kInBin - 1) / kInBin;
+    p.iby = (p.nj + kInBin - 1) / kInBin;
+    const int nbo = p.nbx * p.nby;                              // output bins
+    const int nki = p.ibx * p.iby + 1, nko = nbo * kTile + 1;   // keys, the out-of-grid ones last
+    ScanSide a, b;
+    a.n = nki;
+    b.n = nko;
+    a.segs = (nki + 1023) / 1024;
+    b.segs = (nko + 1023) / 1024;
 
-    // workspace: counts, starts, records, the grid and its transpose, FFT tables
+    // workspace: counts, starts, records, the grid parts, the chirp-z tables
+    const size_t cells = (size_t)p.Px * p.Py, mixed = (size_t)p.Qx * p.Py, spec = (size_t)p.Qx * p.Qy;
     size_t need = 0;
     {
-        const size_t sz[] = {al(sizeof(int) * (nki + 2)) * 2 + al(sizeof(int) * (nko + 2)) * 2,
-                             al(sizeof(int) * ((nki + 1) / 1024 + 2)) + al(sizeof(int) * ((nko + 1) / 1024 + 2)),
-                             al(sizeof(InRec) * len_in) * 2, al(sizeof(int2) * len_in) * 2,
+        const size_t sz[] = {(al(sizeof(int) * nki) + al(sizeof(int) * nko)) * 2,
+                             al(sizeof(int) * a.segs) + al(sizeof(int) * b.segs),
+                             al(sizeof(InRec) * len_in) * 2, al(sizeof(int2) * len_in),
                              al(sizeof(OutRec) * len_out) * 2, al(sizeof(int2) * len_out),
-                             al(sizeof(double2) * cells) * 2,
-                             al(sizeof(double2) * mx) * 2 + al(sizeof(double2) * p.Mrx),
-                             al(sizeof(double2) * my) * 2 + al(sizeof(double2) * p.Mry)};
+                             al(sizeof(double2) * cells) + al(sizeof(double2) * mixed) + al(sizeof(double2) * spec),
+                             al(sizeof(double2) * mx) * 2 + al(sizeof(double2) * p.Px) + al(sizeof(double2) * p.Qx),
+                             al(sizeof(double2) * my) * 2 + al(sizeof(double2) * p.Py) + al(sizeof(double2) * p.Qy)};
         for (size_t v : sz) need += v;
     }
     if ((rc = ensure(ws, need))) return rc;
     Carve cv{ws.ptr};
-    int *cnt_in = cv.take<int>(nki + 2), *cnt_out = cv.take<int>(nko + 2);
-    int *st_in = cv.take<int>(nki + 2), *st_out = cv.take<int>(nko + 2);
-    int *tot_in = cv.take<int>((nki + 1) / 1024 + 2), *tot_out = cv.take<int>((nko + 1) / 1024 + 2);
+    a.cnt = cv.take<int>(nki);
+    b.cnt = cv.take<int>(nko);
+    a.start = cv.take<int>(nki);
+    b.start = cv.take<int>(nko);
+    a.tot = cv.take<int>(a.segs);
+    b.tot = cv.take<int>(b.segs);
     InRec *rin = cv.take<InRec>(len_in), *sin_ = cv.take<InRec>(len_in);
-    int2 *kin = cv.take<int2>(len_in), *cin = cv.take<int2>(len_in);
+    int2 *kin = cv.take<int2>(len_in);
     OutRec *rout = cv.take<OutRec>(len_out), *sout = cv.take<OutRec>(len_out);
     int2 *kout = cv.take<int2>(len_out);
-    double2 *G = cv.take<double2>(cells), *GT = cv.take<double2>(cells);
-    double2 *twx = cv.take<double2>(mx), *bhx = cv.take<double2>(mx), *chx = cv.take<double2>(p.Mrx);
-    double2 *twy = cv.take<double2>(my), *bhy = cv.take<double2>(my), *chy = cv.take<double2>(p.Mry);
+    double2 *G = cv.take<double2>(cells), *T = cv.take<double2>(mixed), *S = cv.take<double2>(spec);
+    auto axis = [&](int n, int P, int Q, int p0, int q0, int m) {
+        AxisTables t;
+        t.cin = cv.take<double2>(P);
+        t.cout = cv.take<double2>(Q);
+        t.hhat = cv.take<double2>(m);
+        t.tw = cv.take<double2>(m);
+        t.n = n; t.P = P; t.Q = Q; t.p0 = p0; t.q0 = q0; t.m = m;
+        return t;
+    };
+    const AxisTables tx = axis(p.Mrx, p.Px, p.Qx, p.gi, p.qi, mx), ty = axis(p.Mry, p.Py, p.Qy, p.gj, p.qj, my);
 
     hipStream_t st = nullptr;
-    NFFT2D_HIP_TRY(hipMemsetAsync(cnt_in, 0, al(sizeof(int) * (nki + 2)) + al(sizeof(int) * (nko + 2)), st));
-    const unsigned gin = (unsigned)((len_in + 255) / 256), gout = (unsigned)((len_out + 255) / 256);
-    hipLaunchKernelGGL(k3_prep_in, dim3(gin), dim3(256), 0, st, x, y, reinterpret_cast<const double2 *>(f), len_in,
-                       p, rin, kin, cnt_in);
+    NFFT2D_HIP_TRY(hipMemsetAsync(a.cnt, 0, al(sizeof(int) * nki) + al(sizeof(int) * nko), st));
+    const int gin = (len_in + 255) / 256, gout = (len_out + 255) / 256;
+    hipLaunchKernelGGL(k3_prep, dim3(gin + gout), dim3(256), 0, st, x, y, reinterpret_cast<const double2 *>(f), len_in,
+                       gin, p, rin, kin, a.cnt, s, t, len_out, rout, kout, b.cnt, reinterpret_cast<double2 *>(F));
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k3_prep_out, dim3(gout), dim3(256), 0, st, s, t, len_out, p, rout, kout, cnt_out,
-                       reinterpret_cast<double2 *>(F));
+    hipLaunchKernelGGL(k3_scan_local, dim3(a.segs + b.segs + (std::max(mx, my) + 1023) / 1024), dim3(1024), 0, st, a, b,
+                       tx, ty);
     NFFT2D_LAUNCH_CHECK();
-    // keys: nki bins (+ 1 out-of-grid) for the inputs, nko bin rows (+ 1) for the outputs
-    for (int side = 0; side < 2; ++side) {
-        const int n = (side ? nko : nki) + 1, segs = (n + 1023) / 1024;
-        int *cnt = side ? cnt_out : cnt_in, *start = side ? st_out : st_in, *tot = side ? tot_out : tot_in;
-        hipLaunchKernelGGL(k3_scan_local, dim3(segs), dim3(1024), 0, st, cnt, n, start, tot);
-        NFFT2D_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k3_scan_totals, dim3(1), dim3(1024), 0, st, tot, segs);
-        NFFT2D_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k3_scan_add, dim3(n / 256 + 1), dim3(256), 0, st, start, n, tot);
-        NFFT2D_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(k3_scatter_in, dim3(gin), dim3(256), 0, st, rin, kin, len_in, st_in, sin_, cin);
+    hipLaunchKernelGGL(k3_scan_totals, dim3(2), dim3(1024), 0, st, a, b);
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k3_scatter<OutRec>, dim3(gout), dim3(256), 0, st, rout, kout, len_out, st_out, sout);
+    if ((rc = kernel_fft<nfft2d::kCztMinLog>(mx, tx, ty, st))) return rc;
+    if (my != mx && (rc = kernel_fft<nfft2d::kCztMinLog>(my, tx, ty, st))) return rc;
+    hipLaunchKernelGGL(k3_scatter, dim3(gin + gout), dim3(256), 0, st, rin, kin, len_in, gin, a, sin_, rout, kout,
+                       len_out, b, sout);
     NFFT2D_LAUNCH_CHECK();
-
-    // FFT tables (twiddles; chirps and their transforms for Bluestein lines)
-    auto tables = [&](int n, int m, double2 *tw, double2 *ch, double2 *bh) -> int {
-        hipLaunchKernelGGL(k3_twiddles, dim3((m + 255) / 256), dim3(256), 0, st, m, tw);
-        NFFT2D_LAUNCH_CHECK();
-        if (is_pow2(n)) return NFFT2D_OK;
-        hipLaunchKernelGGL(k3_chirp, dim3((m + 255) / 256), dim3(256), 0, st, n, m, ch, bh);
-        NFFT2D_LAUNCH_CHECK();
-        const int T = std::min(1024, std::max(64, m / 4));
-        hipLaunchKernelGGL(k3_fft_lines, dim3(1), dim3(T), sizeof(double2) * fft_lds_entries(m), st, bh, m, m, tw,
-                           (const double2 *)nullptr, (const double2 *)nullptr);
-        NFFT2D_LAUNCH_CHECK();
-        return NFFT2D_OK;
-    };
-    NFFT2D_HIP_TRY(hipFuncSetAttribute((const void *)k3_fft_lines, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)sizeof(double2) * fft_lds_entries(kMaxFft)));
-    if ((rc = tables(p.Mrx, mx, twx, chx, bhx))) return rc;
-    if ((rc = tables(p.Mry, my, twy, chy, bhy))) return rc;
 
     // spread
-    hipLaunchKernelGGL(k3_spread, dim3(nb), dim3(64 * kSpreadWaves), 0, st, sin_, cin, st_in, p, G);
+    const int ntx = (p.Px + kTile - 1) / kTile, nty = (p.Py + kTile - 1) / kTile;
+    hipLaunchKernelGGL((mask ? k3_spread<true> : k3_spread<false>), dim3(ntx * nty),
+                       dim3(64 * kSpreadWaves), 0, st, sin_, a.start, a.tot, p, ntx, G);
     NFFT2D_LAUNCH_CHECK();
 
-    // 2-D DFT: rows (length Mrx), transpose, rows of the transpose (length Mry)
-    auto lines = [&](double2 *data, int n, int m, int count, const double2 *tw, const double2 *ch,
-                     const double2 *bh) -> int {
-        const int T = std::min(1024, std::max(64, m / 4));
-        const bool blue = !is_pow2(n);
-        hipLaunchKernelGGL(k3_fft_lines, dim3(count), dim3(T), sizeof(double2) * fft_lds_entries(m), st, data, n, m,
-                           tw,
-                           blue ? ch : (const double2 *)nullptr, blue ? bh : (const double2 *)nullptr);
-        NFFT2D_LAUNCH_CHECK();
-        return NFFT2D_OK;
-    };
-    if ((rc = lines(G, p.Mrx, mx, p.Mry, twx, chx, bhx))) return rc;
-    hipLaunchKernelGGL(k3_transpose, dim3((p.Mrx + 31) / 32, (p.Mry + 31) / 32), dim3(256), 0, st, G, GT, p.Mry,
-                       p.Mrx);
-    NFFT2D_LAUNCH_CHECK();
-    if ((rc = lines(GT, p.Mry, my, p.Mrx, twy, chy, bhy))) return rc;
+    // 2-D DFT: G's rows (j) to the read x frequencies, written side by side: T[qi][j]; then T's rows: S[qi][qj]
+    const double *none = nullptr;
+    if ((rc = nfft2d::czt_launch<double, 2>(lines_of(tx), p.Py, (const double2 *)G, p.Px, 1, T, 1, p.Py, none, none,
+                                            false, false, st)))
+        return rc;
+    if ((rc = nfft2d::czt_launch<double, 0>(lines_of(ty), p.Qx, (const double2 *)T, p.Py, 1, S, p.Qy, 1, none, none,
+                                            false, false, st)))
+        return rc;
 
     // interpolation at the outputs
-    const int W = kTile + 2 * p.msp;
+    const int W = kTile + 2 * p.reach;
     const size_t lds = sizeof(double2) * (size_t)W * W;
-    NFFT2D_HIP_TRY(hipFuncSetAttribute((const void *)k3_interp, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k3_interp, dim3(nb), dim3(64 * kInterpWaves), lds, st, GT, sout, st_out, p,
+    auto interp = mask ? k3_interp<true> : k3_interp<false>;
+    NFFT2D_HIP_TRY(hipFuncSetAttribute((const void *)interp, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(interp, dim3(nbo), dim3(64 * kInterpWaves), lds, st, S, sout, b.start, b.tot, p,
                        reinterpret_cast<double2 *>(F));
     NFFT2D_LAUNCH_CHECK();
     return NFFT2D_OK;
@@ -972,7 +1057,8 @@ extern "C" int NUFFT_2D_GPU_params(const double *x, const double *y, const doubl
     std::lock_guard<std::mutex> lk(g_mu);
     int dev = 0;
     NFFT2D_HIP_TRY(hipGetDevice(&dev));
-    return params(g_ws[dev], x, y, s, t, eps, len_in, len_out, out);
+    double ext[9];
+    return params(g_ws[dev], x, y, s, t, eps, len_in, len_out, ext, out);
 }
 
 extern "C" int NUFFT_2D_GPU_host(const double *x, const double *y, const double *s, const double *t,
