@@ -87,8 +87,9 @@ int NFFT1_2D_GPU_c128(nfft2d_c128 *result, const nfft2d_c128 *data, const double
 /* NFFT2_2D_GPU_c64 that allocates nothing: no counterpart in the reference.
  * For callers that cannot allocate device memory (code under hipGraph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments and
- * result as NFFT2_2D_GPU_c64 (the same kernels), plus the
- * stream the work is ordered on (NULL: the legacy default stream).  Every
+ * result as NFFT2_2D_GPU_c64 (to FP32 rounding: it always sorts and spreads,
+ * where NFFT2_2D_GPU_c64 sums small transforms directly), plus the stream the
+ * work is ordered on (NULL: the legacy default stream).  Every
  * buffer of the transform lives in one file-scope device array of 22 MiB that
  * each GPU the library runs on holds until the process ends; hence the limits
  * N1, N2 <= 256 (even) and M <= 262144, NFFT2D_ERR_SIZE beyond them.  All
@@ -339,7 +340,10 @@ int nfft2d_batch_get_gather_blocks(const nfft2d_batch *batch);
  *                  spread tiles; N1, N2 >= 22 (NFFT2D_ERR_SIZE otherwise);
  *   type1          4 launches (spread, tile merge, the two FFT passes with
  *                  crop and deconvolution), needs setpts;
- *   setpts_type1   setpts then type1 on `stream` (9 launches). */
+ *   setpts_type1   setpts then type1 on `stream` (9 launches); batches of
+ *                  equal, small transforms: setpts, then direct sums of the
+ *                  caller's points on the matrix cores (1 or 2 launches),
+ *                  within FP32 rounding of type1. */
 int nfft2d_batch_set_io_type1(nfft2d_batch *batch, const nfft2d_c64 *const *data, nfft2d_c64 *const *result);
 int nfft2d_batch_type1(nfft2d_batch *batch, void *stream);
 int nfft2d_batch_setpts_type1(nfft2d_batch *batch, void *stream);

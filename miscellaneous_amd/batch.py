@@ -120,7 +120,7 @@ class Batch:
             check(self._lib.nfft2d_batch_type1(self._h, _stream(self.device)), "nfft2d_batch_type1")
 
     def setpts_type1(self) -> None:
-        """setpts() then type1() (9 launches in all)."""
+        """setpts() then type1() (9 launches in all); equal, small transforms as direct sums (6 or 7)."""
         with torch.cuda.device(self.device):
             check(self._lib.nfft2d_batch_setpts_type1(self._h, _stream(self.device)), "nfft2d_batch_setpts_type1")
 

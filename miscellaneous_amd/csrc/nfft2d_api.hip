@@ -22,6 +22,7 @@
 #include "nfft2d_kernels.hpp"
 #include "nfft1d_kernels.hpp"
 #include "nfft2d_czt.hpp"
+#include "nfft2d_t1sum.hpp"
 
 using namespace nfft2d;
 
@@ -1083,6 +1084,56 @@ int cached_plan(int N1, int N2, int dtype, nfft2d_plan **out)
     return NFFT2D_OK;
 }
 
+// The most products of 16 points that one FP32 sum may take, so that the direct
+// sum's error stays below the NFFT's.  Measured rel-L2: direct sum after n
+// products 1e-7 sqrt(2.0 + 0.19 n) (1.5e-7 after 3, 2.7e-7 after 30, 4.1e-7
+// after 78); type-1 passes as matrix-core DFTs 1e-7 sqrt(3.9 + 0.065 (N1 + N2))
+// (2.6e-7 at 22 x 22, 3.9e-7 at 88 x 88, 4.5e-7 at 126 x 126), FFT and chirp-z
+// passes from 2.2e-7.
+int t1_sum_chain(int N1, int N2)
+{
+    auto mm = [](int N) { return N <= kT1MmMaxN && (N & (N - 1)) != 0; };
+    return mm(N1) && mm(N2) ? (int)(9.0 + 0.315 * (N1 + N2)) : 16;
+}
+
+// Time of a batch's spread, merge and FFT passes, us (fitted to batches of 20 to
+// 250: 88 x 88 from 1,936 points 383 us for 250, 22 x 126 from 2,500 173,
+// 22 x 22 from 4,096 80, 64 x 64 from 1,500 179, 12 of 130 x 88 from 2,500 66;
+// at least four launches).
+double t1_passes_us(int N1, int N2, int M, int count)
+{
+    const bool fft = (N1 & (N1 - 1)) == 0 || (N2 & (N2 - 1)) == 0;
+    return std::max(30.0, (fft ? 0.8 : 1.0) * (25.0 + count * (0.03 + 3.5e-5 * M + 1.9e-4 * N1 * N2)));
+}
+
+// complex64 type-1 as a direct sum (k_t1_sum) instead of sort, spread and FFT passes.
+bool t1_sum_better(int N1, int N2, int M)
+{
+    return M > 0 && M <= kT1SumOnePoints && N1 <= kT1SumMaxN && N2 <= kT1SumMaxN && (double)N1 * N2 * M <= kT1SumOneWork;
+}
+
+// The partial sums go to the plan's spread scratch, so the result array is
+// written after every input was read, whatever the caller's arrays overlap.
+int dropin_t1_sum(nfft2d_plan *p, void *result, const void *data, const void *x, const void *y, int M)
+{
+    T1SumPlan q = t1_sum_plan(p->N1, p->N2, M, 1, 16);   // kT1SumOnePoints / 12 ranges / 32: always has a split
+    const long long need = ((long long)q.a.S * p->N1 * p->N2 + kTileCells - 1) / kTileCells;
+    if (need > p->scratchcap) {
+        free_scratch(p);
+        if (nfft2d_malloc(&p->scratch, sizeof(float2) * kTileCells * (size_t)need) != hipSuccess)
+            return nfft2d_fail(NFFT2D_ERR_ALLOC, "type-1: hipMalloc of %d partial sums failed", q.a.S);
+        p->scratchcap = (int)need;
+    }
+    q.a.x = (const float *)x;
+    q.a.y = (const float *)y;
+    q.a.d = (const float2 *)data;
+    q.a.F = (float2 *)result;
+    q.a.part = (float2 *)p->scratch;
+    t1_sum_launch(q, 1, nullptr);
+    NFFT2D_LAUNCH_CHECK();
+    return NFFT2D_OK;
+}
+
 int dropin(int dtype, bool type2, void *result, const void *data, const void *x, const void *y, int N1, int N2, int M)
 {
     if (M < 0) return nfft2d_fail(NFFT2D_ERR_ARG, "M < 0");
@@ -1093,6 +1144,7 @@ int dropin(int dtype, bool type2, void *result, const void *data, const void *x,
     int rc = cached_plan(N1, N2, dtype, &p);
     if (rc) return rc;
     if (type2) return nfft2d_setpts_type2(p, result, data, x, y, M, nullptr);
+    if (dtype == NFFT2D_C64 && t1_sum_better(N1, N2, M)) return dropin_t1_sum(p, result, data, x, y, M);
     if ((rc = nfft2d_setpts(p, x, y, M, nullptr))) return rc;
     return nfft2d_type1(p, result, data, nullptr);
 }
@@ -1500,6 +1552,8 @@ struct nfft2d_batch_s {
     bool have_points = false, have_io = false, have_io1 = false;
     bool sorted = false;                  // the subproblem list matches the points and sizes (batch_setpts ran)
     Fork fk;                              // setpts beside the grid passes (nfft2d_batch_setpts_type2)
+    bool t1_sum = false;                  // setpts_type1 takes the direct sums (batch_choose_t1_sum)
+    T1SumPlan t1_sum_plan = {};           // its split, for the largest M of the batch
     std::vector<int> dmax;                // per transform: direct-gather cut-off (BatchDesc::dmax)
     int gather_blocks = kBatchGatherWaveBlocks;   // width of the persistent wave gather
 };
@@ -1564,8 +1618,10 @@ static void batch_fill_desc(nfft2d_batch *b, int t)
     d.cztm2 = p->cztm[1];
 }
 
+static void batch_choose_t1_sum(nfft2d_batch *b);
 static int batch_upload(nfft2d_batch *b)
 {
+    batch_choose_t1_sum(b);
     NFFT2D_HIP_TRY(hipMemcpy(b->ddesc, b->hdesc.data(), sizeof(BatchDesc) * b->count, hipMemcpyHostToDevice));
     return NFFT2D_OK;
 }
@@ -1904,9 +1960,59 @@ extern "C" int nfft2d_batch_type1(nfft2d_batch *b, void *stream)
     return NFFT2D_OK;
 }
 
-// setpts then type-1 (the spread needs the sorted points; one stream).
+// The direct sums of a batch of equal sizes write the modes while other blocks
+// still read samples and coordinates: no result may overlap an input.
+static bool batch_results_apart(const nfft2d_batch *b)
+{
+    using R = std::pair<uintptr_t, uintptr_t>;
+    std::vector<R> out;
+    for (const BatchDesc &d : b->hdesc)
+        out.emplace_back((uintptr_t)d.F1, (uintptr_t)d.F1 + sizeof(float2) * d.N1 * d.N2);
+    std::sort(out.begin(), out.end());
+    for (size_t i = 1; i < out.size(); ++i)
+        if (out[i].first < out[i - 1].second) return false;
+    auto hits = [&](const void *p, size_t bytes) {
+        auto it = std::lower_bound(out.begin(), out.end(), R((uintptr_t)p + bytes, 0));   // first result at or past the end
+        return bytes > 0 && it != out.begin() && std::prev(it)->second > (uintptr_t)p;
+    };
+    for (const BatchDesc &d : b->hdesc)
+        if (hits(d.d1, sizeof(float2) * d.M) || hits(d.x, sizeof(float) * d.M) || hits(d.y, sizeof(float) * d.M)) return false;
+    return true;
+}
+
+// Whether setpts_type1 takes the direct sums: equal sizes, faster by the
+// estimates of both sides (with a tenth to spare), results apart from the inputs.
+static void batch_choose_t1_sum(nfft2d_batch *b)
+{
+    b->t1_sum = false;
+    if (!b->have_points || !b->have_io1) return;
+    const BatchDesc &e = b->hdesc[0];
+    int M = 0;
+    for (const BatchDesc &d : b->hdesc) {
+        if (d.N1 != e.N1 || d.N2 != e.N2) return;
+        M = std::max(M, d.M);
+    }
+    if (e.N1 > kT1SumMaxN || e.N2 > kT1SumMaxN || M == 0 || !batch_results_apart(b)) return;
+    b->t1_sum_plan = t1_sum_plan(e.N1, e.N2, M, b->count, t1_sum_chain(e.N1, e.N2));
+    b->t1_sum_plan.a.bd = b->ddesc;
+    b->t1_sum = b->t1_sum_plan.blocks > 0 && 1.1 * b->t1_sum_plan.t < t1_passes_us(e.N1, e.N2, M, b->count);
+}
+
+// setpts, then type-1: small equal transforms as direct sums, which read the
+// caller's arrays (a later type1 or type2 call finds the points sorted, as
+// after any setpts), the others from the sorted points.  One stream: the
+// direct sums leave no LDS for a sort beside them, and the cross-stream waits
+// of an eager call cost more than the sort (165 against 150 us for 250
+// transforms of 88 x 88 modes from 1,936 points).
 extern "C" int nfft2d_batch_setpts_type1(nfft2d_batch *b, void *stream)
 {
+    if (b && b->t1_sum) {
+        const int rc = nfft2d_batch_setpts(b, stream);
+        if (rc) return rc;
+        t1_sum_launch(b->t1_sum_plan, b->count, (hipStream_t)stream);
+        NFFT2D_LAUNCH_CHECK();
+        return NFFT2D_OK;
+    }
     int rc = nfft2d_batch_setpts(b, stream);
     return rc ? rc : nfft2d_batch_type1(b, stream);
 }
