@@ -1609,7 +1609,11 @@ __device__ __forceinline__ void pairs_mac(const Lds& L, int l, const WinArgs& wa
 // pairs_mac for a point (columns c0..c0+13 with the weights shifted for an odd
 // cell, then the 13 rows), so the same bits.  For subproblems of a few points,
 // where a tile, a sort and a wave's sums per subproblem cost more than the
-// 182 cached reads per point.
+// cached reads of the point's window: 91 of 16 bytes (the window's first column
+// and L1 are even, so a pair of columns starts on 16 bytes and does not
+// straddle the wrap).  What binds is the number of scattered load instructions:
+// with 182 of 8 bytes the batch of 256 uneven transforms spent 243 us here, 180
+// with 91.
 __device__ __forceinline__ float2 direct_point(const PtRec<float>& rec, int O1, int O2, const float2* __restrict__ Gt,
                                                const BinGeom& geo, const WinArgs& wa)
 {
@@ -1626,13 +1630,13 @@ __device__ __forceinline__ float2 direct_point(const PtRec<float>& rec, int O1, 
         e[j] = odd ? a1 : a0;
     }
     const bool big = geo.L1 >= kTileW && geo.L2 >= kTileW;
-    int g1[kW + 1];
+    int g1[(kW + 1) / 2];                                    // column pairs: even starts, 16-byte loads
 #pragma unroll
-    for (int j = 0; j <= kW; ++j) {
-        const int o1 = O1 - kK + c0 + j;
+    for (int j = 0; j < (kW + 1) / 2; ++j) {
+        const int o1 = O1 - kK + c0 + 2 * j;
         g1[j] = big ? wrap1(o1, geo.L1) : wrap(o1, geo.L1);
     }
-    // one row (14 loads) in flight at a time; the row weights shift down so
+    // one row (7 loads) in flight at a time; the row weights shift down so
     // that the current one is w2[0] (register arrays take static indices only)
     float x = 0.f, y = 0.f;
 #pragma unroll 1
@@ -1641,10 +1645,12 @@ __device__ __forceinline__ float2 direct_point(const PtRec<float>& rec, int O1, 
         const float2* __restrict__ row = Gt + (size_t)(big ? wrap1(o2, geo.L2) : wrap(o2, geo.L2)) * geo.L1;
         float sx = 0.f, sy = 0.f;
 #pragma unroll
-        for (int j = 0; j <= kW; ++j) {
-            const float2 u = row[g1[j]];
-            sx = fmaf(e[j], u.x, sx);
-            sy = fmaf(e[j], u.y, sy);
+        for (int j = 0; j < (kW + 1) / 2; ++j) {
+            const float4 u = *reinterpret_cast<const float4*>(row + g1[j]);
+            sx = fmaf(e[2 * j], u.x, sx);
+            sy = fmaf(e[2 * j], u.y, sy);
+            sx = fmaf(e[2 * j + 1], u.z, sx);
+            sy = fmaf(e[2 * j + 1], u.w, sy);
         }
         x = fmaf(w2[0], sx, x);
         y = fmaf(w2[0], sy, y);
