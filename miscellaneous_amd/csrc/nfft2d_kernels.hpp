@@ -1935,15 +1935,24 @@ struct SpreadWaveLds {
     unsigned rc[64];               // (15 - r_p) | (15 - c_p) << 16 of the wave's 64 points
 };
 
-__device__ __forceinline__ unsigned pack_h2(_Float16 lo16, _Float16 hi16)
+// Two values x = hi + lo in FP16, rounded to nearest: hi and lo hold the pair's
+// halves.  Two packed conversions and two mixed-precision differences (x - hi
+// is exact).
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef float f2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_h2(float a, float b, unsigned& hi, unsigned& lo)
 {
-    return (unsigned)__builtin_bit_cast(unsigned short, lo16) | ((unsigned)__builtin_bit_cast(unsigned short, hi16) << 16);
+    const h2v h = __builtin_convertvector((f2v){a, b}, h2v);
+    const h2v l = __builtin_convertvector((f2v){fmaf((float)h.x, -1.f, a), fmaf((float)h.y, -1.f, b)}, h2v);
+    hi = __builtin_bit_cast(unsigned, h);
+    lo = __builtin_bit_cast(unsigned, l);
 }
-
-__device__ __forceinline__ void split_h(float x, _Float16& hi, _Float16& lo)
+// One value as {hi, lo}.
+__device__ __forceinline__ unsigned split_h1(float x)
 {
-    hi = (_Float16)x;
-    lo = (_Float16)(x - (float)hi);
+    const float hi = (float)(_Float16)x;
+    const h2v r = __builtin_convertvector((f2v){x, fmaf(hi, -1.f, x)}, h2v);
+    return __builtin_bit_cast(unsigned, r);
 }
 
 // A block spreads up to kSpUnit consecutive subproblems of one bin (up to
@@ -2029,12 +2038,8 @@ __device__ __forceinline__ void spread_halo_body(int s, int4 d, const PtRec<floa
         unsigned bw[kW];
 #pragma unroll
         for (int m = 0; m < kW; ++m) {
-            _Float16 rh, rlo, ih, ilo, bh, blo;
-            split_h(vx * w2[m], rh, rlo);
-            split_h(vy * w2[m], ih, ilo);
-            split_h(w1[m], bh, blo);
-            aw[m] = make_uint2(pack_h2(rh, ih), pack_h2(rlo, ilo));
-            bw[m] = pack_h2(bh, blo);
+            split_h2(vx * w2[m], vy * w2[m], aw[m].x, aw[m].y);
+            bw[m] = split_h1(w1[m]);
         }
         L.rc[lane] = (unsigned)(kSpTap0 - rl) | ((unsigned)(kSpTap0 - cl) << 16);
         wave_sync_lds();

@@ -107,17 +107,7 @@ __device__ __forceinline__ unsigned turn_of(double x, double inv2n, int N)
     return (unsigned)__double2loint(fma(r, inv2n, 1572864.0));
 }
 
-// 4 values (one operand row at 4 points) split into FP16 planes, 8 bytes each:
-// two packed conversions and two mixed-precision differences per pair of values
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef float f2v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split_h2(float a, float b, unsigned& hi, unsigned& lo)
-{
-    const h2v h = __builtin_convertvector((f2v){a, b}, h2v);
-    const h2v l = __builtin_convertvector((f2v){fmaf((float)h.x, -1.f, a), fmaf((float)h.y, -1.f, b)}, h2v);
-    hi = __builtin_bit_cast(unsigned, h);
-    lo = __builtin_bit_cast(unsigned, l);
-}
+// 4 values (one operand row at 4 points) split into FP16 planes, 8 bytes each
 __device__ __forceinline__ void put_split(char* hi, char* lo, float a, float b, float c, float d)
 {
     uint2 h, l;
