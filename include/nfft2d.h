@@ -340,7 +340,7 @@ int nfft2d_batch_get_gather_blocks(const nfft2d_batch *batch);
  *                  spread tiles; N1, N2 >= 22 (NFFT2D_ERR_SIZE otherwise);
  *   type1          4 launches (spread, tile merge, the two FFT passes with
  *                  crop and deconvolution), needs setpts;
- *   setpts_type1   setpts then type1 on `stream` (9 launches); batches of
+ *   setpts_type1   setpts then type1 on `stream`; batches of
  *                  equal, small transforms: setpts, then direct sums of the
  *                  caller's points on the matrix cores (1 or 2 launches),
  *                  within FP32 rounding of type1. */

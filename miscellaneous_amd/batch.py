@@ -4,7 +4,7 @@
 per transform (complex64, K = 6, c = 2; N1, N2 even in [2, 1024]: powers of
 two from 8 run the Stockham passes, other sizes direct ones).  Every stage
 then runs as one kernel launch over all transforms: ``setpts()`` is 5
-launches, ``type2()`` and ``type1()`` 4 each, so they can be captured into one
+launches (2 for batches of transforms of at most 4096 points), ``type2()`` and ``type1()`` 4 each, so they can be captured into one
 graph.  ``type1`` (N1, N2 >= 22) is the reference's NFFT2_2D_GPU for every
 transform, e.g. the far fields of one PSO generation
 (``Synthesis/PSO/PSO.cu:348``, ``Synthesis.cu:395``) in one graph.  Arrays are kept by reference (``set_points`` / ``set_io``): keep
@@ -120,7 +120,7 @@ class Batch:
             check(self._lib.nfft2d_batch_type1(self._h, _stream(self.device)), "nfft2d_batch_type1")
 
     def setpts_type1(self) -> None:
-        """setpts() then type1() (9 launches in all); equal, small transforms as direct sums (6 or 7)."""
+        """setpts() then type1(); equal, small transforms as direct sums (1 or 2 launches after setpts())."""
         with torch.cuda.device(self.device):
             check(self._lib.nfft2d_batch_setpts_type1(self._h, _stream(self.device)), "nfft2d_batch_setpts_type1")
 

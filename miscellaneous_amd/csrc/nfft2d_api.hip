@@ -1552,6 +1552,7 @@ struct nfft2d_batch_s {
     bool have_points = false, have_io = false, have_io1 = false;
     bool sorted = false;                  // the subproblem list matches the points and sizes (batch_setpts ran)
     Fork fk;                              // setpts beside the grid passes (nfft2d_batch_setpts_type2)
+    bool sort_one = false;                // setpts: one block sorts one transform (kb_sort_one)
     bool t1_sum = false;                  // setpts_type1 takes the direct sums (batch_choose_t1_sum)
     T1SumPlan t1_sum_plan = {};           // its split, for the largest M of the batch
     std::vector<int> dmax;                // per transform: direct-gather cut-off (BatchDesc::dmax)
@@ -1647,6 +1648,7 @@ extern "C" int nfft2d_batch_create(nfft2d_batch **out, int count, const int *N1,
     b->plans.assign(count, nullptr);
     b->hdesc.assign(count, BatchDesc{});
     b->dmax.assign(count, kDirectDefault);
+    b->sort_one = count <= kSortOneCount;
     std::vector<int2> own;
     long long subcap = 0;
     for (int t = 0; t < count; ++t) {
@@ -1661,6 +1663,7 @@ extern "C" int nfft2d_batch_create(nfft2d_batch **out, int count, const int *N1,
         b->hdesc[t].M = M[t];
         batch_fill_desc(b, t);
         b->max_nbins = std::max(b->max_nbins, p->nbins);
+        b->sort_one = b->sort_one && M[t] <= kOnePts && p->nbins <= kSmallBins;
         subcap += p->nbins + (M[t] + kBatchMinMaxpts - 1) / kBatchMinMaxpts;
     }
     auto add_stage = [&](int &off, int &n, auto blocks_of) {
@@ -1825,6 +1828,14 @@ extern "C" int nfft2d_batch_setpts(nfft2d_batch *b, void *stream)
     int rc = nfft2d_check_device(b->device);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
+    if (b->sort_one) {
+        hipLaunchKernelGGL(kb_sort_one, dim3(b->count), dim3(kScatThreads), sizeof(int) * 2 * b->max_nbins, s, b->ddesc);
+        NFFT2D_LAUNCH_CHECK();
+        hipLaunchKernelGGL(kb_sub_list, dim3(b->count), dim3(256), 0, s, b->ddesc, b->count, b->base, b->bsub);
+        NFFT2D_LAUNCH_CHECK();
+        b->sorted = true;
+        return NFFT2D_OK;
+    }
     if (b->n_hist > 0)
         hipLaunchKernelGGL(kb_hist, dim3(b->n_hist), dim3(kHistThreads), sizeof(int) * b->max_nbins, s, b->ddesc,
                            b->own + b->off_hist);
@@ -2003,8 +2014,8 @@ static void batch_choose_t1_sum(nfft2d_batch *b)
 // caller's arrays (a later type1 or type2 call finds the points sorted, as
 // after any setpts), the others from the sorted points.  One stream: the
 // direct sums leave no LDS for a sort beside them, and the cross-stream waits
-// of an eager call cost more than the sort (165 against 150 us for 250
-// transforms of 88 x 88 modes from 1,936 points).
+// of an eager call cost more than the sort (165 us on two streams, 143 on one
+// for 250 transforms of 88 x 88 modes from 1,936 points).
 extern "C" int nfft2d_batch_setpts_type1(nfft2d_batch *b, void *stream)
 {
     if (b && b->t1_sum) {

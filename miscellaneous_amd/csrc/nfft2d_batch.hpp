@@ -8,7 +8,7 @@
 // batch is created (the block counts of these stages depend on the sizes
 // only).  The gather is persistent: its blocks walk one list of the
 // subproblems of all transforms, each entry tagged with its transform.
-// Together: 5 launches for setpts, 4 for the type-2 and 4 for the type-1,
+// Together: 5 launches for setpts (2 for batches of small transforms), 4 for the type-2 and 4 for the type-1,
 // whatever the number of transforms, all stream-ordered and free of
 // allocation, so the whole sequence can be captured into one hipGraph.
 #pragma once
@@ -148,6 +148,45 @@ __global__ __launch_bounds__(1024) void kb_sub_prefix(const BatchDesc* __restric
         __syncthreads();
     }
     if (t == 0) base[count] = carry;
+}
+
+// Batches of at most kSortOneCount transforms of at most kOnePts points and
+// kSmallBins bins each: one block sorts one transform (k_scatter_small's
+// single-block form, subproblems into the plan's own list), and a second launch
+// copies the lists into the batch's, each block summing the counts of the
+// transforms before its own.  At these sizes the five launches of the general
+// sort are bound by their fixed costs and dependent loads: 250 transforms of
+// 1,936 points on 88 x 88 modes 22 -> 13 us.
+constexpr int kSortOneCount = 2048;
+__global__ __launch_bounds__(kScatThreads) void kb_sort_one(const BatchDesc* __restrict__ bd)
+{
+    extern __shared__ int small_lds[];
+    const BatchDesc& d = bd[blockIdx.x];
+    scatter_small_body<float, true>(small_lds, d.x, d.y, d.M, max(d.M, 1), d.L1, d.L2, d.inv1, d.inv2, d.nb1, d.nbins,
+                                    d.maxpts, nullptr, d.tot, d.pts, d.subbeg, d.sub, d.nsub);
+}
+__global__ __launch_bounds__(256) void kb_sub_list(const BatchDesc* __restrict__ bd, int count, int* __restrict__ base,
+                                                   int4* __restrict__ bsub)
+{
+    __shared__ int part[4];
+    const int tr = blockIdx.x, t = threadIdx.x;
+    int v = 0;
+    for (int u = t; u < tr; u += 256) v += *bd[u].nsub;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if ((t & 63) == 0) part[t >> 6] = v;
+    __syncthreads();
+    const int at = part[0] + part[1] + part[2] + part[3];
+    const BatchDesc& d = bd[tr];
+    const int n = *d.nsub;
+    if (t == 0) {
+        base[tr] = at;
+        if (tr == count - 1) base[count] = at + n;
+    }
+    for (int i = t; i < n; i += 256) {
+        const int4 e = d.sub[i];
+        bsub[at + i] = make_int4(e.x, e.y, e.z, e.z <= d.dmax ? ~tr : tr);   // tagged as by kb_scatter_lds
+    }
 }
 
 // Scatter of every transform's points, and each transform's subproblems into

@@ -1109,12 +1109,11 @@ __global__ __launch_bounds__(kScatThreads) void k_scatter_lds(
 constexpr int kOnePts = kScatThreads * kScatPer;      // one batch of the block's points, held in registers
 constexpr int kSmallBins = 4096, kSmallHist = 32768;
 template <typename T, bool ONE>
-__global__ __launch_bounds__(kScatThreads) void k_scatter_small(
-    const T* __restrict__ x, const T* __restrict__ y, int M, int chunk, int L1, int L2, T inv1, T inv2, int nb1,
-    int nbins, int maxpts, const int* __restrict__ hist, int* __restrict__ tot, PtRec<T>* __restrict__ pts,
+__device__ __forceinline__ void scatter_small_body(
+    int* small_lds, const T* __restrict__ x, const T* __restrict__ y, int M, int chunk, int L1, int L2, T inv1, T inv2,
+    int nb1, int nbins, int maxpts, const int* __restrict__ hist, int* __restrict__ tot, PtRec<T>* __restrict__ pts,
     int* __restrict__ subbeg, int4* __restrict__ sub, int* __restrict__ nsub)
 {
-    extern __shared__ int small_lds[];
     int *base = small_lds, *tl = small_lds + nbins;       // positions, totals of the bins
     __shared__ int w_a[kScatThreads / 64], w_b[kScatThreads / 64];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -1220,6 +1219,17 @@ __global__ __launch_bounds__(kScatThreads) void k_scatter_small(
             }
         }
     }
+}
+
+template <typename T, bool ONE>
+__global__ __launch_bounds__(kScatThreads) void k_scatter_small(
+    const T* __restrict__ x, const T* __restrict__ y, int M, int chunk, int L1, int L2, T inv1, T inv2, int nb1,
+    int nbins, int maxpts, const int* __restrict__ hist, int* __restrict__ tot, PtRec<T>* __restrict__ pts,
+    int* __restrict__ subbeg, int4* __restrict__ sub, int* __restrict__ nsub)
+{
+    extern __shared__ int small_lds[];
+    scatter_small_body<T, ONE>(small_lds, x, y, M, chunk, L1, L2, inv1, inv2, nb1, nbins, maxpts, hist, tot, pts, subbeg,
+                               sub, nsub);
 }
 
 // ================================================================= window taps
