@@ -57,6 +57,8 @@ struct T1SumArgs {
     double inv1, inv2;            // 1 / (2 N)
 };
 
+typedef __attribute__((address_space(1))) float gfloat;
+typedef __attribute__((address_space(1))) f2v gfloat2;
 constexpr int kSumThreads = 512;
 constexpr int kSumMaxLds = 160 * 1024;
 constexpr int kT1SumMaxN = 256;          // (2j + 1) 2^-33 turn phase error stays below FP32 rounding
@@ -145,6 +147,11 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
         a.part = d.scratch;
         a.M = d.M;
     }
+    // global, not flat: a flat load in flight counts as an LDS operation, and the
+    // next wait for an operand would wait for memory too
+    const gfloat* gx = (const gfloat*)a.x;
+    const gfloat* gy = (const gfloat*)a.y;
+    const gfloat2* gd = (const gfloat2*)a.d;
     const int j1o = c1 * a.k1c, n1 = min(a.k1c, a.N1 / 2 - j1o);
     const int j2o = c2 * a.k2c, n2 = min(a.k2c, a.N2 / 2 - j2o);
     const int nst_all = (a.M + KC - 1) / KC, per = (nst_all + a.S - 1) / a.S;
@@ -157,14 +164,14 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
     // point data: thread roles (u1 w1), (u2 w2), (d') of a stage's points, on
     // the waves whose operand tasks are the cheaper B rows
     const int role = (tid ^ 256) / KC, rp = tid % KC;
-    struct Pt { float x, y; float2 v; };
+    struct Pt { float x, y; f2v v; };
     auto load_point = [&](int st) {
         const int p = p_lo + st * KC + rp;
         const bool ok = role < 3 && p < p_hi;
         Pt r;
-        r.x = ok && role != 1 ? a.x[p] : 0.f;
-        r.y = ok && role != 0 ? a.y[p] : 0.f;
-        r.v = ok && role == 2 ? a.d[p] : make_float2(0.f, 0.f);
+        r.x = ok && role != 1 ? gx[p] : 0.f;
+        r.y = ok && role != 0 ? gy[p] : 0.f;
+        r.v = ok && role == 2 ? gd[p] : f2v{0.f, 0.f};
         return r;
     };
     const Pt first = load_point(0), second = load_point(1);
@@ -172,9 +179,9 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
     // the scale 2^(13 - e), e = exponent of the range's largest sample component
     float mx = 0.f;
     for (int p0 = p_lo; p0 < p_hi; p0 += 4 * kSumThreads) {   // 4 loads in flight
-        float2 v[4];
+        f2v v[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = a.d[min(p0 + k * kSumThreads + tid, p_hi - 1)];
+        for (int k = 0; k < 4; ++k) v[k] = gd[min(p0 + k * kSumThreads + tid, p_hi - 1)];
 #pragma unroll
         for (int k = 0; k < 4; ++k) mx = fmaxf(mx, fmaxf(fabsf(v[k].x), fabsf(v[k].y)));
     }
@@ -301,7 +308,7 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
     put_point(0, first);
     put_point(1, second);
     __syncthreads();
-    float2* out = a.S == 1 && a.bd ? a.F : a.part + (size_t)s * a.N1 * a.N2;
+    gfloat2* out = (gfloat2*)(a.S == 1 && a.bd ? a.F : a.part + (size_t)s * a.N1 * a.N2);
     const float sg = (lane & 1) ? 1.f : -1.f;       // even lanes write s2 = +, odd lanes s2 = -
     if (nst > 0) {
         operands(0);
@@ -355,8 +362,8 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
                 const int j1 = 8 * (rgi * TR + i) + 2 * q + (lane >> 5), j2 = 16 * j + (i32 >> 1);
                 if (j1 < n1 && j2 < n2) {
                     const int col = odd ? a.N2 / 2 - 1 - j2o - j2 : a.N2 / 2 + j2o + j2;
-                    out[(size_t)(a.N1 / 2 + j1o + j1) * a.N2 + col] = fp;
-                    out[(size_t)(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col] = fm;
+                    out[(size_t)(a.N1 / 2 + j1o + j1) * a.N2 + col] = f2v{fp.x, fp.y};
+                    out[(size_t)(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col] = f2v{fm.x, fm.y};
                 }
             }
         }
