@@ -347,6 +347,10 @@ int nfft2d_batch_get_gather_blocks(const nfft2d_batch *batch);
 int nfft2d_batch_set_io_type1(nfft2d_batch *batch, const nfft2d_c64 *const *data, nfft2d_c64 *const *result);
 int nfft2d_batch_type1(nfft2d_batch *batch, void *stream);
 int nfft2d_batch_setpts_type1(nfft2d_batch *batch, void *stream);
+/* setpts_type1 of a batch of equal sizes with every result[t] multiplied by the
+ * N1 x N2 real factors scale (device array, read during the call's work;
+ * NFFT2D_ERR_SIZE when the sizes differ). */
+int nfft2d_batch_setpts_type1_scaled(nfft2d_batch *batch, const float *scale, void *stream);
 
 /* ------------------------------------------------------------------------
  * Type-3 2-D NUFFT (non-uniform to non-uniform), FP64:

@@ -119,10 +119,16 @@ class Batch:
         with torch.cuda.device(self.device):
             check(self._lib.nfft2d_batch_type1(self._h, _stream(self.device)), "nfft2d_batch_type1")
 
-    def setpts_type1(self) -> None:
-        """setpts() then type1(); equal, small transforms as direct sums (1 or 2 launches after setpts())."""
+    def setpts_type1(self, scale=None) -> None:
+        """setpts() then type1(); equal, small transforms as direct sums (1 or 2 launches after setpts()).
+        ``scale`` (N1 x N2 float32, for transforms of equal size) multiplies every result."""
         with torch.cuda.device(self.device):
-            check(self._lib.nfft2d_batch_setpts_type1(self._h, _stream(self.device)), "nfft2d_batch_setpts_type1")
+            if scale is None:
+                check(self._lib.nfft2d_batch_setpts_type1(self._h, _stream(self.device)), "nfft2d_batch_setpts_type1")
+            else:
+                _check(scale, torch.float32, self.sizes[0][0] * self.sizes[0][1], "scale", self.device)
+                check(self._lib.nfft2d_batch_setpts_type1_scaled(self._h, ctypes.c_void_p(scale.data_ptr()),
+                                                                 _stream(self.device)), "nfft2d_batch_setpts_type1_scaled")
 
     def autotune(self, reps: int = 3) -> list:
         """Choose by timing the subproblem size and the direct-gather cut-off per size class and the

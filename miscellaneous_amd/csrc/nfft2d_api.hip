@@ -2016,17 +2016,33 @@ static void batch_choose_t1_sum(nfft2d_batch *b)
 // direct sums leave no LDS for a sort beside them, and the cross-stream waits
 // of an eager call cost more than the sort (165 us on two streams, 143 on one
 // for 250 transforms of 88 x 88 modes from 1,936 points).
-extern "C" int nfft2d_batch_setpts_type1(nfft2d_batch *b, void *stream)
+static int batch_setpts_type1(nfft2d_batch *b, const float *scale, void *stream)
 {
-    if (b && b->t1_sum) {
-        const int rc = nfft2d_batch_setpts(b, stream);
-        if (rc) return rc;
-        t1_sum_launch(b->t1_sum_plan, b->count, (hipStream_t)stream);
+    int rc = nfft2d_batch_setpts(b, stream);
+    if (rc) return rc;
+    if (b->t1_sum) {
+        T1SumPlan q = b->t1_sum_plan;
+        q.a.scale = scale;
+        t1_sum_launch(q, b->count, (hipStream_t)stream);
         NFFT2D_LAUNCH_CHECK();
         return NFFT2D_OK;
     }
-    int rc = nfft2d_batch_setpts(b, stream);
-    return rc ? rc : nfft2d_batch_type1(b, stream);
+    if ((rc = nfft2d_batch_type1(b, stream)) || !scale) return rc;
+    const int n = b->hdesc[0].N1 * b->hdesc[0].N2;
+    hipLaunchKernelGGL(kb_t1_scale, dim3(grid1d(n, 256), b->count), dim3(256), 0, (hipStream_t)stream, b->ddesc, scale, n);
+    NFFT2D_LAUNCH_CHECK();
+    return NFFT2D_OK;
+}
+
+extern "C" int nfft2d_batch_setpts_type1(nfft2d_batch *b, void *stream) { return batch_setpts_type1(b, nullptr, stream); }
+
+extern "C" int nfft2d_batch_setpts_type1_scaled(nfft2d_batch *b, const float *scale, void *stream)
+{
+    if (!b || !scale) return nfft2d_fail(NFFT2D_ERR_ARG, "batch_setpts_type1_scaled: null argument");
+    for (const BatchDesc &d : b->hdesc)
+        if (d.N1 != b->hdesc[0].N1 || d.N2 != b->hdesc[0].N2)
+            return nfft2d_fail(NFFT2D_ERR_SIZE, "batch_setpts_type1_scaled: the transforms' sizes differ");
+    return batch_setpts_type1(b, scale, stream);
 }
 
 // setpts + type-2 of the batch with the bin sort on the batch's second stream,

@@ -350,6 +350,15 @@ __global__ __launch_bounds__(256) void kb_t2_cols(const BatchDesc* __restrict__ 
 }
 
 // ---------------------------------------------------------------- type-1
+// Modes of equal transforms times common factors (block y = transform).
+__global__ __launch_bounds__(256) void kb_t1_scale(const BatchDesc* __restrict__ bd, const float* __restrict__ scale, int n)
+{
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= n) return;
+    float2* F = bd[blockIdx.y].F1;
+    F[e] = cscale(F[e], scale[e]);
+}
+
 // Spread: one block per entry of the batch's subproblem list (base[count]
 // entries), the plan kernel's split-FP16 MFMA tiles into each transform's
 // own tile scratch, indexed by the subproblem's place in its transform.

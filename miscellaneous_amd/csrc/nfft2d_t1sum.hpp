@@ -49,6 +49,7 @@ struct T1SumArgs {
     const float2* d;
     float2* F;                    // S = 1 of a batch writes the modes, else the partial sums go to part
     float2* part;                 // [S][N1][N2]
+    const float* scale;           // null, or N1 x N2 factors of the modes
     int M, N1, N2;
     int S, m1, m2;                // point ranges, mode chunks per dimension
     int k1c, k2c;                 // pairs j per chunk
@@ -328,8 +329,23 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
     // the point groups' sums in a fixed order, one row of tiles at a time, then
     // the four modes of every pair of pairs: an even lane holds the c2 sums of
     // its j2, the odd lane next to it the sin2 sums
+    const gfloat* gs = a.S == 1 && a.bd ? (const gfloat*)a.scale : nullptr;   // else k_t1_sum_add scales
 #pragma unroll
     for (int i = 0; i < TR; ++i) {
+        // this row's factors, in flight together during the exchange
+        float fs[CT][4][2];
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j1 = 8 * (rgi * TR + i) + 2 * q + (lane >> 5), j2 = 16 * j + (i32 >> 1);
+                fs[j][q][0] = fs[j][q][1] = 1.f;
+                if (gs && kgi == 0 && j1 < n1 && j2 < n2) {
+                    const int col = (lane & 1) ? a.N2 / 2 - 1 - j2o - j2 : a.N2 / 2 + j2o + j2;
+                    fs[j][q][0] = gs[(a.N1 / 2 + j1o + j1) * a.N2 + col];
+                    fs[j][q][1] = gs[(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col];
+                }
+            }
         __syncthreads();
         if (kgi > 0) {
 #pragma unroll
@@ -362,8 +378,8 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
                 const int j1 = 8 * (rgi * TR + i) + 2 * q + (lane >> 5), j2 = 16 * j + (i32 >> 1);
                 if (j1 < n1 && j2 < n2) {
                     const int col = odd ? a.N2 / 2 - 1 - j2o - j2 : a.N2 / 2 + j2o + j2;
-                    out[(size_t)(a.N1 / 2 + j1o + j1) * a.N2 + col] = f2v{fp.x, fp.y};
-                    out[(size_t)(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col] = f2v{fm.x, fm.y};
+                    out[(size_t)(a.N1 / 2 + j1o + j1) * a.N2 + col] = f2v{fp.x * fs[j][q][0], fp.y * fs[j][q][0]};
+                    out[(size_t)(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col] = f2v{fm.x * fs[j][q][1], fm.y * fs[j][q][1]};
                 }
             }
         }
@@ -385,7 +401,7 @@ __global__ __launch_bounds__(256) void k_t1_sum_add(T1SumArgs a)
     float2 v = make_float2(0.f, 0.f);
 #pragma unroll 4
     for (int s = 0; s < a.S; ++s) v = cadd(v, part[(size_t)s * n + e]);
-    F[e] = v;
+    F[e] = a.scale ? cscale(v, a.scale[e]) : v;
 }
 
 // ---------------------------------------------------------------- host side

@@ -50,9 +50,14 @@ class FarFieldGeneration:
         self._graph = None
 
     def run(self) -> torch.Tensor:
-        """One generation, eagerly: batched setpts + type-1, then the filter."""
-        self.batch.setpts_type1()
-        self.far_field.mul_(self.filter.view(1, *self.far_field.shape[1:]))
+        """One generation, eagerly: batched setpts + type-1 with the filter's factors on the modes."""
+        f = self.filter
+        if f.dtype == torch.float32 and f.device == self.device and f.is_contiguous() and not f.is_neg() \
+                and f.numel() == self.far_field[0].numel() and not f.requires_grad:
+            self.batch.setpts_type1(scale=f)
+        else:                                        # another filter tensor put in the place of the class's own
+            self.batch.setpts_type1()
+            self.far_field.mul_(f.view(1, *self.far_field.shape[1:]))
         return self.far_field
 
     def capture(self) -> "torch.cuda.CUDAGraph":

@@ -101,3 +101,25 @@ def test_batch_direct_sum(N1, N2, Ms):
         assert oracle.rel_l2(outs[t].cpu().numpy(), got[t]) < 2e-6
         r2 = oracle.ndft_type2(fs[t].cpu().numpy().astype(np.complex128), x1[:64], x2[:64])
         assert oracle.rel_l2(t2[t].cpu().numpy()[:64], r2) < 1e-5
+
+
+# scaled in the sums' epilogue, in the addition of the partial sums, and after the passes of larger transforms
+@pytest.mark.parametrize("P,N1,N2,M", [(250, 88, 88, 60), (3, 40, 54, 900), (2, 64, 300, 700)])
+def test_batch_scaled(P, N1, N2, M):
+    """setpts_type1(scale) is the unscaled result times the factors, bit for bit where the sums are direct."""
+    g = torch.Generator(device=DEV).manual_seed(9)
+    xs = [(torch.rand(M, generator=g, device=DEV) - 0.5) * N1 for _ in range(P)]
+    ys = [(torch.rand(M, generator=g, device=DEV) - 0.5) * N2 for _ in range(P)]
+    ds = [torch.randn(M, generator=g, dtype=torch.complex64, device=DEV) for _ in range(P)]
+    outs = [torch.zeros(N1 * N2, dtype=torch.complex64, device=DEV) for _ in range(P)]
+    b = m.Batch([(N1, N2, M)] * P, device=DEV).set_points(xs, ys).set_io_type1(ds, outs)
+    scale = torch.rand(N1 * N2, generator=g, device=DEV) + 0.5
+    b.setpts_type1()
+    ref = torch.stack(outs) * scale
+    b.setpts_type1(scale=scale)
+    got = torch.stack(outs)
+    if max(N1, N2) <= 256:
+        assert torch.equal(got, ref)
+    assert (got - ref).abs().max().item() < 1e-5 * ref.abs().max().item()
+    with pytest.raises(ValueError):
+        b.setpts_type1(scale=scale[1:])
