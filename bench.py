@@ -737,8 +737,8 @@ def bench_ndft_dropin(args, dev):
         flops = 8.0 * M * nu * nu
         res[tag] = {"config": f"{nu}x{nu} meshgrid outputs, M = {M} points, FP64", "ms": s * 1e3,
                     "fp64_tflops": flops / s / 1e12, "mfma_util": 0.5 * flops / s / 78.6e12}
-    res["note"] = "FP64 flops 8 M N of the plain sum over host-timed calls (half are executed, by conjugate pairs: mfma_util); "
-                   "peak 78.6 TFLOP/s FP64 matrix (spec)"
+    res["note"] = ("FP64 flops 8 M N of the plain sum over host-timed calls (half are executed, by conjugate pairs: "
+                   "mfma_util); peak 78.6 TFLOP/s FP64 matrix (spec)")
     return res
 
 
