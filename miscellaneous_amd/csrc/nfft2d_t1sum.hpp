@@ -28,10 +28,10 @@
 // with e^{2 JS i pi x/N}, computed once per point and stage.
 //
 // Measured (gfx950): 250 transforms of 88 x 88 modes from 1,936 points in one
-// launch 111 us, where spread, column pass and row pass took 144 + 195 + 51;
-// 47 GFLOP executed, 0.42 PFLOP/s: a stage's 27 products per wave (0.8 us of
-// matrix time on each SIMD) and its ~320 VALU instructions per wave pair up to
-// 3.1 us, held by the latency of the operand chain at 2 waves per SIMD.  One
+// launch 105 us, where spread, column pass and row pass took 144 + 195 + 51;
+// 45 GFLOP executed, 0.43 PFLOP/s: a stage's 27 products per wave (0.8 us of
+// matrix time on each SIMD) and its ~400 VALU instructions per wave make 2.9 us,
+// held by the latency of the operand chain at 2 waves per SIMD.  One
 // transform of that size: 9.5 + 3.0 us in two launches, where sort, spread and
 // passes took 30.
 #pragma once
@@ -446,9 +446,9 @@ inline T1SumPlan t1_sum_plan(int N1, int N2, int M, int count, int chain)
         if (s_min > kT1SumMaxS) continue;
         a.S = (int)std::max<long long>(s_min, std::min<long long>(std::min(kT1SumMaxS, st), 256 / tiles));
         p.blocks = tiles * a.S;
-        // us, one block per CU at a time: per point 9 ns, 0.35 ns per pair of the
+        // us, one block per CU at a time, fitted: per point 9 ns, 0.35 ns per pair of the
         // chunk and 0.6 ns per tile slot; per block 8 us and 1 us per tile of a wave
-        // (88 x 88 modes: 111 us for 1,936 points, 126 x 126: 181 for 2,500); then
+        // (88 x 88 modes: 105 us for 1,936 points, 126 x 126: 180 for 2,500); then
         // the partial sums, written and read
         p.t = (double)((p.blocks + 255) / 256) *
               (((st + a.S - 1) / a.S) * KC * (0.009 + 0.00035 * (a.k1c + a.k2c) + 0.0006 * p.rg * p.tr * p.ct) + 8.0 + p.tr * p.ct);
