@@ -177,7 +177,10 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
     };
     const Pt first = load_point(0), second = load_point(1);
 
-    // the scale 2^(13 - e), e = exponent of the range's largest sample component
+    // the scale 2^se brings the range's largest sample component to [2^13, 2^14).  For
+    // samples below 2^-98 it and its inverse take two factors each, the second one 1 for
+    // all others (ldexp on every mode instead, or a branch that scales the sums: 105.2 ->
+    // 107.5 us for 250 transforms of 88 x 88 modes)
     float mx = 0.f;
     for (int p0 = p_lo; p0 < p_hi; p0 += 4 * kSumThreads) {   // 4 loads in flight
         f2v v[4];
@@ -194,9 +197,10 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
 #pragma unroll
     for (int k = 0; k < 8; ++k) mx = fmaxf(mx, red[k]);
     __syncthreads();
-    const int ex = max((int)((__float_as_uint(mx) >> 23) & 0xff) - 127, -95);
-    const float sc = __uint_as_float((unsigned)(127 + 13 - ex) << 23);
-    const float inv_sc = __uint_as_float((unsigned)(127 - 13 + ex) << 23) * 6.103515625e-05f;   // 2^-14: the phasors'
+    const int se = __builtin_amdgcn_readfirstlane(14 - __builtin_amdgcn_frexp_expf(mx));
+    const int sa = min(se, 112), sb = se - sa;
+    auto pow2 = [](int e) { return __uint_as_float((unsigned)(127 + e) << 23); };
+    const float sc = pow2(sa), sc2 = pow2(sb), inv_sc = pow2(-sa - 14), inv_sc2 = pow2(-sb);   // and the phasors' 2^14
 
     auto put_point = [&](int st, const Pt& r) {
         SumPoint& q = pd[(st & 1) * KC + rp];
@@ -210,7 +214,7 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
             q.w2 = turn_cs(2u * (unsigned)a.js2 * u);
         } else if (role == 2) {
             const float2 e = turn_cs(turn_of((double)r.x, a.inv1, a.N1) + turn_of((double)r.y, a.inv2, a.N2));
-            const float vx = r.v.x * sc, vy = r.v.y * sc;
+            const float vx = r.v.x * sc * sc2, vy = r.v.y * sc * sc2;
             float2 v = make_float2(vx * e.x - vy * e.y, vx * e.y + vy * e.x);
             // coordinates beyond the transform's range give NaN, as locate() does
             if (!(fabsf((float)kC * r.x) < 1073741824.f) || !(fabsf((float)kC * r.y) < 1073741824.f))
@@ -378,8 +382,8 @@ __global__ __launch_bounds__(kSumThreads) void k_t1_sum(T1SumArgs a)
                 const int j1 = 8 * (rgi * TR + i) + 2 * q + (lane >> 5), j2 = 16 * j + (i32 >> 1);
                 if (j1 < n1 && j2 < n2) {
                     const int col = odd ? a.N2 / 2 - 1 - j2o - j2 : a.N2 / 2 + j2o + j2;
-                    out[(size_t)(a.N1 / 2 + j1o + j1) * a.N2 + col] = f2v{fp.x * fs[j][q][0], fp.y * fs[j][q][0]};
-                    out[(size_t)(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col] = f2v{fm.x * fs[j][q][1], fm.y * fs[j][q][1]};
+                    out[(size_t)(a.N1 / 2 + j1o + j1) * a.N2 + col] = f2v{fp.x * (fs[j][q][0] * inv_sc2), fp.y * (fs[j][q][0] * inv_sc2)};
+                    out[(size_t)(a.N1 / 2 - 1 - j1o - j1) * a.N2 + col] = f2v{fm.x * (fs[j][q][1] * inv_sc2), fm.y * (fs[j][q][1] * inv_sc2)};
                 }
             }
         }
