@@ -159,7 +159,9 @@ __device__ __forceinline__ float2 expi_neg(int k, float x, double invN)
 //   part t % 2 (0: Re, 1: Im); for P (Q with EQ, OQ):
 //   Re P = sum c Re EP - (-s) Im OP,  Im P = sum c Im EP + (-s) Re OP.
 // Entries with j1 >= N1 / 2 or j2 >= N2 / 2 are zero (padding to whole tiles).
-// The sums of four modes are taken in FP64 and rounded once.
+// The sums of four modes are taken in FP64 and rounded once, as their quarter:
+// four modes beyond a quarter of the FP32 range would overflow in a plain sum
+// whose results still fit.  The results take the 4 back with the half steps.
 // Single modes (FP16): k2 index j2 as above with components (Re B, Im B), k1
 // index j1 = ch * 16 C + 32 (t / 2) + cc, part t % 2 of T:
 //   Re T = sum Re B Re F - Im B Im F,  Im T = sum Re B Im F + Im B Re F.
@@ -195,8 +197,8 @@ __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F,
                 o.x = ((double)pp.x - (double)pm.x) + sq * ((double)mp.x - (double)mm.x);
                 o.y = ((double)pp.y - (double)pm.y) + sq * ((double)mp.y - (double)mm.y);
             }
-            v[2 * q] = (float)(part == 0 ? e.x : e.y);
-            v[2 * q + 1] = (float)(part == 0 ? -o.y : o.x);
+            v[2 * q] = (float)(0.25 * (part == 0 ? e.x : e.y));
+            v[2 * q + 1] = (float)(0.25 * (part == 0 ? -o.y : o.x));
         }
     } else {
         const int j1 = ch * 16 * C + 32 * (t >> 1) + cc;
@@ -532,11 +534,13 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
             }
         }
     }
-    // pairs: y carries e^{pi i (x1 / N1 + x2 / N2)}, the half steps of both dimensions
+    // pairs: y carries 4 e^{pi i (x1 / N1 + x2 / N2)}, the half steps of both dimensions (and the operand's quarter)
     float2 half[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int r = 0; r < R; ++r) {
         half[r] = kPair ? expi_neg_turns(-((double)xr1[r] * pu1 + (double)xr2[r] * pu2)) : make_float2(1.f, 0.f);
+        if (kPair) half[r] = make_float2(4.f * half[r].x, 4.f * half[r].y);
+    }
     // the two halves of each row, then (SPLIT = 2) the two column shares
 #pragma unroll
     for (int r = 0; r < R; ++r) {
