@@ -363,7 +363,7 @@ static int czt_buffer(int N, void **out, int *mout)
     };
     pass(N, L, -N / 2, 0);   // type-2
     pass(L, N, 0, -N / 2);   // type-1
-    for (int j = 0; j < m; ++j) put(std::polar(1.0, -2.0 * kPi * (double)j / m));
+    for (int e = 0; e < m; ++e) put(std::polar(1.0, -2.0 * kPi * (double)czt_tw_index(m, e) / m));
     if (nfft2d_malloc(out, sizeof(C) * h.size()) != hipSuccess)
         return nfft2d_fail(NFFT2D_ERR_ALLOC, "plan tables: hipMalloc of the chirp-z tables failed");
     NFFT2D_HIP_TRY(hipMemcpy(*out, h.data(), sizeof(C) * h.size(), hipMemcpyHostToDevice));

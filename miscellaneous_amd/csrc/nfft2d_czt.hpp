@@ -22,7 +22,13 @@
 // leaves them: the kernel product and the start of the second FFT need no
 // exchange, and each FFT makes stages - 1 (three) trips through LDS.  Measured
 // on FP64 lines of 500 and 250 (500 x 250 modes, both passes of a type-2 /
-// type-1): 36 / 35 -> 25 / 24 us.
+// type-1): 36 / 35 -> 25 / 24 us.  The twiddles come from global memory, so
+// they lie in the order in which a stage's roles read them: as one table
+// e^{-2 pi i j / m} read at strides of m / (8 NS) they were up to 448 cache lines
+// per wave and stage, and long lines ran behind the LDS form (type-2 of N x N
+// modes to 20,000 points, LDS form / one table / stage order: complex64 N =
+// 1,500 386 / 447 / 307 us, 3,000 2,571 / 4,800 / 1,633, complex128 1,800 1,040
+// / 880 / 529).
 #pragma once
 
 #include <mutex>
@@ -38,7 +44,7 @@ struct CztTables {
     const cplx<T> *cin = nullptr;    // c[p + p0], P
     const cplx<T> *cout = nullptr;   // c[q + q0], Q
     const cplx<T> *hhat = nullptr;   // FFT_m of the kernel conj(c[d + q0 - p0]), d = q - p
-    const cplx<T> *tw = nullptr;     // e^{-2 pi i j / m}, m
+    const cplx<T> *tw = nullptr;     // the FFT's twiddles, m (czt_tw_index)
     int P = 0, Q = 0, m = 0;
 };
 
@@ -51,6 +57,19 @@ __host__ __device__ constexpr int czt_m(int N)
     int m = 1;
     while (m < 3 * N - 1) m <<= 1;
     return m;
+}
+
+// Entry e of the twiddle table is e^{-2 pi i czt_tw_index(m, e) / m}: the stages'
+// twiddles w^{r k}, r = 1..7, k < NS, one stage after the other in the order
+// [r][k], so that neighbouring roles read neighbouring entries (m - r0 in all).
+__host__ __device__ constexpr int czt_tw_index(int m, int e)
+{
+    int n = 0, t = 0;
+    while ((1 << n) < m) ++n;
+    const int r0 = n % 3 == 0 ? 3 : n % 3, q = e + (1 << r0);   // stage s: q in [NS, 8 NS)
+    while ((1 << (t + 1)) <= q) ++t;
+    t = (t - r0) / 3 * 3 + r0;
+    return t < n ? (((q - (1 << t)) >> t) + 1) * (q & ((1 << t) - 1)) * (m / 8 >> t) : 0;
 }
 
 // The chirp-z tables of a line length N inside one table buffer (layout
@@ -127,14 +146,15 @@ __device__ __forceinline__ void czt_fft(cplx<T> (&v)[K][8], cplx<T>* lds, const 
     for (int s = 1; s < S; ++s) {
         const int NS = FftPlan<M>::ns(s);
         const bool last = s == S - 1;
-        // the stage's twiddles, in flight across the barrier and the LDS reads
-        C w[K][7];
+        // the stage's twiddles, in flight across the barrier and the LDS reads; with
+        // two roles a thread only when each is played (both roles' spill)
+        C w[7];
+        auto twiddles = [&](int j) {
+            const C* __restrict__ t = tw + NS - R0 + (j & (NS - 1));
 #pragma unroll
-        for (int u = 0; u < K; ++u) {
-            const int e = ((last ? jo[u] : jm[u]) & (NS - 1)) * (TPL / NS);
-#pragma unroll
-            for (int r = 1; r < 8; ++r) w[u][r - 1] = tw[r * e];
-        }
+            for (int r = 1; r < 8; ++r) w[r - 1] = t[(r - 1) * NS];
+        };
+        if constexpr (K == 1) twiddles(last ? jo[0] : jm[0]);
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < K; ++u) {
@@ -148,8 +168,9 @@ __device__ __forceinline__ void czt_fft(cplx<T> (&v)[K][8], cplx<T>* lds, const 
 #pragma unroll
         for (int u = 0; u < K; ++u) {
             const int j = last ? jo[u] : jm[u], k = j & (NS - 1);
+            if constexpr (K > 1) twiddles(j);
 #pragma unroll
-            for (int r = 1; r < 8; ++r) v[u][r] = cmul_f(v[u][r], w[u][r - 1]);
+            for (int r = 1; r < 8; ++r) v[u][r] = cmul_f(v[u][r], w[r - 1]);
             dft8<-1>(v[u]);
             if (!last && act[u]) {
                 const int o = (j - k) * 8 + k;
@@ -177,6 +198,9 @@ __device__ __forceinline__ void czt_lines(int line0, int lines, cplx<T>* lds, co
 {
     using C = cplx<T>;
     constexpr int M = 1 << LOGM, TPL = M / 8;
+    // kernel and output factors loaded ahead of the FFT they follow; at 1,024
+    // threads (128 registers each) only when they are used
+    constexpr bool kAhead = LOGM < 13;
     bool act[K];
     int la[K], ja[K], lm[K], jm[K], lo[K], jo[K];
 #pragma unroll
@@ -217,19 +241,25 @@ __device__ __forceinline__ void czt_lines(int line0, int lines, cplx<T>* lds, co
             x = cmul_f(x, c[q]);
             v[u][q] = ja[u] + q * TPL < tb.P ? x : mk((T)0, (T)0);
         }
+        if constexpr (kAhead)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) h[u][q] = tb.hhat[(jm[u] + q * TPL) & (M - 1)];
+            for (int q = 0; q < 8; ++q) h[u][q] = tb.hhat[(jm[u] + q * TPL) & (M - 1)];
     }
     czt_fft<T, LOGM, K>(v, lds, tb.tw, act, la, ja, lm, jm, lm, jm);
 #pragma unroll
-    for (int u = 0; u < K; ++u)
+    for (int u = 0; u < K; ++u) {
+        if constexpr (!kAhead)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) h[u][q] = tb.hhat[(jm[u] + q * TPL) & (M - 1)];
 #pragma unroll
         for (int q = 0; q < 8; ++q) v[u][q] = cconj(cmul_f(v[u][q], h[u][q]));
+    }
     __syncthreads();
+    if constexpr (kAhead)
 #pragma unroll
-    for (int u = 0; u < K; ++u)
+        for (int u = 0; u < K; ++u)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) h[u][q] = tb.cout[min(jo[u] + q * TPL, tb.Q - 1)];
+            for (int q = 0; q < 8; ++q) h[u][q] = tb.cout[min(jo[u] + q * TPL, tb.Q - 1)];
     czt_fft<T, LOGM, K>(v, lds, tb.tw, act, lm, jm, lm, jm, lo, jo);
     const T inv = (T)1 / (T)M;
 #pragma unroll
@@ -241,6 +271,7 @@ __device__ __forceinline__ void czt_lines(int line0, int lines, cplx<T>* lds, co
         for (int q = 0; q < 8; ++q) {
             const int o = jo[u] + q * TPL;
             if (o < tb.Q) {
+                if constexpr (!kAhead) h[u][q] = tb.cout[o];
                 C x = cmul_f(cscale(cconj(v[u][q]), inv), h[u][q]);
                 if (conj) x = cconj(x);
                 if (!scale_in && sl) x = cscale(x, lsc * se[o]);

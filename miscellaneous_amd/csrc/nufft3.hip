@@ -262,7 +262,7 @@ __device__ __forceinline__ void axis_entry(const AxisTables &t, int e)
     }
     if (e < t.m) {
         double sn, cs;
-        sincospi(2.0 * e / t.m, &sn, &cs);
+        sincospi(2.0 * nfft2d::czt_tw_index(t.m, e) / t.m, &sn, &cs);
         t.tw[e] = make_double2(cs, -sn);
         double2 h = make_double2(0.0, 0.0);
         const int d = e < t.Q ? e : e - t.m;
