@@ -574,7 +574,7 @@ static int setpts_impl(nfft2d_plan *p, const T *x, const T *y, int M, hipStream_
     const bool lds = p->nbins <= kMaxLdsBins;
     const T inv1 = (T)(1.0 / p->L1), inv2 = (T)(1.0 / p->L2);
     const bool one = p->nbins <= kSmallBins && M <= kOnePts;
-    const bool small = one || (p->nbins <= kSmallBins && (long long)nblk * p->nbins <= kSmallHist);
+    const bool small = one || (nblk <= kSmallBlocks && p->nbins <= kSmallBins && (long long)nblk * p->nbins <= kSmallHist);
     if (one) {
         // counted by the scatter block
     } else if (lds) {

@@ -1107,7 +1107,11 @@ __global__ __launch_bounds__(kScatThreads) void k_scatter_lds(
 // three launches, 7.9 in one; 16,384 points on 128^2 16.9 -> 12.3 us in two.
 // Writes tot, subbeg, sub and nsub as k_colscan and k_scatter_lds do.
 constexpr int kOnePts = kScatThreads * kScatPer;      // one batch of the block's points, held in registers
-constexpr int kSmallBins = 4096, kSmallHist = 32768;
+// A block reads its bins' counts of all blocks, 8 rows at a time: a chain of
+// nblk / 8 loads, which three launches undercut from about 80 blocks on (points on
+// 64^2 modes, two launches / three, us: 64 blocks 13.6 / 15.7, 79 14.6 / 15.8, 128
+// 17.2 / 16.0, 196 21.5 / 17.0).
+constexpr int kSmallBins = 4096, kSmallHist = 32768, kSmallBlocks = 64;
 template <typename T, bool ONE>
 __device__ __forceinline__ void scatter_small_body(
     int* small_lds, const T* __restrict__ x, const T* __restrict__ y, int M, int chunk, int L1, int L2, T inv1, T inv2,
