@@ -908,9 +908,11 @@ extern "C" int nfft2d_type2(nfft2d_plan *p, void *result, const void *data, void
 // the chip or is a few launches long: two streams against one, eager, 128^2 /
 // 16K points 54.9 / 26.8 us, 512^2 / 1M 81.9 / 71.2, 1024^2 / 4M 216 / 214.
 // The chirp-z passes of large grids leave room beside them: 500^2 / 300K 79.2
-// / 74.1, 1000^2 / 1M 194 / 211.  In a captured graph the branches cost less:
-// 256^2 / 64K 38.8 / 36.1, 512^2 / 1M 71.0 / 76.1, 1024^2 / 4M 205 / 219.
-static bool fork_pays(const nfft2d_plan *p, hipStream_t s)
+// / 74.1, 1000^2 / 1M 194 / 211.  In a captured graph the branches cost less,
+// and either long grid passes or a long sort hide one in the other: 128^2 / 131K
+// 42.4 / 38.1, 256^2 / 262K 47.2 / 45.0, 512^2 / 1M 70.9 / 77.6, 1024^2 / 4M 205 /
+// 218; 64^2 / 524K 46.2 / 50.3, 128^2 / 524K 50.1 / 52.5, 256^2 / 2M 94.7 / 103.
+static bool fork_pays(const nfft2d_plan *p, int M, hipStream_t s)
 {
     const long long modes = (long long)p->N1 * p->N2;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -918,7 +920,7 @@ static bool fork_pays(const nfft2d_plan *p, hipStream_t s)
         (void)hipGetLastError();
         cs = hipStreamCaptureStatusNone;
     }
-    if (cs == hipStreamCaptureStatusActive) return modes >= 1 << 18;
+    if (cs == hipStreamCaptureStatusActive) return modes >= 1 << 18 || M >= 1 << 19;
     return (p->czt[0] || p->czt[1]) && modes >= 1 << 19;
 }
 
@@ -940,7 +942,7 @@ extern "C" int nfft2d_setpts_type2(nfft2d_plan *p, void *result, const void *dat
     hipStream_t s = (hipStream_t)stream;
     rc = p->fk.init(p->device);
     if (rc) return rc;
-    if (!fork_pays(p, s)) {
+    if (!fork_pays(p, M, s)) {
         if ((rc = nfft2d_setpts(p, x, y, M, stream))) return rc;
         return nfft2d_type2(p, result, data, stream);
     }
