@@ -113,12 +113,16 @@ void Destroy_cuFFT_plan_NFFT2_2D(void);
  * (:44,56) before its gemv (:67); neither happens here.  Outputs on a meshgrid
  * (u, v arithmetic progressions, either flattening; detected on the device)
  * take the FP64 matrix-core contraction, any other (u, v) the direct sum.  Runs
- * on the legacy default stream.  A workspace of at most 256 N + 5 M complex
- * values (4.2 million + 5 M from N = 16,384 outputs on, N + 5 M from 4.2
- * million on) is kept per device and grown when a call needs more (the growth
- * synchronises the device); concurrent calls on one device serialise on it. */
+ * on the legacy default stream.  A workspace (nfft2d_ndft_workspace_bytes) is
+ * kept per device and grown when a call needs more (the growth synchronises
+ * the device); concurrent calls on one device serialise on it. */
 int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, const double *u, const double *v,
                  const nfft2d_c128 *in, nfft2d_c128 *out, int Nu, int Nv, int M, int N);
+
+/* Bytes of the workspace that an NDFT2_2D_GPU call of M points and N outputs
+ * needs, 16 per complex value: partial sums (at most 256 N values, 8.4 million
+ * from N = 32,768 outputs on, N from 8.4 million on) and 4 M for the points. */
+long long nfft2d_ndft_workspace_bytes(int M, int N);
 
 /* No counterpart in the reference; for callers and tests that check which path
  * an NDFT2_2D_GPU call took.  Synchronises the current device and reports the

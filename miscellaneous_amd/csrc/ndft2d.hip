@@ -405,7 +405,28 @@ __global__ __launch_bounds__(kThreads) void k_ndft_finish(const double2 *__restr
     out[n] = make_double2(sr, si);
 }
 
+// Point ranges: a work item per CU at the tile count that a square grid of N
+// outputs has at least, each range at least one chunk of points.
+int point_ranges(int M, int N)
+{
+    const int ranges = std::max(1, kGridBlocks / std::max(1, N / (4 * kTilePairs * kTilePairs)));
+    return std::max(1, std::min(ranges, (M + kGridChunk - 1) / kGridChunk));
+}
+// The workspace, in complex values: ranges N partial sums (256 N below two
+// tiles' outputs, then at most 1 + 1 / k times 256 tiles' for N / 16,384 = k, or
+// N), then the prepared points.
+size_t workspace_values(int M, int N)
+{
+    return (size_t)point_ranges(M, N) * (size_t)N + sizeof(GridPt) / sizeof(double2) * (size_t)M;
+}
+
 }  // namespace
+
+extern "C" long long nfft2d_ndft_workspace_bytes(int M, int N)
+{
+    if (M < 0 || N < 0) return nfft2d_fail(NFFT2D_ERR_ARG, "nfft2d_ndft_workspace_bytes: M = %d, N = %d", M, N);
+    return N == 0 ? 0 : (long long)(sizeof(double2) * workspace_values(M, N));
+}
 
 extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, const double *u, const double *v,
                             const nfft2d_c128 *in, nfft2d_c128 *out, int Nu, int Nv, int M, int N)
@@ -418,11 +439,7 @@ extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, cons
         return nfft2d_fail(NFFT2D_ERR_ARG, "NDFT2_2D_GPU: null pointer");
     // (u, v) a grid: FP64 MFMA contraction; otherwise the direct sum (k_ndft_grid
     // reads the detector's finding and does one or the other).
-    // Point ranges: a work item per CU at the tile count a square grid of N
-    // outputs would have, each range at least one chunk of points.
-    const long long ntile_est = std::max<long long>(1, (long long)N / (4 * kTilePairs * kTilePairs));
-    int ranges = (int)std::max<long long>(1, kGridBlocks / ntile_est);
-    ranges = std::max(1, std::min(ranges, (M + kGridChunk - 1) / kGridChunk));
+    const int ranges = point_ranges(M, N);
     const int chunk = ((M + ranges - 1) / ranges + kGridChunk - 1) / kGridChunk * kGridChunk;
     const int dev = [] { int d = 0; (void)hipGetDevice(&d); return d; }();
     double2 *part = nullptr;
@@ -431,8 +448,7 @@ extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, cons
     std::lock_guard<std::mutex> lk(g_ws_mu);
     {
         GridWs &ws = g_ws[dev];
-        // partial sums, then the prepared points
-        const size_t need = (size_t)ranges * (size_t)N + sizeof(GridPt) / sizeof(double2) * (size_t)M;
+        const size_t need = workspace_values(M, N);
         if (ws.count < need) {
             if (ws.ptr) {
                 (void)hipDeviceSynchronize();
