@@ -186,14 +186,16 @@ __global__ __launch_bounds__(kThreads) void k_grid_verify(const double *__restri
 // accumulator element r of lane l is C[4 r + l / 16][l % 16].  A block takes a
 // tile of 64 x 64 pairs (128 x 128 outputs) over one range of the points: wave
 // w the 16 x 32 pairs of row tile w / 2, column tiles 2 (w % 2) and + 1 (16
-// accumulator tiles, 128 VGPRs; 2 waves per SIMD).  FP64 VALU work does not
-// run under FP64 MFMAs, so the phasors are evaluated once per block: for a
+// accumulator tiles, 128 VGPRs; 2 waves per SIMD); where only one row or column
+// tile is in use, wave w < 4 its w-th (1 x 20,000 outputs from M = 65,536: 6.5 ->
+// 3.8 ms; two waves of two tiles each left two SIMDs idle).  FP64 VALU work does
+// not run under FP64 MFMAs, so the phasors are evaluated once per block: for a
 // chunk of 16 points each of the 512 threads takes one (point, row or column
 // index mod 16) by an FP64 phase reduction and sincospi, advances it three
 // times by the point's 16-step phasor, and leaves the four in LDS (two
 // buffers) while the previous chunk's products run.
-// 256 x 256 outputs from M = 65,536: 0.32 ms a call, 0.75 of the FP64 matrix rate (one wave per 32 x 64
-// outputs with its own phasors and complex products: 0.69 ms).
+// 256 x 256 outputs from M = 65,536: 0.30 ms a call, 0.22 at the FP64 matrix rate
+// (one wave per 32 x 64 outputs with its own phasors and complex products: 0.69).
 // The partial sums go to range r's slice of a workspace; k_ndft_finish adds
 // the ranges in a fixed order (the result does not depend on the launch).
 // Work items are walked persistently (their count is known on the device only).
@@ -240,6 +242,18 @@ __device__ __forceinline__ void direct_item(const double *__restrict__ X, const 
     acc = make_double2(ar, ai);
 }
 
+// Point ranges in use on a grid.  A thin grid has far more tiles than a square
+// one of as many outputs, and every item has its fixed cost (its first chunk,
+// its partial sums written and added): where the ranges given would be shorter
+// than 16 chunks, no more than four items per block.
+// Outputs 1 x 4,096 from M = 5,000, 32 tiles: 256 ranges 215 us, 32 120 (75 with
+// one tile per wave); 1 x 20,000 1,001 -> 555 (328); 2 x 2,000 118 -> 68 (47).
+__device__ __forceinline__ int grid_ranges(const GridInfo &g, int M, int ranges)
+{
+    const int tiles = ((g.nu + 1) / 2 + kTilePairs - 1) / kTilePairs * (((g.nv + 1) / 2 + kTilePairs - 1) / kTilePairs);
+    return min(ranges, max(max(1, 4 * kGridBlocks / tiles), M / (16 * kGridChunk)));
+}
+
 __global__ __launch_bounds__(kGridThreads) void k_ndft_grid(const GridPt *__restrict__ pts,
                                                             double2 *__restrict__ part, int M, int ranges, int chunk,
                                                             const double *__restrict__ X, const double *__restrict__ Y,
@@ -267,19 +281,28 @@ __global__ __launch_bounds__(kGridThreads) void k_ndft_grid(const GridPt *__rest
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
     const int nu2 = (g.nu + 1) / 2, nv2 = (g.nv + 1) / 2;    // pairs (an odd length's centre is a pair of its own)
     const int tcols = (nv2 + kTilePairs - 1) / kTilePairs;
+    ranges = grid_ranges(g, M, ranges);
+    chunk = ((M + ranges - 1) / ranges + kGridChunk - 1) / kGridChunk * kGridChunk;
     const int items = (nu2 + kTilePairs - 1) / kTilePairs * tcols * ranges;
     const long long N = (long long)g.nu * g.nv;
     // phasor role of this thread: side, point of the chunk, index mod 16
-    const int side = t >> 8, pt = (t >> 4) & 15, pq = t & 15;
-    const int rt = w >> 1, ct = 2 * (w & 1);
-    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int side = w >> 2, pt = (t >> 4) & 15, pq = t & 15;
+    // rounds of one item per block; where a round spans tiles every other one goes
+    // backwards, so that a block that took a whole tile's share gets an edge tile's next
+    for (int i0 = 0, back = 0; i0 < items; i0 += gridDim.x, back ^= ranges < (int)gridDim.x) {
+        const int item = i0 + (int)(back ? gridDim.x - 1 - blockIdx.x : blockIdx.x);
+        if (item >= items) continue;
         const int r = item % ranges, st = item / ranges;
         const int p1 = (st / tcols) * kTilePairs, p2 = (st % tcols) * kTilePairs;   // first pairs of the tile
         const int m_lo = min(M, r * chunk), m_hi = min(M, m_lo + chunk);
         const double idx = side ? p2 + pq + (g.nv & 1 ? 0.0 : 0.5) : p1 + pq + (g.nu & 1 ? 0.0 : 0.5);
         const double off = idx * (side ? g.dv : g.du);
-        const bool act = p1 + 16 * rt < nu2;
-        const bool act0 = act && p2 + 16 * ct < nv2, act1 = act && p2 + 16 * ct + 16 < nv2;
+        // the tile's 16-pair rows and columns in use; a single one of either lies on
+        // four waves of four SIMDs, not on two
+        const int nrt = min(4, (nu2 - p1 + 15) / 16), nct = min(4, (nv2 - p2 + 15) / 16);
+        const int rt = nrt == 1 ? 0 : nct == 1 ? w : w >> 1, ct = nrt == 1 ? w : nct == 1 ? 0 : 2 * (w & 1);
+        const bool act0 = rt < nrt && ct < nct, act1 = nrt > 1 && rt < nrt && ct + 1 < nct;
+        const int nst = side ? nct : nrt;
         struct Pt {
             double2 d, step;
             double x;
@@ -301,8 +324,9 @@ __global__ __launch_bounds__(kGridThreads) void k_ndft_grid(const GridPt *__rest
             double2 z = phasor(off * p.x);
 #pragma unroll
             for (int h = 0; h < 4; ++h) {
+                if (h >= nst) break;
+                if (h > 0) z = zmul(z, p.step);
                 s_ph[b][side][pt][16 * h + pq] = z;
-                if (h < 3) z = zmul(z, p.step);
             }
             if (side == 0 && pq == 0) s_d[b][pt] = p.d;
         };
@@ -321,24 +345,25 @@ __global__ __launch_bounds__(kGridThreads) void k_ndft_grid(const GridPt *__rest
             const Pt cur = nxt;
             nxt = load(m0 + 2 * kGridChunk + pt);
             if (m0 + kGridChunk < m_hi) stage(cur, b ^ 1);
+            if (act0)
 #pragma unroll
-            for (int s = 0; s < kGridChunk / 4; ++s) {
-                const double2 d = s_d[b][4 * s + k], a = s_ph[b][0][4 * s + k][16 * rt + q];
-                const double cr = d.x * a.x, ci = d.y * a.x, tr = d.x * a.y, ti = d.y * a.y;
+                for (int s = 0; s < kGridChunk / 4; ++s) {
+                    const double2 d = s_d[b][4 * s + k], a = s_ph[b][0][4 * s + k][16 * rt + q];
+                    const double cr = d.x * a.x, ci = d.y * a.x, tr = d.x * a.y, ti = d.y * a.y;
 #pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    if (!(c ? act1 : act0)) continue;
-                    const double2 v = s_ph[b][1][4 * s + k][16 * (ct + c) + q];
-                    ar[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(cr, v.x, ar[c][0], 0, 0, 0);
-                    ai[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ci, v.x, ai[c][0], 0, 0, 0);
-                    ar[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, v.x, ar[c][1], 0, 0, 0);
-                    ai[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, v.x, ai[c][1], 0, 0, 0);
-                    ar[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(cr, v.y, ar[c][2], 0, 0, 0);
-                    ai[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(ci, v.y, ai[c][2], 0, 0, 0);
-                    ar[c][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, v.y, ar[c][3], 0, 0, 0);
-                    ai[c][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, v.y, ai[c][3], 0, 0, 0);
+                    for (int c = 0; c < 2; ++c) {
+                        if (c && !act1) continue;
+                        const double2 v = s_ph[b][1][4 * s + k][16 * (ct + c) + q];
+                        ar[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(cr, v.x, ar[c][0], 0, 0, 0);
+                        ai[c][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(ci, v.x, ai[c][0], 0, 0, 0);
+                        ar[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, v.x, ar[c][1], 0, 0, 0);
+                        ai[c][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, v.x, ai[c][1], 0, 0, 0);
+                        ar[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(cr, v.y, ar[c][2], 0, 0, 0);
+                        ai[c][2] = __builtin_amdgcn_mfma_f64_16x16x4f64(ci, v.y, ai[c][2], 0, 0, 0);
+                        ar[c][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(tr, v.y, ar[c][3], 0, 0, 0);
+                        ai[c][3] = __builtin_amdgcn_mfma_f64_16x16x4f64(ti, v.y, ai[c][3], 0, 0, 0);
+                    }
                 }
-            }
             __syncthreads();
         }
         // the four outputs of each pair of pairs: rows nu / 2 + p and nu - 1 - (nu / 2 + p)
@@ -347,6 +372,7 @@ __global__ __launch_bounds__(kGridThreads) void k_ndft_grid(const GridPt *__rest
         for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
+                if (!(c ? act1 : act0)) continue;
                 const int i = g.nu / 2 + p1 + 16 * rt + 4 * e + k, j = g.nv / 2 + p2 + 16 * (ct + c) + q;
                 if (i >= g.nu || j >= g.nv) continue;
 #pragma unroll
@@ -374,7 +400,7 @@ std::map<int, GridWs> g_ws;
 // caller's flattening: 64 outputs per block, 4 threads each over every fourth
 // range.
 constexpr int kSumOut = 64;
-__global__ __launch_bounds__(kThreads) void k_ndft_finish(const double2 *__restrict__ part, int ranges,
+__global__ __launch_bounds__(kThreads) void k_ndft_finish(const double2 *__restrict__ part, int M, int ranges,
                                                           double2 *__restrict__ out, int N)
 {
     const GridInfo g = g_grid;
@@ -386,6 +412,7 @@ __global__ __launch_bounds__(kThreads) void k_ndft_finish(const double2 *__restr
         if (g.ok) {
             const int i = g.vmajor ? n % g.nu : n / g.nv, j = g.vmajor ? n / g.nu : n % g.nv;
             e = (size_t)i * g.nv + j;
+            ranges = grid_ranges(g, M, ranges);
         }
         const double2 *src = part + e;
 #pragma unroll 4
@@ -476,7 +503,7 @@ extern "C" int NDFT2_2D_GPU(void *handle, const double *X, const double *Y, cons
     hipLaunchKernelGGL(k_ndft_grid, dim3(kGridBlocks), dim3(kGridThreads), 0, nullptr, pts, part, M, ranges, chunk, X, Y,
                        u, v, din, 1.0 / Nu, 1.0 / Nv, N);
     NFFT2D_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_ndft_finish, dim3((N + kSumOut - 1) / kSumOut), dim3(kThreads), 0, nullptr, part, ranges,
+    hipLaunchKernelGGL(k_ndft_finish, dim3((N + kSumOut - 1) / kSumOut), dim3(kThreads), 0, nullptr, part, M, ranges,
                        reinterpret_cast<double2 *>(out), N);
     NFFT2D_LAUNCH_CHECK();
     return NFFT2D_OK;
