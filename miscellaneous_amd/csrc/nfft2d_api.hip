@@ -1887,7 +1887,7 @@ static int batch_gather(nfft2d_batch *b, hipStream_t s)
                        b->plans[0]->wa);
     NFFT2D_LAUNCH_CHECK();
     constexpr int per_block = 256 / kDirectLanes;   // list entries per block
-    hipLaunchKernelGGL(kb_gather_direct, dim3((unsigned)(((b->bsubcap + per_block - 1) / per_block + 63) & ~63ll)), dim3(256), 0, s,
+    hipLaunchKernelGGL(kb_gather_direct, dim3((unsigned)((b->bsubcap + per_block - 1) / per_block)), dim3(256), 0, s,
                        b->ddesc, b->bsub, b->base + b->count, b->plans[0]->wa);
     NFFT2D_LAUNCH_CHECK();
     return NFFT2D_OK;
