@@ -351,6 +351,10 @@ int nfft2d_batch_get_gather_blocks(const nfft2d_batch *batch);
 int nfft2d_batch_set_io_type1(nfft2d_batch *batch, const nfft2d_c64 *const *data, nfft2d_c64 *const *result);
 int nfft2d_batch_type1(nfft2d_batch *batch, void *stream);
 int nfft2d_batch_setpts_type1(nfft2d_batch *batch, void *stream);
+/* How the next setpts_type1 goes with the arrays set now: 0 the passes of
+ * type1, S > 0 the direct sums with the points in S ranges (S > 1: partial sums
+ * and a second launch that adds them). */
+int nfft2d_batch_get_type1_ranges(const nfft2d_batch *batch);
 /* setpts_type1 of a batch of equal sizes with every result[t] multiplied by the
  * N1 x N2 real factors scale (device array, read during the call's work;
  * NFFT2D_ERR_SIZE when the sizes differ). */

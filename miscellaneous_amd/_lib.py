@@ -103,6 +103,7 @@ _SIGS = {
     "nfft2d_batch_set_io_type1": (_i, [_vp, ctypes.POINTER(_vp), ctypes.POINTER(_vp)]),
     "nfft2d_batch_type1": (_i, [_vp, _vp]),
     "nfft2d_batch_setpts_type1": (_i, [_vp, _vp]),
+    "nfft2d_batch_get_type1_ranges": (_i, [_vp]),
     "nfft2d_batch_setpts_type1_scaled": (_i, [_vp, _vp, _vp]),
     "nfft2d_batch_set_maxpts": (_i, [_vp, _i, _i]),
     "nfft2d_batch_get_maxpts": (_i, [_vp, _i]),

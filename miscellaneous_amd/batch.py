@@ -130,6 +130,10 @@ class Batch:
                 check(self._lib.nfft2d_batch_setpts_type1_scaled(self._h, ctypes.c_void_p(scale.data_ptr()),
                                                                  _stream(self.device)), "nfft2d_batch_setpts_type1_scaled")
 
+    def type1_ranges(self) -> int:
+        """How the next setpts_type1() goes: 0 the passes of type1(), S > 0 direct sums over S ranges of the points."""
+        return self._lib.nfft2d_batch_get_type1_ranges(self._h)
+
     def autotune(self, reps: int = 3) -> list:
         """Choose by timing the subproblem size and the direct-gather cut-off per size class and the
         width of the persistent gather (``tuning()``); returns the per-transform subproblem sizes."""

@@ -2036,6 +2036,12 @@ static int batch_setpts_type1(nfft2d_batch *b, const float *scale, void *stream)
     return NFFT2D_OK;
 }
 
+extern "C" int nfft2d_batch_get_type1_ranges(const nfft2d_batch *b)
+{
+    if (!b) return nfft2d_fail(NFFT2D_ERR_ARG, "batch_get_type1_ranges: null batch");
+    return b->t1_sum ? b->t1_sum_plan.a.S : 0;
+}
+
 extern "C" int nfft2d_batch_setpts_type1(nfft2d_batch *b, void *stream) { return batch_setpts_type1(b, nullptr, stream); }
 
 extern "C" int nfft2d_batch_setpts_type1_scaled(nfft2d_batch *b, const float *scale, void *stream)
