@@ -287,8 +287,10 @@ int nfft1d_type1(nfft1d_plan *plan, nfft2d_c64 *result, const nfft2d_c64 *data, 
  * that are not powers of two, where a plan runs chirp-z passes and the batch
  * direct ones and the two agree to rounding; any M), run as ONE kernel launch
  * per stage over all of them:
- * nfft2d_batch_setpts is 5 launches, nfft2d_batch_type2 and type1 4 each,
- * whatever the number of transforms.  Neither allocates nor records a
+ * nfft2d_batch_setpts is 5 launches (2 for at most 2,048 transforms of at most
+ * 4,096 points and bins each), nfft2d_batch_type2 and type1 4 each, and one
+ * more per FFT pass and form of its lines (FFT or direct, chirp-z, in type1
+ * matrix cores) that the batch's sizes mix, whatever the number of transforms.  Neither allocates nor records a
  * hipMemset, so both can be captured into one hipGraph and replayed.  There is
  * no reference counterpart: the reference runs one NFFT2_2D_GPU call per
  * transform (e.g. once per particle per generation in
@@ -342,8 +344,8 @@ int nfft2d_batch_get_gather_blocks(const nfft2d_batch *batch);
  *   set_io_type1   data[t] (M[t] samples) and result[t] (N1 x N2): device
  *                  arrays, kept by reference; allocates each transform's
  *                  spread tiles; N1, N2 >= 22 (NFFT2D_ERR_SIZE otherwise);
- *   type1          4 launches (spread, tile merge, the two FFT passes with
- *                  crop and deconvolution), needs setpts;
+ *   type1          spread, tile merge, the two FFT passes with crop and
+ *                  deconvolution (4 launches and up, above), needs setpts;
  *   setpts_type1   setpts then type1 on `stream`; batches of
  *                  equal, small transforms: setpts, then direct sums of the
  *                  caller's points on the matrix cores (1 or 2 launches),

@@ -2,13 +2,16 @@
 
 ``Batch(sizes, device)`` with ``sizes = [(N1, N2, M), ...]`` builds one plan
 per transform (complex64, K = 6, c = 2; N1, N2 even in [2, 1024]: powers of
-two from 8 run the Stockham passes, other sizes direct ones).  Every stage
-then runs as one kernel launch over all transforms: ``setpts()`` is 5
-launches (2 for batches of transforms of at most 4096 points), ``type2()`` and ``type1()`` 4 each, so they can be captured into one
+two from 8 run the Stockham passes, other sizes chirp-z passes from 128 to 682
+and direct ones otherwise).  Every stage then runs as one kernel launch over
+all transforms: ``setpts()`` is 5 launches (2 for batches of transforms of at
+most 4096 points), ``type2()`` and ``type1()`` 4 each and one more per FFT pass
+and form of its lines that the sizes mix, so they can be captured into one
 graph.  ``type1`` (N1, N2 >= 22) is the reference's NFFT2_2D_GPU for every
 transform, e.g. the far fields of one PSO generation
-(``Synthesis/PSO/PSO.cu:348``, ``Synthesis.cu:395``) in one graph.  Arrays are kept by reference (``set_points`` / ``set_io``): keep
-the tensors alive while the batch uses them.
+(``Synthesis/PSO/PSO.cu:348``, ``Synthesis.cu:395``) in one graph.  Arrays are
+kept by reference (``set_points`` / ``set_io``): keep the tensors alive while
+the batch uses them.
 """
 from __future__ import annotations
 

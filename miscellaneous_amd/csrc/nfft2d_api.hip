@@ -1202,8 +1202,9 @@ extern "C" void Destroy_cuFFT_plan_NFFT2_2D(void)
 // the library is loaded on it until the process ends.  Its device address is
 // taken once per device with hipGetSymbolAddress (the array's name is a host
 // stand-in, not a device address) and kept in g_noalloc_ptr.  The kernels
-// and their order are those of NFFT2_2D_GPU_c64 (the results agree to FP32
-// rounding: the bin sort orders a bin's points as the waves reach its
+// and their order are those of a plan's setpts and type1 (the results agree
+// with NFFT2_2D_GPU_c64's, which sums small transforms directly, to FP32
+// rounding; the bin sort orders a bin's points as the waves reach its
 // counter, which the spread's sums follow).  Every call on a GPU shares that GPU's array: calls that overlap on one
 // GPU (different streams, or threads) race on it.  Every buffer is written
 // before it is read within a call (the setpts passes write every histogram

@@ -2,15 +2,17 @@
 //
 // A batch holds one plan per transform (complex64, K = 6, c = 2, N1 and N2
 // even, up to 1024; powers of two from 8 run the Stockham passes, other sizes
-// the direct ones).  Every stage of setpts and of the type-2 runs as
+// chirp-z passes from 128 to 682 and direct ones otherwise).  Every stage of setpts and of the type-2 runs as
 // ONE kernel over the blocks of all transforms: block b finds its transform
 // and its block index inside the transform in an owner table built when the
 // batch is created (the block counts of these stages depend on the sizes
 // only).  The gather is persistent: its blocks walk one list of the
 // subproblems of all transforms, each entry tagged with its transform.
-// Together: 5 launches for setpts (2 for batches of small transforms), 4 for the type-2 and 4 for the type-1,
-// whatever the number of transforms, all stream-ordered and free of
-// allocation, so the whole sequence can be captured into one hipGraph.
+// Together: 5 launches for setpts (2 for batches of small transforms), 4 for the
+// type-2 and 4 for the type-1, and one more per FFT pass and form of its lines
+// (FFT or direct, chirp-z, in the type-1 matrix cores) that the sizes mix,
+// whatever the number of transforms, all stream-ordered and free of allocation,
+// so the whole sequence can be captured into one hipGraph.
 #pragma once
 
 #include "nfft2d_czt.hpp"
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(kScatThreads) void kb_scatter_lds(const BatchDesc* 
 // both forms: the direct passes stage one line of up to 2 kBatchMaxN.  The
 // chirp-z lines (up to kBatchCztMaxM points; longer ones take the direct
 // passes) have launches of their own, kb_czt: inside these kernels their
-// registers (120 against 60) would halve the Stockham passes' occupancy (a
+// registers (120 against 60 when measured, 88 now) would halve the Stockham passes' occupancy (a
 // batch of 256 power-of-two transforms: column pass 303 -> 530 us).
 constexpr int kBatchCztMaxM = 2048;
 constexpr int kBatchLineLds = 2 * kBatchMaxN;

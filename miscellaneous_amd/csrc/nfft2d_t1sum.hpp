@@ -27,13 +27,13 @@
 // cosine polynomials) and steps to j + JS, j + 2 JS ... by complex products
 // with e^{2 JS i pi x/N}, computed once per point and stage.
 //
-// Measured (gfx950): 250 transforms of 88 x 88 modes from 1,936 points in one
-// launch 105 us, where spread, column pass and row pass took 144 + 195 + 51;
-// 45 GFLOP executed, 0.43 PFLOP/s: a stage's 27 products per wave (0.8 us of
-// matrix time on each SIMD) and its ~400 VALU instructions per wave make 2.9 us,
-// held by the latency of the operand chain at 2 waves per SIMD.  One
-// transform of that size: 9.5 + 3.0 us in two launches, where sort, spread and
-// passes took 30.
+// Measured (gfx950): 250 transforms of 88 x 88 modes from 1,936 points, a call of
+// 105 us with the two launches of its sort (about 14 us) in it, where spread,
+// column pass and row pass alone took 144 + 195 + 51; 45 GFLOP executed, about
+// 0.5 PFLOP/s: a stage's 27 products per wave (0.8 us of matrix time on each
+// SIMD) and its ~400 VALU instructions per wave make 2.9 us, held by the latency
+// of the operand chain at 2 waves per SIMD.  One transform of that size: 13.1 us
+// a call in two launches, where sort, spread and passes took 30.
 #pragma once
 
 #include "nfft2d_batch.hpp"
@@ -62,7 +62,10 @@ typedef __attribute__((address_space(1))) float gfloat;
 typedef __attribute__((address_space(1))) f2v gfloat2;
 constexpr int kSumThreads = 512;
 constexpr int kSumMaxLds = 160 * 1024;
-constexpr int kT1SumMaxN = 256;          // (2j + 1) 2^-33 turn phase error stays below FP32 rounding
+// A phase is off by at most (2j + 1) 2^-33 turns, 1.9e-7 rad per dimension at the
+// last mode of N = 256 (about 6e-8 rms over its modes and points), beside 1e-7 of
+// the phasors' FP32 evaluation and 1.5e-7 and more of the sums.
+constexpr int kT1SumMaxN = 256;
 constexpr int kT1SumMaxS = 12;           // every batch plan's spread scratch holds 12 partial results
 // A lone transform: up to 12 ranges of 8 stages of 64 points, and the work where
 // the sort, spread and FFT passes (30-38 us, launches mostly) are as fast.

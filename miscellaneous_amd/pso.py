@@ -9,10 +9,11 @@ scales the element positions to grid units (``:389-390``), calls
 (``farFieldFiltering``, ``:345-351``): one transform, one set of allocations and
 one synchronising call per particle, 250 particles per generation.
 
-Here the whole generation's far fields are ONE batch: the tile sort, the
-spread, the FFT passes and the filter of every particle in 10 kernel launches,
-captured into one graph and replayed every generation with the new positions
-and excitations written into its input arrays.  The aperture field, the
+Here the whole generation's far fields are ONE batch: the tile sort of every
+particle in two launches, then its modes as direct sums with the filter's
+factors in one or two more (larger grids or point sets: spread, FFT passes and
+filter, one launch per stage), captured into one graph and replayed every
+generation with the new positions and excitations written into its input arrays.  The aperture field, the
 positions (Zernike / Lagrange expansions) and the cost functional around this
 step are the synthesis code, not the NFFT, and are not part of this library.
 """
