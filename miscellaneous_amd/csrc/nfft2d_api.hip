@@ -907,8 +907,8 @@ extern "C" int nfft2d_type2(nfft2d_plan *p, void *result, const void *data, void
 // between the launches), more than the overlap saves where each branch fills
 // the chip or is a few launches long: two streams against one, eager, 128^2 /
 // 16K points 54.9 / 26.8 us, 512^2 / 1M 81.9 / 71.2, 1024^2 / 4M 216 / 214.
-// The chirp-z passes of large grids leave room beside them: 500^2 / 300K 79.2
-// / 74.1, 1000^2 / 1M 194 / 211.  In a captured graph the branches cost less,
+// The chirp-z passes of large grids leave room beside them: 500^2 / 262K 67.6
+// / 64.7, 860^2 / 262K 119 / 128, 1000^2 / 1M 157 / 172.  In a captured graph the branches cost less,
 // and either long grid passes or a long sort hide one in the other: 128^2 / 131K
 // 42.4 / 38.1, 256^2 / 262K 47.2 / 45.0, 512^2 / 1M 70.9 / 77.6, 1024^2 / 4M 205 /
 // 218; 64^2 / 524K 46.2 / 50.3, 128^2 / 524K 50.1 / 52.5, 256^2 / 2M 94.7 / 103.

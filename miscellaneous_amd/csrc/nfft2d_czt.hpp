@@ -22,7 +22,7 @@
 // leaves them: the kernel product and the start of the second FFT need no
 // exchange, and each FFT makes stages - 1 (three) trips through LDS.  Measured
 // on FP64 lines of 500 and 250 (500 x 250 modes, both passes of a type-2 /
-// type-1): 36 / 35 -> 25 / 24 us.  The twiddles come from global memory, so
+// type-1): 36 / 35 -> 21 / 21 us.  The twiddles come from global memory, so
 // they lie in the order in which a stage's roles read them: as one table
 // e^{-2 pi i j / m} read at strides of m / (8 NS) they were up to 448 cache lines
 // per wave and stage, and long lines ran behind the LDS form (type-2 of N x N
