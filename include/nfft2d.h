@@ -239,7 +239,8 @@ int nfft2d_plan_num_points(const nfft2d_plan *plan);
  * FP32 and BF16X3 sum conjugate pairs of modes (k, -1 - k) with real cosines
  * and sines, half the products; FP16 sums single modes.
  * Layouts and units are those of NFFT1_2D_GPU_c64.  The plan holds the mode
- * operand in the matrix cores' operand order (about 4 N1 N2 bytes for BF16X3);
+ * operand in the matrix cores' operand order (about 8 N1 N2 bytes; FP32 and
+ * BF16X3 twice that, a second copy scaled for sums beyond the FP32 range);
  * nfft2d_ndft_set_modes fills it, nfft2d_ndft_eval contracts it with M
  * points, nfft2d_ndft_type2 does both.  N1, N2 even, at most 8192. */
 typedef struct nfft2d_ndft_plan_s nfft2d_ndft_plan;

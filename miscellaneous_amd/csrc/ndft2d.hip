@@ -531,12 +531,13 @@ namespace {
 constexpr int kNdftMaxN = 8192;
 constexpr int kNdftC = ndft::kChunkTiles;  // MFMA column tiles per chunk
 
-size_t ndft_slice_bytes(int prec)
+// Bytes of the mode operand of `tiles` tiles.
+size_t ndft_operand_bytes(int prec, long long tiles)
 {
     switch (prec) {
-    case NFFT2D_NDFT_FP32: return sizeof(ndft::Slice<ndft::kNdftFp32>);
-    case NFFT2D_NDFT_BF16X3: return sizeof(ndft::Slice<ndft::kNdftBf16x3>);
-    default: return sizeof(ndft::Slice<ndft::kNdftFp16>);
+    case NFFT2D_NDFT_FP32: return ndft::operand_bytes<ndft::kNdftFp32>(tiles);
+    case NFFT2D_NDFT_BF16X3: return ndft::operand_bytes<ndft::kNdftBf16x3>(tiles);
+    default: return ndft::operand_bytes<ndft::kNdftFp16>(tiles);
     }
 }
 
@@ -569,7 +570,7 @@ extern "C" int nfft2d_ndft_plan_create(nfft2d_ndft_plan **plan, int N1, int N2, 
     const int kn = precision == NFFT2D_NDFT_FP16 ? N2 : N2 / 2;
     p->nch = (N1 + ndft::kChunkK1 - 1) / ndft::kChunkK1;
     p->nks = (kn + 8 * ndft::kKsPad - 1) / (8 * ndft::kKsPad) * ndft::kKsPad;
-    const size_t gbytes = (size_t)p->nch * p->nks * kNdftC * 64 * ndft_slice_bytes(precision);
+    const size_t gbytes = ndft_operand_bytes(precision, (long long)p->nch * p->nks * kNdftC);
     if (nfft2d_malloc(&p->G, gbytes) != hipSuccess || nfft2d_malloc(&p->scale, sizeof(float) * N1) != hipSuccess ||
         nfft2d_malloc(&p->inv_scale, sizeof(float) * N1) != hipSuccess) {
         (void)hipGetLastError();

@@ -159,12 +159,20 @@ __device__ __forceinline__ float2 expi_neg(int k, float x, double invN)
 //   part t % 2 (0: Re, 1: Im); for P (Q with EQ, OQ):
 //   Re P = sum c Re EP - (-s) Im OP,  Im P = sum c Im EP + (-s) Re OP.
 // Entries with j1 >= N1 / 2 or j2 >= N2 / 2 are zero (padding to whole tiles).
-// The sums of four modes are taken in FP64 and rounded once, as their quarter:
-// four modes beyond a quarter of the FP32 range would overflow in a plain sum
-// whose results still fit.  The results take the 4 back with the half steps.
-// Single modes (FP16): k2 index j2 as above with components (Re B, Im B), k1
-// index j1 = ch * 16 C + 32 (t / 2) + cc, part t % 2 of T:
-//   Re T = sum Re B Re F - Im B Im F,  Im T = sum Re B Im F + Im B Re F.
+// The sums of four modes are taken in FP64 and rounded once.  Large modes
+// overflow in them, or in the FP32 sums over them, where the results still fit;
+// one scale for all inputs would push small modes into the denormals instead
+// (BF16x3 modes of 1e-36: error 1.9e-5, with a quarter 7.4e-5).  So the operand
+// is stored twice, the second time over kPairUp, which no sum overflows, and the
+// contraction takes the second one only where the first gave a result that is
+// not finite.
+constexpr float kPairUp = 0x1p32f;
+// Bytes of the operand of `tiles` tiles.
+template <int P> constexpr size_t operand_bytes(long long tiles)
+{
+    return (size_t)tiles * 64 * sizeof(Slice<P>) * (paired<P>() ? 2 : 1);
+}
+
 template <int P, int C>
 __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F, const float* __restrict__ rowscale,
                                                    Slice<P>* __restrict__ G, int N1, int N2, int nch, int nks)
@@ -180,7 +188,7 @@ __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F,
     const int ch = (int)(r / nks);
     const int h = lane >> 5, cc = lane & 31;
     const int part = t & 1;
-    float v[8];
+    float v[8], d[8];
     if constexpr (paired<P>()) {
         const int j1 = ch * 8 * C + 16 * (t >> 1) + (cc >> 1);
         const double sq = (cc & 1) ? -1.0 : 1.0;       // P adds, Q subtracts the second k1 row
@@ -197,8 +205,10 @@ __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F,
                 o.x = ((double)pp.x - (double)pm.x) + sq * ((double)mp.x - (double)mm.x);
                 o.y = ((double)pp.y - (double)pm.y) + sq * ((double)mp.y - (double)mm.y);
             }
-            v[2 * q] = (float)(0.25 * (part == 0 ? e.x : e.y));
-            v[2 * q + 1] = (float)(0.25 * (part == 0 ? -o.y : o.x));
+            v[2 * q] = (float)(part == 0 ? e.x : e.y);
+            v[2 * q + 1] = (float)(part == 0 ? -o.y : o.x);
+            d[2 * q] = (float)((1.0 / kPairUp) * (part == 0 ? e.x : e.y));
+            d[2 * q + 1] = (float)((1.0 / kPairUp) * (part == 0 ? -o.y : o.x));
         }
     } else {
         const int j1 = ch * 16 * C + 32 * (t >> 1) + cc;
@@ -213,31 +223,35 @@ __global__ __launch_bounds__(256) void k_ndft_prep(const float2* __restrict__ F,
             v[e] = part == 0 ? (comp == 0 ? f.x : -f.y) : (comp == 0 ? f.y : f.x);
         }
     }
-    Slice<P> s;
-    if constexpr (P == kNdftFp32) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s.v[e] = v[e];
-    } else if constexpr (P == kNdftBf16x3) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            __bf16 hh, ll;
-            split_bf16(v[e], hh, ll);
-            s.hi[e] = hh;
-            s.lo[e] = ll;
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s.h[e] = (_Float16)v[e];
-    }
     // a tile stores its lanes' slices as 16-byte parts, part-major:
     // word (tile * kParts + part) * 64 + lane, so that one ds_read_b128 of a
     // part by 64 lanes reads 1 KB of consecutive LDS
     constexpr int kParts = (int)sizeof(Slice<P>) / 16;
-    const uint4* sw = reinterpret_cast<const uint4*>(&s);
     uint4* Gw = reinterpret_cast<uint4*>(G);
     const long long tile = i >> 6;
+    auto store = [&](const float (&u)[8], long long at) {
+        Slice<P> s;
+        if constexpr (P == kNdftFp32) {
 #pragma unroll
-    for (int q = 0; q < kParts; ++q) Gw[(tile * kParts + q) * 64 + lane] = sw[q];
+            for (int e = 0; e < 8; ++e) s.v[e] = u[e];
+        } else if constexpr (P == kNdftBf16x3) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                __bf16 hh, ll;
+                split_bf16(u[e], hh, ll);
+                s.hi[e] = hh;
+                s.lo[e] = ll;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s.h[e] = (_Float16)u[e];
+        }
+        const uint4* sw = reinterpret_cast<const uint4*>(&s);
+#pragma unroll
+        for (int q = 0; q < kParts; ++q) Gw[(at * kParts + q) * 64 + lane] = sw[q];
+    };
+    store(v, tile);
+    if constexpr (paired<P>()) store(d, (total >> 6) + tile);
 }
 
 // Slice (tile, lane) of a part-major tile array in LDS.
@@ -354,12 +368,13 @@ __device__ __forceinline__ void wave_sync()
 // each instead of 256), so that one wave's VALU work and LDS waits run under
 // the other wave's MFMAs; both generate the same point operands, and the two
 // partial sums of a point meet in LDS at the end.
+//
+// Pairs: G is over 1 or kPairUp, `up` is that factor.  Returns, the same to every
+// wave, whether a point with finite coordinates got a result that is not finite.
 template <int P, int EANCHOR, int SPLIT>
-__global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __restrict__ G,
-                                                            const float* __restrict__ inv_scale,
-                                                            const float* __restrict__ x1, const float* __restrict__ x2,
-                                                            float2* __restrict__ out, int N1, int N2, int M, int nch,
-                                                            int nks)
+__device__ __forceinline__ bool contract(const Slice<P>* __restrict__ G, float up, const float* __restrict__ inv_scale,
+                                         const float* __restrict__ x1, const float* __restrict__ x2,
+                                         float2* __restrict__ out, int N1, int N2, int M, int nch, int nks)
 {
     constexpr int C = kChunkTiles, R = kRowTiles, CW = C / SPLIT, NT = 256 * SPLIT;
     constexpr int kWords = C * 64 * (int)sizeof(Slice<P>) / 16;      // 16-byte words per K-step
@@ -374,7 +389,8 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
     __shared__ uint4 s_stage3[kWords];
     __shared__ float2 s_t[kWaves * SPLIT][32][33];
     __shared__ float2 s_y[SPLIT > 1 ? kWaves * R * 32 : 1];
-    const int tid = threadIdx.x;
+    int tid = threadIdx.x;
+    if (paired<P>()) asm volatile("" : "+v"(tid));   // no value is kept in registers from one call for the other
     const int lane = tid & 63, w = tid >> 6;
     const int pg = w % kWaves, hc = w / kWaves;                    // point group, column share
     const int h = lane >> 5, cc = lane & 31;
@@ -388,7 +404,6 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
     auto ph2 = [&](int j) { return kPair ? 2 * j + 1 : j - half2; };
     const int total = nch * nks;
     const uint4* Gw = reinterpret_cast<const uint4*>(G);
-
     // copy K-step gs (clamped to the last one) into buffer dst
     auto issue = [&](int gs, uint4* dst) {
         const uint4* src = Gw + (size_t)min(gs, total - 1) * kWords + 64 * w + lane;
@@ -534,12 +549,12 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
             }
         }
     }
-    // pairs: y carries 4 e^{pi i (x1 / N1 + x2 / N2)}, the half steps of both dimensions (and the operand's quarter)
+    // pairs: y carries e^{pi i (x1 / N1 + x2 / N2)}, the half steps of both dimensions, and the operand's factor
     float2 half[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         half[r] = kPair ? expi_neg_turns(-((double)xr1[r] * pu1 + (double)xr2[r] * pu2)) : make_float2(1.f, 0.f);
-        if (kPair) half[r] = make_float2(4.f * half[r].x, 4.f * half[r].y);
+        if (kPair) half[r] = make_float2(up * half[r].x, up * half[r].y);
     }
     // the two halves of each row, then (SPLIT = 2) the two column shares
 #pragma unroll
@@ -549,6 +564,7 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
         if (SPLIT > 1 && hc == 1 && h == 0) s_y[(pg * R + r) * 32 + cc] = y[r];
     }
     if constexpr (SPLIT > 1) __syncthreads();
+    bool bad = false;
     if (hc == 0 && h == 0) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -559,8 +575,43 @@ __global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __re
                 v.y += o.y;
             }
             const int m = m0 + 32 * r + cc;
-            if (m < M) out[m] = kPair ? cmul(v, half[r]) : v;
+            if (kPair) {
+                v = cmul(v, half[r]);
+                bad = bad || (m < M && !isfinite(v.x + v.y) && isfinite(half[r].x));
+            }
+            if (m < M) out[m] = v;
         }
+    }
+    if constexpr (!kPair) return false;
+    __shared__ int s_bad[kWaves];
+    const bool any = __any(bad);
+    if (hc == 0 && lane == 0) s_bad[pg] = any;
+    wait_vm<0>();        // the copies past the last K-step: the LDS is free again
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) all |= s_bad[k];
+    return all;
+}
+
+// The second call is a copy of its own behind a branch: as a loop over both
+// operands the compiler keeps more values alive through the K-steps (BF16x3, 16 x
+// 16 modes at 262,144 points: 55.8 us; now 51.7; without the second operand 50.9;
+// 256 x 256 at 65,536: now 54.2, without 53.4; FP32 the same).  A flag that the
+// operand's kernel sets and this one reads first: 53.0 at 16 x 16, FP32 + 0.4.
+template <int P, int EANCHOR, int SPLIT>
+__global__ __launch_bounds__(256 * SPLIT, 1) void k_ndft_t2(const Slice<P>* __restrict__ G,
+                                                            const float* __restrict__ inv_scale,
+                                                            const float* __restrict__ x1, const float* __restrict__ x2,
+                                                            float2* __restrict__ out, int N1, int N2, int M, int nch,
+                                                            int nks)
+{
+    const bool bad = contract<P, EANCHOR, SPLIT>(G, 1.f, inv_scale, x1, x2, out, N1, N2, M, nch, nks);
+    if (__builtin_expect(__builtin_amdgcn_readfirstlane(bad), 0)) {
+        // no value of the sizes is kept in registers from the first call either
+        asm volatile("" : "+s"(N1), "+s"(N2), "+s"(M), "+s"(nch), "+s"(nks));
+        const size_t slices = (size_t)nch * nks * kChunkTiles * 64;
+        contract<P, EANCHOR, SPLIT>(G + slices, kPairUp, inv_scale, x1, x2, out, N1, N2, M, nch, nks);
     }
 }
 
